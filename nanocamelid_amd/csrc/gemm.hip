@@ -1740,13 +1740,13 @@ int launch_gemm(const QMatDev& w, const GemmParams& p0, hipStream_t st, hipEvent
     p.groups = (int)w.groups;
     p.M = (int)w.rows;
     p.K = (int)w.cols;
-    if (p.N < 1 || p.N > 16) return fail(NC_EINVAL, "gemm: batch must be 1..16");
     if (w.layout == LAYOUT_Q6K) {
         if (ev0) NC_HIP(hipEventRecord(ev0, st));
         const int rc = launch_gemm_q6k(w, p, st);
         if (!rc && ev1) NC_HIP(hipEventRecord(ev1, st));
         return rc;
     }
+    if (p.N < 1 || p.N > 16) return fail(NC_EINVAL, "gemm: batch must be 1..16");
     if (w.layout == LAYOUT_R16) {
         // dot products by v_dot4c (AUTO: the faster path at every measured shape and width) or,
         // on request, by int8 MFMA

@@ -65,6 +65,9 @@ constexpr int kQ40R16QuadBytes = 1024 + 128;  // 1152; 8 per chunk = kQ40ChunkBy
 // f16 scales as [4 blocks][64 lanes].  Every load of a wave is 1 KB (or 128 B) contiguous.
 constexpr int kQ80GroupBlocks = 4;
 constexpr int kQ80ChunkBytes = kQ80GroupBlocks * 2048 + kQ80GroupBlocks * 128;  // 8704
+// Q6_K layout: 16-row tiles, super-blocks in quads; per (tile, quad) 13 x [64 lanes x 16 B] (lane
+// 16*q + r = super-block 4*quad + q of row r: ql 8 slots, qh 4, scales 1), then [64 lanes] f16 d.
+constexpr int kQ6KQuadBytes = 13 * 1024 + 128;
 enum Layout : int { LAYOUT_R64 = 0, LAYOUT_R16 = 1, LAYOUT_R16K = 2, LAYOUT_Q6K = 3, LAYOUT_Q80 = 4 };  // R16K: Q4_K on 16-row tiles
 
 struct QMatDev {
@@ -142,9 +145,9 @@ struct GemmParams {
 int launch_gemm(const QMatDev& w, const GemmParams& p, hipStream_t stream, hipEvent_t ev0 = nullptr,
                 hipEvent_t ev1 = nullptr);
 int launch_blockdots(const QMatDev& w, const int8_t* x, int32_t* dots, int N, hipStream_t stream);
-// Q6_K matmul (plain outputs or the head's logits + argmax partials); rows per head tile
+// Q6_K matmul of any number of tokens (plain outputs or the head's logits + argmax partials)
 int launch_gemm_q6k(const QMatDev& w, const GemmParams& p, hipStream_t stream);
-int q6k_rows_per_tile(int64_t cols);
+int64_t q6k_layout_bytes(int64_t rows, int64_t cols);
 
 // ---------------------------------------------------------------- layer kernels
 int launch_rmsnorm_q8(const float* hidden, const float* weight, int N, int d, float eps, int8_t* xq, float* xs,

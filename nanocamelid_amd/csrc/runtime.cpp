@@ -272,21 +272,23 @@ struct Part {
     int half;
 };
 
-// Builds one device matrix from one or more GGUF row blocks (fused q|k|v, interleaved
-// gate/up, or a single matrix).
-// Q6_K blocks (ql 128 | qh 64 | scales 16 | d 2 bytes) split into aligned planes
-static void repack_q6_k_planes(const uint8_t* src, int64_t nblk, uint8_t* dst) {
-    parallel_for(nblk, 0, [&](int64_t lo, int64_t hi) {
-        for (int64_t i = lo; i < hi; i++) {
-            const uint8_t* b = src + i * 210;
-            std::memcpy(dst + i * 128, b, 128);
-            std::memcpy(dst + nblk * 128 + i * 64, b + 128, 64);
-            std::memcpy(dst + nblk * 192 + i * 16, b + 192, 16);
-            std::memcpy(dst + nblk * 208 + i * 2, b + 208, 2);
-        }
+// Q6_K blocks (ql 128 | qh 64 | scales 16 | d 2 bytes) into 16-row tiles of super-block quads
+static void repack_q6_k(const uint8_t* src, int64_t rows, int64_t nsb, uint8_t* dst) {
+    const int64_t nquads = (nsb + 3) / 4;
+    parallel_for(rows, 0, [&](int64_t lo, int64_t hi) {
+        for (int64_t r = lo; r < hi; r++)
+            for (int64_t b = 0; b < nsb; b++) {
+                const uint8_t* blk = src + (r * nsb + b) * 210;
+                const int64_t lane = 16 * (b % 4) + r % 16;
+                uint8_t* chunk = dst + (r / 16 * nquads + b / 4) * kQ6KQuadBytes;
+                for (int i = 0; i < 13; i++) std::memcpy(chunk + i * 1024 + lane * 16, blk + 16 * i, 16);
+                std::memcpy(chunk + 13 * 1024 + lane * 2, blk + 208, 2);
+            }
     });
 }
 
+// Builds one device matrix from one or more GGUF row blocks (fused q|k|v, interleaved
+// gate/up, or a single matrix).
 static int upload_matrix(int type, int64_t rows, int64_t cols, const std::vector<Part>& parts, QMatDev& out) {
     if (cols % 32 || ((type == NC_TYPE_Q4_K || type == NC_TYPE_Q5_K || type == NC_TYPE_Q6_K) && cols % 256))
         return fail(NC_EINVAL, "matrix columns must be a multiple of 32 (Q4_K, Q5_K, Q6_K: 256)");
@@ -298,12 +300,12 @@ static int upload_matrix(int type, int64_t rows, int64_t cols, const std::vector
         out.rows = rows;
         out.cols = cols;
         out.units = cols / 256;
-        out.tiles = (rows + q6k_rows_per_tile(cols) - 1) / q6k_rows_per_tile(cols);
+        out.tiles = (rows + 15) / 16;
         out.groups = 0;
         out.algo_bytes = rows * (cols / 256) * 210;
-        out.dev_bytes = out.algo_bytes + 4;
+        out.dev_bytes = q6k_layout_bytes(rows, cols);
         std::vector<uint8_t> host(out.dev_bytes, 0);
-        repack_q6_k_planes(parts[0].src, rows * (cols / 256), host.data());
+        repack_q6_k(parts[0].src, rows, cols / 256, host.data());
         NC_HIP(hipMalloc((void**)&out.dev, out.dev_bytes));
         NC_HIP(hipMemcpy(out.dev, host.data(), out.dev_bytes, hipMemcpyHostToDevice));
         return NC_OK;
@@ -1157,6 +1159,14 @@ static bool prompt_matrix_ok(const QMatDev& q) {
     return false;
 }
 
+// Tokens per launch of a matrix without a prompt kernel: the Q6_K kernel takes any number (its token
+// groups share a launch), the others 16.
+static int slice_tokens(const QMatDev& q, int n) { return q.type == NC_TYPE_Q6_K ? n : 16; }
+
+// Whether the verify kernels of a matrix read the activations' block sums (the offset of the unsigned
+// values of Q4_0 and the mins of Q4_K and Q5_K).
+static bool needs_block_sums(const QMatDev& q) { return q.type != NC_TYPE_Q6_K && q.type != NC_TYPE_Q8_0; }
+
 // Prompt passes take every layer matrix on a prompt kernel, or Q5_K, Q6_K and Q8_0 ones in 16-row slices.
 static bool prompt_path_ok(const nc_model* m) {
     for (const LayerDev& L : m->layers)
@@ -1205,12 +1215,13 @@ static int prompt_gemm(nc_session* s, const QMatDev& w, const int8_t* xq, const 
                        int ld = 0) {
     if (ld == 0) ld = (int)w.rows;
     if (prompt_matrix_ok(w)) return prompt_matmul(w, xq, xs, out, ld, n, s->stream, s->p_xm, s->p_xsm, s->p_xam);
-    for (int i = 0; i < n; i += 16) {
+    const int slice = slice_tokens(w, n);
+    for (int i = 0; i < n; i += slice) {
         GemmParams p;
         p.x = xq + (size_t)i * w.cols;
         p.xs = xs + (size_t)i * (w.cols / 32);
         p.xs8 = s->p_xs8 + (size_t)i * (w.cols / 32);
-        p.N = std::min(16, n - i);
+        p.N = std::min(slice, n - i);
         p.epi = EPI_STORE;
         p.out = out + (size_t)i * ld;
         p.ld_out = ld;
@@ -1535,11 +1546,14 @@ int nc_matmul_quantized_batch(nc_ctx* ctx, const nc_qmat* w, const int8_t* x_i8,
     // more than 16 tokens: the MFMA prompt matmul (Q4_0), or 16-token slices (Q4_K)
     if (batch_size > 16 && prompt_matrix_ok(w->m) && prompt_slice_tokens(cols) >= 16)
         return ctx_prompt_matmul(ctx, w->m, x_i8, x_scales, out, batch_size, st);
-    for (int i = 0; i < batch_size; i += 16) {
-        const int nb = std::min(16, batch_size - i);
-        int rc = ensure_xsum(ctx, (size_t)nb * (cols / 32));
-        if (rc) return rc;
-        if ((rc = launch_block_sums(x_i8 + (size_t)i * cols, nb, (int)cols, ctx->xsum, st))) return rc;
+    const int slice = slice_tokens(w->m, batch_size);
+    for (int i = 0; i < batch_size; i += slice) {
+        const int nb = std::min(slice, batch_size - i);
+        int rc = NC_OK;
+        if (needs_block_sums(w->m) &&
+            ((rc = ensure_xsum(ctx, (size_t)nb * (cols / 32))) ||
+             (rc = launch_block_sums(x_i8 + (size_t)i * cols, nb, (int)cols, ctx->xsum, st))))
+            return rc;
         GemmParams p;
         p.kernel = ctx->gemm_kernel;
         p.x = x_i8 + (size_t)i * cols;

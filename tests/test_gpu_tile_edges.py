@@ -1,0 +1,39 @@
+"""Quantised matmuls at the edges of their tiles: ragged rows, columns that cut the super-block
+quads and block groups, every token-group size and prompt slices, bit-exact against the oracle (which
+evaluates the reference's per-row chains left to right)."""
+import numpy as np
+import pytest
+
+import nanocamelid_amd as nc
+from oracle import oracle as O
+from tests import gguf_writer as GW
+from tests.gpu_util import q8_activations
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    return nc.Context(0)
+
+
+def check(ctx, qtype, w, ref, M, K, batches, seed):
+    import torch
+    qm = nc.QMat(ctx, qtype, M, K, w)
+    for N in batches:
+        _, xq, xs = q8_activations(N, K, seed + N)
+        xq.reshape(-1)[:5] = [-128, 127, 0, -1, 1]  # the operator takes any int8
+        out = torch.full((N, M), float("nan"), device="cuda")
+        nc.matmul_quantized_batch(ctx, qm, torch.from_numpy(xq).cuda(), torch.from_numpy(xs).cuda(), out=out)
+        got = out.cpu().numpy()
+        want = ref(xq, xs, w, N, M, K, nthreads=8)
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (M, K, N)
+    qm.close()
+
+
+# K: one super-block, a cut quad (2, 5), a whole one and more quads than waves; N: every token-group
+# size 1..8, two and three uneven groups, prompt slices
+@pytest.mark.parametrize("M,K", [(1, 256), (17, 512), (100, 1280), (64, 1024), (33, 9472), (16, 16384)])
+def test_q6_k_tile_edges(ctx, M, K):
+    w = GW.q6_k_weights(M * K // 256, seed=M + K).reshape(M, K // 256, 210)
+    check(ctx, nc._ffi.NC_TYPE_Q6_K, w, O.matmul_q6_k, M, K, [1, 2, 3, 4, 5, 6, 7, 8, 9, 16, 17, 50], 3)
