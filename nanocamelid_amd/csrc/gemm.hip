@@ -236,10 +236,11 @@ __device__ __forceinline__ int dot32_bcast_scaled(int acc, float& c, int xp, int
 }
 
 // Term of token n (compile-time) for one block: t = (ws * xs) * (float)sum (nib - 8) * x.
-template <int n>
+template <int n, bool Q8 = false>
 __device__ __forceinline__ float term_q40(const int* xp, const int* meta, const int (&lo)[4], const int (&hi)[4],
                                           float ws) {
-    int d = bcast_i<8 + (n & 7)>(meta[n >> 3]);  // -8 * sum x: sum (nib-8)*x = sum nib*x - 8 sum x
+    // -8 * sum x: sum (nib-8)*x = sum nib*x - 8 sum x (Q8_0 weights are signed)
+    int d = Q8 ? 0 : bcast_i<8 + (n & 7)>(meta[n >> 3]);
     float c;                                       // x_scale * ws (IEEE product, commutative)
     d = dot32_bcast_scaled<8 * (n & 1), n & 7>(d, c, xp[n >> 1], meta[n >> 3], ws, lo[0], lo[1], lo[2], lo[3], hi[0],
                                                 hi[1], hi[2], hi[3]);
@@ -250,22 +251,22 @@ __device__ __forceinline__ float term_q40(const int* xp, const int* meta, const 
 // NMAX is the batch width itself for N <= 9.  With S > 1 the terms go to a double-
 // buffered LDS array, one barrier per round, and the chain threads add them in block order.
 // Terms of all NMAX tokens of one block (token pairs through dot32_bcast_pair).
-template <int NMAX>
+template <int NMAX, bool Q8 = false>
 __device__ __forceinline__ void terms_q40(float (&t)[NMAX], const int* xp, const int* meta, const int (&lo)[4],
                                           const int (&hi)[4], float ws) {
     [&]<int... P>(std::integer_sequence<int, P...>) {
         (([&] {
              constexpr int n0 = 2 * P, n1 = 2 * P + 1;
              if constexpr (n1 < NMAX) {
-                 int d0 = bcast_i<8 + (n0 & 7)>(meta[n0 >> 3]);
-                 int d1 = bcast_i<8 + (n1 & 7)>(meta[n1 >> 3]);
+                 int d0 = Q8 ? 0 : bcast_i<8 + (n0 & 7)>(meta[n0 >> 3]);
+                 int d1 = Q8 ? 0 : bcast_i<8 + (n1 & 7)>(meta[n1 >> 3]);
                  float c0, c1;  // x_scale * ws (meta[n0 >> 3] == meta[n1 >> 3]: n0, n1 differ in bit 0)
                  dot32_bcast_pair_scaled<n0 & 7, n1 & 7>(d0, d1, c0, c1, xp[P], meta[n0 >> 3], ws, lo[0], lo[1],
                                                          lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]);
                  t[n0] = c0 * (float)d0;
                  t[n1] = c1 * (float)d1;
              } else {
-                 t[n0] = term_q40<n0>(xp, meta, lo, hi, ws);
+                 t[n0] = term_q40<n0, Q8>(xp, meta, lo, hi, ws);
              }
          }()),
          ...);
@@ -384,93 +385,6 @@ __global__ __launch_bounds__(64 * S) void gemm_q4_0_kernel(GemmParams p) {
         }
     }
 #undef NC_R64_LOAD
-    gemm_epilogue<NMAX, S>(p, acc, tile, wave, lane);
-}
-
-// ---------------------------------------------------------------- Q8_0 (64-row tiles)
-// matmul_q8_0_batch (inference.rs:1343-1383): per row and token, sum += ws * xs * dot over the
-// 32-blocks in order, dot = the signed int8 block dot (dot_i8_scalar, q8.rs:3376-3382), ws the
-// block's f16 scale.  Lane l owns row 64*tile + l; in round r wave w takes block r*S + w (its
-// 32 weight bytes as two 16-byte loads, its scale); the token's 32 activation bytes and x_scale
-// are wave-uniform, read as scalar loads.  Terms of the S blocks of a round go through a
-// double-buffered LDS array and are added in block order by the chain threads (thread
-// (w, l): tokens w, w + S, ...), one barrier per round; the epilogues are the 64-row ones.
-template <int NMAX, int S>
-__global__ __launch_bounds__(64 * S) void gemm_q8_0_kernel(GemmParams p) {
-    constexpr int TPW = (NMAX + S - 1) / S;  // chain tokens per thread
-    constexpr int D = 2;                      // ring of rounds in flight
-    extern __shared__ float lds[];            // [2][S][NMAX][64] terms when S > 1
-    const int tile = blockIdx.x;
-    const int wave = wave_id_uniform();
-    const int lane = threadIdx.x & 63;
-    const int N = p.N, nb = p.units;
-    const uint8_t* wt = p.w + (size_t)tile * p.groups * kQ80ChunkBytes;
-    const int nrounds = (nb + S - 1) / S;
-    float acc[TPW];
-#pragma unroll
-    for (int j = 0; j < TPW; j++) acc[j] = 0.0f;
-    uint4 rw[D][2];
-    uint32_t rs[D];
-    // loads are unconditional, with the block index clamped into the row (a clamped block's
-    // term is never added)
-#define NC_Q80_LOAD(R, SLOT)                                                                       \
-    do {                                                                                           \
-        const int b_ = min(min((R), nrounds - 1) * S + wave, nb - 1);                              \
-        const uint8_t* c_ = wt + (size_t)(b_ / kQ80GroupBlocks) * kQ80ChunkBytes;                  \
-        const int u_ = b_ % kQ80GroupBlocks;                                                       \
-        rw[SLOT][0] = *(const uint4*)(c_ + (2 * u_) * 1024 + lane * 16);                           \
-        rw[SLOT][1] = *(const uint4*)(c_ + (2 * u_ + 1) * 1024 + lane * 16);                       \
-        rs[SLOT] = *(const uint16_t*)(c_ + kQ80GroupBlocks * 2048 + u_ * 128 + lane * 2);          \
-    } while (0)
-    NC_Q80_LOAD(0, 0);
-    for (int r0 = 0; r0 < nrounds; r0 += D) {
-#pragma unroll
-        for (int k = 0; k < D; k++) {
-            const int r = r0 + k;
-            if (r >= nrounds) break;  // uniform
-            NC_Q80_LOAD(r + 1, (k + 1) % D);
-            const int b = r * S + wave;
-            float* buf = lds + (size_t)(r & 1) * S * NMAX * 64;
-            if (b < nb) {  // uniform
-                const float ws = f16_to_f32((uint16_t)rs[k]);
-                const int wv[8] = {(int)rw[k][0].x, (int)rw[k][0].y, (int)rw[k][0].z, (int)rw[k][0].w,
-                                   (int)rw[k][1].x, (int)rw[k][1].y, (int)rw[k][1].z, (int)rw[k][1].w};
-                float t[NMAX];
-#pragma unroll
-                for (int n = 0; n < NMAX; n++) {
-                    // tokens >= N read the last token's activations and are never stored
-                    const int nn = min(n, N - 1);
-                    sptr_i32 xw = as_scalar_i32(p.x + (size_t)nn * p.K + (size_t)b * 32);
-                    sptr_f32 xsp = as_scalar_f32(p.xs + (size_t)nn * nb + b);
-                    int dot = 0;
-#pragma unroll
-                    for (int i = 0; i < 8; i++) dot = __builtin_amdgcn_sdot4(wv[i], xw[i], dot, false);
-                    t[n] = ws * xsp[0] * (float)dot;
-                }
-#pragma unroll
-                for (int n = 0; n < NMAX; n++) {
-                    if constexpr (S == 1) acc[n] = acc[n] + t[n];
-                    else buf[(wave * NMAX + n) * 64 + lane] = t[n];
-                }
-            }
-            if constexpr (S > 1) {
-                // buffer r & 1 is rewritten in round r + 2, after every thread passed round r + 1's
-                // barrier
-                __syncthreads();
-                const int nblk = min(S, nb - r * S);
-#pragma unroll
-                for (int j = 0; j < TPW; j++) {
-                    const int n = wave + j * S;
-                    if (n < N) {
-                        float a = acc[j];
-                        for (int bl = 0; bl < nblk; bl++) a = a + buf[(bl * NMAX + n) * 64 + lane];
-                        acc[j] = a;
-                    }
-                }
-            }
-        }
-    }
-#undef NC_Q80_LOAD
     gemm_epilogue<NMAX, S>(p, acc, tile, wave, lane);
 }
 
@@ -680,7 +594,12 @@ __device__ __forceinline__ void r16_swiglu_epilogue(const GemmParams& p, float* 
 // the extra waves is (token c / 16, row c % 16).  TPG = 4: one chain wave per token (CW =
 // NMAX), lane = 16 * tile + row, so the wave holds the token's 32 gate and 32 up outputs and
 // finishes SwiGLU and the Q8_0 block with shuffles.
-template <int NMAX, int S, int U, int D, int TPG, int CW = 0>
+//
+// Q8: Q8_0 weights (matmul_q8_0_batch, inference.rs:1343-1383: sum += ws * xs * dot per block, the same
+// chain).  A lane's block is 32 signed bytes in two 16-byte slots per quad, there is no offset to
+// correct, and the rest is the Q4_0 kernel.  4096 x 14336 at 5 tokens: 12.3 us, where 64-row tiles
+// (64 workgroups) with scalar activation loads took 92.
+template <int NMAX, int S, int U, int D, int TPG, int CW = 0, bool Q8 = false>
 __global__ __launch_bounds__(64 * (S * TPG + CW)) void gemm_q4_0_r16_kernel(GemmParams p) {
     static_assert(CW > 0 ? 16 * NMAX <= 64 * CW : 16 * NMAX <= 64 * S, "chain threads must fit their waves");
     static_assert(U == 1 || U == 2 || U == 4, "quads per wave per round");
@@ -690,6 +609,8 @@ __global__ __launch_bounds__(64 * (S * TPG + CW)) void gemm_q4_0_r16_kernel(Gemm
     constexpr int BR = 4 * QR;               // blocks per round
     constexpr int NP = (NMAX + 1) / 2;       // token-pair activation dwords per block
     constexpr int NM = (NMAX + 7) / 8;       // meta dwords per block
+    constexpr int NW = Q8 ? 2 : 1;           // 16-byte weight pieces per lane and quad
+    constexpr int QB = r16_quad_bytes(Q8), CB = 8 * QB;
     extern __shared__ float lds_all[];       // per tile group: [2][BR][NMAX][16]
     const int wave_all = wave_id_uniform();
     if constexpr (CW > 0 && TPG == 4) {
@@ -713,11 +634,11 @@ __global__ __launch_bounds__(64 * (S * TPG + CW)) void gemm_q4_0_r16_kernel(Gemm
     const int j = lane >> 4, i16 = lane & 15;
     const int N = p.N, nb = p.units;
     const int nq = (nb + 3) / 4;
-    const uint8_t* wt = p.w + (size_t)tile * p.groups * kQ40ChunkBytes;
+    const uint8_t* wt = p.w + (size_t)tile * p.groups * CB;
     const int xtok = i16 >> 3, mtok = i16 & 7;
     const int nrounds = (nq + QR - 1) / QR;
 
-    uint4 rw[D][U];
+    uint4 rw[D][U][NW];
     uint32_t rs[D][U];
     int rx[D][U][NP], rm[D][U][NM];
     // Unconditional loads (see the R64 kernel): exact wait counts across the ring.  Weights
@@ -728,7 +649,7 @@ __global__ __launch_bounds__(64 * (S * TPG + CW)) void gemm_q4_0_r16_kernel(Gemm
     // clamped (those terms are never added).
     const int qmax = 8 * p.groups - U;  // last wave-round start inside the padded groups (U | 8)
     const __amdgpu_buffer_rsrc_t wres =
-        __builtin_amdgcn_make_buffer_rsrc((void*)wt, 0, p.groups * kQ40ChunkBytes, 0x00020000);
+        __builtin_amdgcn_make_buffer_rsrc((void*)wt, 0, p.groups * CB, 0x00020000);
     const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc((void*)p.x, 0, N * p.K, 0x00020000);
     const __amdgpu_buffer_rsrc_t sres = __builtin_amdgcn_make_buffer_rsrc((void*)p.xs, 0, N * nb * 4, 0x00020000);
     const __amdgpu_buffer_rsrc_t s8res = __builtin_amdgcn_make_buffer_rsrc((void*)p.xs8, 0, N * nb * 4, 0x00020000);
@@ -745,17 +666,18 @@ __global__ __launch_bounds__(64 * (S * TPG + CW)) void gemm_q4_0_r16_kernel(Gemm
     // Block scales: lanes 0-7 of a row take xs, lanes 8-15 xs8.  For 3..8 rows two buffer
     // loads and a select measured faster than one load through a per-lane pointer; for
     // other widths the single clamped load is faster.
-    constexpr bool kMetaBuf = NMAX >= 3 && NMAX <= 8;
-    const bool meta_s = i16 < 8;
+    constexpr bool kMetaBuf = Q8 || (NMAX >= 3 && NMAX <= 8);
+    const bool meta_s = Q8 || i16 < 8;
     const int* mbase = meta_s ? (const int*)p.xs : p.xs8;
 #define NC_R16_LOAD(R, SLOT)                                                                         \
     do {                                                                                             \
         const int qd0_ = min(min((R), nrounds - 1) * QR + wave * U, qmax);                           \
-        const int cb_ = (qd0_ >> 3) * kQ40ChunkBytes;                                                \
+        const int cb_ = (qd0_ >> 3) * CB;                                                            \
         _Pragma("unroll") for (int u = 0; u < U; u++) {                                              \
-            const int qo_ = cb_ + ((qd0_ + u) & 7) * kQ40R16QuadBytes;                               \
-            rw[SLOT][u] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(wres, wvo, qo_, 0)); \
-            rs[SLOT][u] = __builtin_amdgcn_raw_buffer_load_b16(wres, svo, qo_ + 1024, 0);            \
+            const int qo_ = cb_ + ((qd0_ + u) & 7) * QB;                                             \
+            _Pragma("unroll") for (int i = 0; i < NW; i++) rw[SLOT][u][i] = __builtin_bit_cast(      \
+                uint4, __builtin_amdgcn_raw_buffer_load_b128(wres, wvo, qo_ + 1024 * i, 0));         \
+            rs[SLOT][u] = __builtin_amdgcn_raw_buffer_load_b16(wres, svo, qo_ + 1024 * NW, 0);       \
         }                                                                                            \
         _Pragma("unroll") for (int u = 0; u < U; u++) {                                              \
             _Pragma("unroll") for (int q = 0; q < NP; q++) rx[SLOT][u][q] = (int)                     \
@@ -764,8 +686,12 @@ __global__ __launch_bounds__(64 * (S * TPG + CW)) void gemm_q4_0_r16_kernel(Gemm
                 if constexpr (kMetaBuf) {                                                            \
                     const int mo_ = mvo[q] + 16 * (qd0_ + u);                                        \
                     const int ms_ = (int)__builtin_amdgcn_raw_buffer_load_b32(sres, mo_, 0, 0);      \
-                    const int m8_ = (int)__builtin_amdgcn_raw_buffer_load_b32(s8res, mo_, 0, 0);     \
-                    rm[SLOT][u][q] = meta_s ? ms_ : m8_;                                             \
+                    if constexpr (Q8) {                                                              \
+                        rm[SLOT][u][q] = ms_;                                                        \
+                    } else {                                                                         \
+                        const int m8_ = (int)__builtin_amdgcn_raw_buffer_load_b32(s8res, mo_, 0, 0); \
+                        rm[SLOT][u][q] = meta_s ? ms_ : m8_;                                         \
+                    }                                                                                \
                 } else {                                                                             \
                     const int b_ = min(4 * (qd0_ + u) + j, nb - 1);                                  \
                     rm[SLOT][u][q] = mbase[(size_t)mt[q] * nb + b_];                                 \
@@ -789,15 +715,24 @@ __global__ __launch_bounds__(64 * (S * TPG + CW)) void gemm_q4_0_r16_kernel(Gemm
 #pragma unroll
                 for (int u = 0; u < U; u++) {
                     if (qd0 + u < nq) {  // uniform
-                        const uint4 v = rw[k][u];
-                        const int lo[4] = {(int)(v.x & 0x0F0F0F0Fu), (int)(v.y & 0x0F0F0F0Fu),
-                                           (int)(v.z & 0x0F0F0F0Fu), (int)(v.w & 0x0F0F0F0Fu)};
-                        const int hi[4] = {(int)((v.x >> 4) & 0x0F0F0F0Fu), (int)((v.y >> 4) & 0x0F0F0F0Fu),
-                                           (int)((v.z >> 4) & 0x0F0F0F0Fu), (int)((v.w >> 4) & 0x0F0F0F0Fu)};
+                        const uint4 v = rw[k][u][0];
+                        int lo[4], hi[4];  // the block's 8 weight dwords: 0-3, 4-7
+                        if constexpr (Q8) {
+                            const uint4 v1 = rw[k][u][NW - 1];
+                            lo[0] = (int)v.x, lo[1] = (int)v.y, lo[2] = (int)v.z, lo[3] = (int)v.w;
+                            hi[0] = (int)v1.x, hi[1] = (int)v1.y, hi[2] = (int)v1.z, hi[3] = (int)v1.w;
+                        } else {
+                            const uint32_t w4[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                            for (int i = 0; i < 4; i++) {
+                                lo[i] = (int)(w4[i] & 0x0F0F0F0Fu);
+                                hi[i] = (int)((w4[i] >> 4) & 0x0F0F0F0Fu);
+                            }
+                        }
                         const float ws = f16_to_f32((uint16_t)rs[k][u]);
                         float* dst = buf + ((size_t)((wave * U + u) * 4 + j) * NMAX) * 16 + i16;
                         float t[NMAX];
-                        terms_q40<NMAX>(t, rx[k][u], rm[k][u], lo, hi, ws);
+                        terms_q40<NMAX, Q8>(t, rx[k][u], rm[k][u], lo, hi, ws);
 #pragma unroll
                         for (int n = 0; n < NMAX; n++) dst[n * 16] = t[n];
                     }
@@ -1520,7 +1455,7 @@ int launch_one(const QMatDev& w, const GemmParams& p, hipStream_t st, hipEvent_t
 // R16: S waves so that the chain threads (16 per token) fit; U = 1 quad per wave-round and
 // one round in flight ahead of the one being computed (the fastest of the measured
 // S x U x D shapes on every layer matrix of the 8B model).
-template <int NMAX>
+template <int NMAX, bool Q8 = false>
 int launch_r16(const QMatDev& w, const GemmParams& p, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
     constexpr int U = 1, D = 2;
     if (p.epi == EPI_SWIGLU_Q8) {
@@ -1532,10 +1467,10 @@ int launch_r16(const QMatDev& w, const GemmParams& p, hipStream_t st, hipEvent_t
         if (p.ntiles % TPG) return fail(NC_EINVAL, "gemm: SwiGLU rows must fill whole 64-row groups");
         const size_t lds = (size_t)TPG * r16_tile_lds<4 * S * U, NMAX, TPG>() * sizeof(float);
         if (ev0)
-            hipExtLaunchKernelGGL((gemm_q4_0_r16_kernel<NMAX, S, U, D, TPG, CW>), dim3(p.ntiles / TPG),
+            hipExtLaunchKernelGGL((gemm_q4_0_r16_kernel<NMAX, S, U, D, TPG, CW, Q8>), dim3(p.ntiles / TPG),
                                   dim3(64 * (S * TPG + CW)), lds, st, ev0, ev1, 0, p);
         else
-            NC_LAUNCH((gemm_q4_0_r16_kernel<NMAX, S, U, D, TPG, CW>), dim3(p.ntiles / TPG),
+            NC_LAUNCH((gemm_q4_0_r16_kernel<NMAX, S, U, D, TPG, CW, Q8>), dim3(p.ntiles / TPG),
                                dim3(64 * (S * TPG + CW)), lds, st, p);
     } else {
         // 8 waves (two per SIMD hide each other's dependency latency); 16 when K is long
@@ -1546,10 +1481,10 @@ int launch_r16(const QMatDev& w, const GemmParams& p, hipStream_t st, hipEvent_t
         auto go = [&]<int S>() {
             const size_t lds = (size_t)2 * 4 * S * U * NMAX * 16 * sizeof(float);
             if (ev0)
-                hipExtLaunchKernelGGL((gemm_q4_0_r16_kernel<NMAX, S, U, D, 1, CW>), dim3(p.ntiles),
+                hipExtLaunchKernelGGL((gemm_q4_0_r16_kernel<NMAX, S, U, D, 1, CW, Q8>), dim3(p.ntiles),
                                       dim3(64 * (S + CW)), lds, st, ev0, ev1, 0, p);
             else
-                NC_LAUNCH((gemm_q4_0_r16_kernel<NMAX, S, U, D, 1, CW>), dim3(p.ntiles), dim3(64 * (S + CW)),
+                NC_LAUNCH((gemm_q4_0_r16_kernel<NMAX, S, U, D, 1, CW, Q8>), dim3(p.ntiles), dim3(64 * (S + CW)),
                                    lds, st, p);
         };
         if constexpr (NMAX <= 6) {
@@ -1563,6 +1498,11 @@ int launch_r16(const QMatDev& w, const GemmParams& p, hipStream_t st, hipEvent_t
     }
     NC_HIP(hipGetLastError());
     return NC_OK;
+}
+
+template <int NMAX>
+int launch_q80(const QMatDev& w, const GemmParams& p, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
+    return launch_r16<NMAX, true>(w, p, st, ev0, ev1);
 }
 
 // R16 with MFMA dots: the same launch shapes as launch_r16 (term waves per tile, dedicated
@@ -1686,28 +1626,6 @@ int launch_k16(const QMatDev& w, const GemmParams& p, hipStream_t st, hipEvent_t
 }
 
 }  // namespace
-
-template <int NMAX>
-int launch_q80(const QMatDev& w, const GemmParams& p, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
-    // K-split waves: enough that ~1000+ waves stream the matrix, at most one per block
-    int S = 1;
-    while (S < 8 && w.tiles * S < 1024 && 2 * S <= w.units) S *= 2;
-    auto go = [&]<int SS>() {
-        const size_t lds = SS > 1 ? (size_t)2 * SS * NMAX * 64 * sizeof(float) : 0;
-        if (ev0)
-            hipExtLaunchKernelGGL((gemm_q8_0_kernel<NMAX, SS>), dim3(p.ntiles), dim3(64 * SS), lds, st, ev0, ev1, 0, p);
-        else
-            NC_LAUNCH((gemm_q8_0_kernel<NMAX, SS>), dim3(p.ntiles), dim3(64 * SS), lds, st, p);
-    };
-    switch (S) {
-        case 1: go.template operator()<1>(); break;
-        case 2: go.template operator()<2>(); break;
-        case 4: go.template operator()<4>(); break;
-        default: go.template operator()<8>(); break;
-    }
-    NC_HIP(hipGetLastError());
-    return NC_OK;
-}
 
 // R64 waves per workgroup: enough K-split waves that ~1000+ waves stream the matrix
 // (1, 2 or 4; LDS terms double-buffered: 2 * S * 4 * NMAX * 64 floats).

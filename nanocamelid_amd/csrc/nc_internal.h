@@ -60,11 +60,11 @@ constexpr int kQ4KChunkBytes = 9 * 1024;
 // 4 blocks x 16 rows and its scales are one contiguous 128-byte line.
 constexpr int kTileRowsR16 = 16;
 constexpr int kQ40R16QuadBytes = 1024 + 128;  // 1152; 8 per chunk = kQ40ChunkBytes
-// Q8_0 layout: rows padded to 64-row tiles; per (tile, group of 4 blocks) an 8704-byte chunk =
-// [4 blocks][2 halves][64 lanes x 16 B] of int8 weights (lane l = row 64*tile + l), then the
-// f16 scales as [4 blocks][64 lanes].  Every load of a wave is 1 KB (or 128 B) contiguous.
-constexpr int kQ80GroupBlocks = 4;
-constexpr int kQ80ChunkBytes = kQ80GroupBlocks * 2048 + kQ80GroupBlocks * 128;  // 8704
+// Q8_0 layout: as R16 with 32 signed bytes per block: a quad is 2 x [64 lanes x 16 B] (a block's bytes
+// 0-15, then 16-31) and the same 128-byte scale line; 8 quads per chunk.
+constexpr int kQ80R16QuadBytes = 2048 + 128;
+constexpr int kQ80ChunkBytes = 8 * kQ80R16QuadBytes;  // 32 blocks x 16 rows
+__host__ __device__ constexpr int r16_quad_bytes(bool q8) { return q8 ? kQ80R16QuadBytes : kQ40R16QuadBytes; }
 // Q6_K layout: 16-row tiles, super-blocks in quads; per (tile, quad) 13 x [64 lanes x 16 B] (lane
 // 16*q + r = super-block 4*quad + q of row r: ql 8 slots, qh 4, scales 1), then [64 lanes] f16 d.
 constexpr int kQ6KQuadBytes = 13 * 1024 + 128;
@@ -74,9 +74,9 @@ struct QMatDev {
     int type = NC_TYPE_Q4_0;
     int layout = LAYOUT_R64;
     int64_t rows = 0, cols = 0;
-    int64_t tiles = 0;       // padded rows / 64 (R16: / 16)
+    int64_t tiles = 0;       // padded rows / 64 (R16, R16K, Q8_0, Q6_K: / 16)
     int64_t units = 0;       // Q4_0, Q8_0: blocks per row; Q4_K: super-blocks per row
-    int64_t groups = 0;      // Q4_0: ceil(blocks / 8) (R16: ceil(blocks / 32)); Q8_0: ceil(blocks / 4)
+    int64_t groups = 0;      // Q4_0: ceil(blocks / 8) (R16, Q8_0: ceil(blocks / 32))
     uint8_t* dev = nullptr;  // repacked bytes
     int64_t dev_bytes = 0;
     int64_t algo_bytes = 0;  // rows * cols * 18/32 (Q4_0) or 144/256 (Q4_K)

@@ -184,24 +184,25 @@ void repack_q4_0(const uint8_t* src, int64_t rows_src, int64_t cols, uint8_t* ds
 }
 
 int64_t q80_layout_bytes(int64_t rows, int64_t cols) {
-    return (rows + 63) / 64 * ((cols / 32 + kQ80GroupBlocks - 1) / kQ80GroupBlocks) * kQ80ChunkBytes;
+    return (rows + 15) / 16 * ((cols / 32 + 31) / 32) * kQ80ChunkBytes;
 }
 
-// Q8_0 block = f16 scale + 32 int8 (34 bytes, Q8_0Block::from_bytes q8.rs:479-487).
+// Q8_0 block = f16 scale + 32 int8 (34 bytes, Q8_0Block::from_bytes q8.rs:479-487); tiles, quads and
+// scale order as repack_q4_0_r16.
 void repack_q8_0(const uint8_t* src, int64_t rows_src, int64_t cols, uint8_t* dst, int64_t groups, int64_t row_off,
                  int half) {
     const int64_t nb = cols / 32;
     parallel_for(rows_src, 0, [&](int64_t lo, int64_t hi) {
         for (int64_t r = lo; r < hi; r++) {
             const int64_t R = dst_row(r, row_off, half);
-            const int64_t t = R / 64, l = R % 64;
+            const int64_t t = R / 16, rr = R % 16;
             for (int64_t b = 0; b < nb; b++) {
                 const uint8_t* blk = src + (r * nb + b) * 34;
-                uint8_t* chunk = dst + (t * groups + b / kQ80GroupBlocks) * kQ80ChunkBytes;
-                const int64_t u = b % kQ80GroupBlocks;
-                std::memcpy(chunk + (2 * u) * 1024 + l * 16, blk + 2, 16);
-                std::memcpy(chunk + (2 * u + 1) * 1024 + l * 16, blk + 18, 16);
-                std::memcpy(chunk + kQ80GroupBlocks * 2048 + u * 128 + l * 2, blk, 2);
+                const int64_t qd = b / 4, j = b % 4, lane = 16 * j + rr;
+                uint8_t* quad = dst + (t * groups + qd / 8) * kQ80ChunkBytes + (qd % 8) * kQ80R16QuadBytes;
+                std::memcpy(quad + lane * 16, blk + 2, 16);
+                std::memcpy(quad + 1024 + lane * 16, blk + 18, 16);
+                std::memcpy(quad + 2048 + 2 * (16 * (rr / 4) + 4 * j + (rr % 4)), blk, 2);
             }
         }
     });
@@ -316,8 +317,8 @@ static int upload_matrix(int type, int64_t rows, int64_t cols, const std::vector
     if (type == NC_TYPE_Q8_0) {
         out.layout = LAYOUT_Q80;
         out.units = cols / 32;
-        out.tiles = (rows + 63) / 64;
-        out.groups = (out.units + kQ80GroupBlocks - 1) / kQ80GroupBlocks;
+        out.tiles = (rows + 15) / 16;
+        out.groups = (out.units + 31) / 32;
         out.dev_bytes = q80_layout_bytes(rows, cols);
         out.algo_bytes = rows * cols / 32 * 34;
         std::vector<uint8_t> host(out.dev_bytes, 0);

@@ -7,7 +7,7 @@ import pytest
 import nanocamelid_amd as nc
 from oracle import oracle as O
 from tests import gguf_writer as GW
-from tests.gpu_util import q8_activations
+from tests.gpu_util import q8_activations, random_q8_0
 
 pytestmark = pytest.mark.gpu
 
@@ -37,3 +37,11 @@ def check(ctx, qtype, w, ref, M, K, batches, seed):
 def test_q6_k_tile_edges(ctx, M, K):
     w = GW.q6_k_weights(M * K // 256, seed=M + K).reshape(M, K // 256, 210)
     check(ctx, nc._ffi.NC_TYPE_Q6_K, w, O.matmul_q6_k, M, K, [1, 2, 3, 4, 5, 6, 7, 8, 9, 16, 17, 50], 3)
+
+
+# K: one block, a cut quad, a whole one, a cut chunk of 8 quads, 12 term waves (>= 64 quads); N: every width
+# the kernel is built for, both widths with their chains on term waves (9, 16) and a cut 16-token slice
+@pytest.mark.parametrize("M,K", [(1, 32), (17, 96), (100, 1024), (64, 1120), (33, 8224), (1040, 64)])
+def test_q8_0_tile_edges(ctx, M, K):
+    w = random_q8_0(M, K, seed=M + K)
+    check(ctx, nc.NC_TYPE_Q8_0, w, O.matmul_q8_0, M, K, [1, 2, 3, 4, 5, 6, 7, 8, 9, 16, 17, 50], 4)
