@@ -186,14 +186,17 @@ int launch_attention(const AttnParams& a, hipStream_t stream);
 int64_t attention_variant(const AttnParams& a);
 
 // ---------------------------------------------------------------- prompt (prefill) path
-// Q4_0 batch matmul for any number of tokens on int8 MFMA: out[n * ld_out + row] (R16 and R64
-// layouts) over xm / xsm, the activations x / xs repacked by launch_prompt_repack (xm:
-// 16 * ceil(N/16) * K bytes, xsm: 16 * ceil(N/16) * ceil(K/128) * 4 floats).
-int launch_gemm_prompt(const QMatDev& w, const int8_t* x, const float* xs, float* out, int ld_out, int N,
-                       hipStream_t stream, const void* xm, const float* xsm);
-// xam (optional, as xsm): the float sums of each 32-value block's int8 values (Q4_K's A_j)
+// Q4_0 / Q8_0 batch matmul for any number of tokens on the matrix cores: out[n * ld_out + row] over
+// xh / xsm, the activations as f16 in operand order with their scales (launch_prompt_repack_f16; xh:
+// 16 * ceil(N/16) * prompt_cols(K) * 2 bytes, xsm: 16 * ceil(N/16) * prompt_cols(K) / 32 floats).
+int launch_gemm_prompt(const QMatDev& w, float* out, int ld_out, int N, hipStream_t stream, const void* xh,
+                       const float* xsm);
+int launch_prompt_repack_f16(const int8_t* x, const float* xs, int N, int K, void* xh, float* xsm, hipStream_t stream);
+inline int64_t prompt_cols(int64_t cols) { return (cols + 127) / 128 * 128; }  // whole quads of blocks
+// The int8 form for the K-quant prompt matmuls (xm: 16 * ceil(N/16) * K bytes, xsm as above).
 int launch_prompt_repack(const int8_t* x, const float* xs, int N, int K, void* xm, float* xsm, hipStream_t stream,
                          float* xam = nullptr);
+// (xam, as xsm: the float sums of each 32-value block's int8 values, Q4_K's A_j)
 // Q4_K batch matmul for any number of tokens on int8 MFMA (R16K and R64 layouts) over
 // activations repacked with their block sums
 int launch_gemm_prompt_q4k(const QMatDev& w, float* out, int ld_out, int N, hipStream_t stream, const void* xm,

@@ -1,23 +1,23 @@
-// Prompt (prefill) path on gfx950: the Q4_0 x Q8_0 batch matmul for many tokens at once on
-// int8 MFMA, and the elementwise steps that the verify GEMMs fuse into their epilogues (RoPE
-// and the KV-cache scatter, the residual add, SwiGLU + Q8_0), as separate kernels over the
-// matmul's f32 output.
+// Prompt (prefill) path on gfx950: the batch matmuls for many tokens at once on the matrix cores,
+// and the elementwise steps that the verify GEMMs fuse into their epilogues (RoPE and the
+// KV-cache scatter, the residual add, SwiGLU + Q8_0), as separate kernels over the matmul's f32
+// output.
 //
-// Each output is the reference's f32 chain over the row's blocks in order
-// (matmul_q4_0_batch, inference.rs:1385-1418, and the swizzled form :1525-1574):
+// Q4_0 and Q8_0: each output is the reference's f32 chain over the row's blocks in order
+// (matmul_q4_0_batch, inference.rs:1385-1418, and the swizzled form :1525-1574; matmul_q8_0_batch
+// :1343-1383):
 //   sum = 0; for b: sum += (w_scale[b] * x_scale[b]) * (float)dot_b
-// so any number of tokens gives the bits of the 1-token loop.  The int32 block dots come from
-// v_mfma_i32_16x16x32_i8 on the raw nibbles (0..15) with the accumulator input set to
-// -8 * sum(x) of the block, itself one MFMA of a constant -8 operand with the same activations:
-//   A (16 rows x 32, weights): lane (g, r) holds row r's nibble bytes 4g..4g+3, i.e. weights
-//     4g..4g+3 (low nibbles) and 16+4g..16+4g+3 (high nibbles);
-//   B (32 x 16 tokens, activations): lane (g, c) holds token c's x[4g..4g+3], x[16+4g..+3];
-//   D lane (g, c): token c, rows 4g..4g+3.
-// A wave owns 32 rows x 32 tokens (2 x 2 MFMA tiles, 16 chains per lane); a workgroup of four
-// waves covers 64 rows x 64 tokens, so each weight byte is read by two waves of one workgroup
-// and each activation by two.  Unlike the verify kernels (one to sixteen tokens, bound by the
-// weight stream), the work here is the chain arithmetic: four VALU operations per (row, token,
-// block); the MFMAs run beside them.
+// so any number of tokens gives the bits of the 1-token loop.  Per 16 x 16 tile and block the chain
+// leaves eight f32 VALU operations per lane (a product and an add for each of its four outputs);
+// everything else comes from the matrix cores, whose results arrive as f32:
+//   dot_b: v_mfma_f32_16x16x32_f16 on the weights and activations as f16.  Both are integers (weights
+//     -8..7 or -128..127, activations -128..127), every partial sum is below 2^20, so the f32 result is
+//     the exact integer: no conversion, and no correction for the unsigned nibble;
+//   w_scale * x_scale: v_mfma_f32_16x16x1_4b_f32, an outer product of one term per block, four blocks
+//     at once.  With one term and a zero addend it rounds like the multiply, subnormals included.
+// Operands: A lane (g, r) = row r's elements 4g..4g+3 and 16+4g..+3 of the block, B lane (g, c) = token
+// c's (both in the order 0, 2, 16, 18, 1, 3, 17, 19 + 4g that unpacking a nibble dword gives), D lane
+// (g, c) = token c, rows 4g..4g+3.
 #include "nc_internal.h"
 #include "nc_device.h"
 
@@ -25,198 +25,208 @@ namespace nc {
 
 typedef int p_v4i __attribute__((ext_vector_type(4)));
 
+typedef float p_v4f __attribute__((ext_vector_type(4)));
+typedef float p_v16f __attribute__((ext_vector_type(16)));
+typedef _Float16 p_h2 __attribute__((ext_vector_type(2)));
+typedef _Float16 p_h8 __attribute__((ext_vector_type(8)));
+
 struct PromptGemm {
     const uint8_t* w = nullptr;
-    int64_t w_bytes = 0;
-    int groups = 0;   // chunks per tile row (R16: 32 blocks each, R64: 8)
+    int groups = 0;   // chunks per tile row (R16, Q8_0: 32 blocks each, R64: 8)
     int tiles16 = 0;  // 16-row tiles present in storage
     int M = 0, nb = 0, N = 0, ld_out = 0;
-    const int8_t* x = nullptr;  // [N][32 * nb]
-    const float* xs = nullptr;  // [N][nb]
-    // the same activations repacked in MFMA operand order (prompt_repack_kernel), or null:
-    // xm [N/16][nb][lane (g, c)] 8 bytes, xsm [N/16][nb/4][c] the 4 scales of a quad
-    const uint2* xm = nullptr;
-    const float4* xsm = nullptr;
-    float* out = nullptr;       // out[n * ld_out + row]
+    // the activations in operand order (prompt_repack_kernel), blocks padded to quads: xh [N/16][4 nq]
+    // units of [64 lanes] 8 f16, xsm [N/16][nq][64 lanes] x_scale of (block lane / 16, token lane % 16)
+    const uint8_t* xh = nullptr;
+    const float* xsm = nullptr;
+    float* out = nullptr;  // out[n * ld_out + row]
 };
 
-template <int LAYOUT, int D, int RT>
-__global__ __launch_bounds__(256) void gemm_q4_0_prompt_kernel(PromptGemm p) {
-    // wave index through readfirstlane: the tile bases below are then scalar (buffer-load
-    // soffsets) instead of per-lane values that the compiler would loop over
+// 8 f16 weights of a lane's nibble dword: 0x6400 | n is 1024 + n, so one packed add gives n - 8.
+// one (a constant in a VGPR) lets the mask and the or be one v_and_or_b32.
+__device__ __forceinline__ p_h8 unpack_q40(uint32_t w, uint32_t one) {
+    uint32_t u[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int sh = i == 0 ? 0 : i == 1 ? 4 : i == 2 ? 8 : 12;  // bytes 0,2 low, high; bytes 1,3 low, high
+        const p_h2 v = __builtin_bit_cast(p_h2, ((w >> sh) & 0x000F000Fu) | one);
+        u[i] = __builtin_bit_cast(uint32_t, v - (p_h2){(_Float16)1032.0f, (_Float16)1032.0f});
+    }
+    return __builtin_bit_cast(p_h8, make_uint4(u[0], u[1], u[2], u[3]));
+}
+// the same of a Q8_0 lane's two dwords of signed bytes
+__device__ __forceinline__ p_h8 unpack_q80(uint32_t w0, uint32_t w1, uint32_t one) {
+    const uint32_t a = w0 ^ 0x80808080u, b = w1 ^ 0x80808080u;
+    uint32_t u[4] = {(a & 0x00FF00FFu) | one, (b & 0x00FF00FFu) | one, ((a >> 8) & 0x00FF00FFu) | one,
+                     ((b >> 8) & 0x00FF00FFu) | one};
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const p_h2 v = __builtin_bit_cast(p_h2, u[i]);
+        u[i] = __builtin_bit_cast(uint32_t, v - (p_h2){(_Float16)1152.0f, (_Float16)1152.0f});
+    }
+    return __builtin_bit_cast(p_h8, make_uint4(u[0], u[1], u[2], u[3]));
+}
+
+// Workgroup = 4 waves x (16 rows x 16 KT tokens): the waves take consecutive row tiles of the same
+// tokens, whose activation units go through LDS (double-buffered stages of one quad of blocks, loaded
+// SD stages ahead into registers), so each is fetched once per workgroup; weights come straight from
+// memory, WD - 1 stages ahead.  Loads past a buffer's end return 0 and stages past the row are never
+// added, so no index is clamped.  blockIdx.x = token group + row group * token groups.
+template <int LAYOUT, int KT, int WD, int SD>
+__global__ __launch_bounds__(256, 4) void gemm_b32_prompt_kernel(PromptGemm p, int tgroups) {
+    constexpr bool Q8 = LAYOUT == LAYOUT_Q80;
+    constexpr int NW = Q8 ? 2 : 1;
+    static_assert(WD % 2 == 0 && WD % SD == 0, "ring slots and LDS buffers follow the unrolled stage");
+    __shared__ __align__(16) uint4 bs[2][4][KT][64];
+    // wave index through readfirstlane: the buffer offsets below are then scalar
     const int lane = threadIdx.x & 63, wv = wave_id_uniform();
-    const int g = lane >> 4, r = lane & 15;  // A/B lane (g, r); D lane (g, c = r)
-    // RT = 2: a wave covers 32 rows x 32 tokens, a workgroup 64 x 64; RT = 1 (matrices whose
-    // 32 x 32 tiles would leave a SIMD one wave): 16 rows x 32 tokens, a workgroup 64 x 32
-    const int row0 = RT == 2 ? blockIdx.x * 64 + (wv & 1) * 32 : blockIdx.x * 64 + wv * 16;
-    const int tok0 = RT == 2 ? blockIdx.y * 64 + (wv >> 1) * 32 : blockIdx.y * 32;
-    if (row0 >= p.M || tok0 >= p.N) return;  // wave-uniform; the kernel has no barriers
-    const int K = 32 * p.nb, nq = (p.nb + 3) / 4;
-    int rt[RT];
-#pragma unroll
-    for (int i = 0; i < RT; i++) rt[i] = min(row0 / 16 + i, p.tiles16 - 1);  // storage is padded to 16 rows
-    const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc((void*)p.w, 0, (int)p.w_bytes, 0x00020000);
-    const int n16 = (p.N + 15) / 16;  // 16-token tiles of the repacked activations
-    const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc((void*)p.xm, 0, n16 * K * 16, 0x00020000);
+    const int g = lane >> 4, r = lane & 15;
+    const int t16 = blockIdx.x / tgroups * 4 + wv, tt = blockIdx.x % tgroups * KT;  // row tile, first token tile
+    const int nq = (p.nb + 3) / 4, n16 = (p.N + 15) / 16;
+    const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc((void*)p.xh, 0, n16 * nq * 4096, 0x00020000);
     const __amdgpu_buffer_rsrc_t sres = __builtin_amdgcn_make_buffer_rsrc((void*)p.xsm, 0, n16 * nq * 256, 0x00020000);
-    int tt[2];  // 16-token tiles (repacked layout), clamped into the buffer
-#pragma unroll
-    for (int k = 0; k < 2; k++) tt[k] = min(tok0 / 16 + k, n16 - 1);
-    // per-lane parts of the addresses
-    int nvo[RT], svo[RT];
-#pragma unroll
-    for (int i = 0; i < RT; i++) {
-        if constexpr (LAYOUT == LAYOUT_R16) {
-            nvo[i] = r * 16 + 4 * g;  // + 256 j within the quad
-            svo[i] = 1024 + 32 * g;   // scales [row / 4][j][row % 4]
-        } else {
-            const int sub = rt[i] & 3;
-            nvo[i] = (16 * sub + r) * 16 + 4 * g;  // + 1024 * (block % 8)
-            svo[i] = 8192 + (16 * sub + 4 * g) * 8;  // scales [row][block % 4], + 512 per half-chunk
-        }
+    // the row tile's storage (clamped into the padded rows) and this lane's offsets in a quad
+    const int tile_bytes = LAYOUT == LAYOUT_R64 ? p.groups * kQ40ChunkBytes : p.groups * 8 * r16_quad_bytes(Q8);
+    const int ts = min(t16, p.tiles16 - 1), sub = ts & 3;
+    const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(p.w + (size_t)(LAYOUT == LAYOUT_R64 ? ts >> 2 : ts) * tile_bytes), 0, tile_bytes, 0x00020000);
+    int nvo, svo;
+    if constexpr (LAYOUT == LAYOUT_R64) {
+        nvo = (16 * sub + r) * 16 + 4 * g;        // + 1024 * (block % 8)
+        svo = 8192 + (16 * sub + r) * 8 + 2 * g;  // scales [row][block % 4], + 512 per half-chunk
+    } else {
+        nvo = r * 16 + 4 * g;                                       // + 256 j within the quad
+        svo = NW * 1024 + 2 * (16 * (r >> 2) + 4 * g + (r & 3));  // scales [row / 4][block][row % 4]
     }
-    auto tile_base = [&](int i, int qd) -> int {
-        if constexpr (LAYOUT == LAYOUT_R16)
-            return (rt[i] * p.groups + (qd >> 3)) * kQ40ChunkBytes + (qd & 7) * kQ40R16QuadBytes;
-        else
-            return ((rt[i] >> 2) * p.groups + (qd >> 1)) * kQ40ChunkBytes;
-    };
-    uint32_t nib[D][RT][4], sw[D][RT][8], xa[D][2][4], xb[D][2][4];
-    float4 xsv[D][2];
-#define NC_PQ_LOAD(QD, SLOT)                                                                                    \
-    do {                                                                                                        \
-        const int qd_ = min((QD), nq - 1);                                                                      \
-        _Pragma("unroll") for (int i = 0; i < RT; i++) {                                                         \
-            const int tb_ = tile_base(i, qd_);                                                                  \
-            _Pragma("unroll") for (int j = 0; j < 4; j++) {                                                     \
-                const int jo_ = LAYOUT == LAYOUT_R16 ? 256 * j : 1024 * ((qd_ & 1) * 4 + j);                   \
-                nib[SLOT][i][j] = __builtin_amdgcn_raw_buffer_load_b32(wres, nvo[i] + jo_, tb_, 0);             \
-            }                                                                                                   \
-            const int so_ = LAYOUT == LAYOUT_R16 ? 0 : 512 * (qd_ & 1);                                         \
-            const uint4 s0_ = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(wres, svo[i] + so_, tb_, 0)); \
-            const uint4 s1_ = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(wres, svo[i] + so_ + 16, tb_, 0)); \
-            sw[SLOT][i][0] = s0_.x; sw[SLOT][i][1] = s0_.y; sw[SLOT][i][2] = s0_.z; sw[SLOT][i][3] = s0_.w;     \
-            sw[SLOT][i][4] = s1_.x; sw[SLOT][i][5] = s1_.y; sw[SLOT][i][6] = s1_.z; sw[SLOT][i][7] = s1_.w;     \
-        }                                                                                                       \
-        _Pragma("unroll") for (int k = 0; k < 2; k++) {                                                         \
-            _Pragma("unroll") for (int j = 0; j < 4; j++) {                                                     \
-                const uint2 v_ = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(                \
-                    xres, lane * 8, (tt[k] * p.nb + 4 * qd_ + j) * 512, 0));                                    \
-                xa[SLOT][k][j] = v_.x;                                                                          \
-                xb[SLOT][k][j] = v_.y;                                                                          \
-            }                                                                                                   \
-            xsv[SLOT][k] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(                   \
-                sres, r * 16, (tt[k] * nq + qd_) * 256, 0));                                                    \
-        }                                                                                                       \
-    } while (0)
-    float acc[RT][2][4];
+    // this wave's share of a stage's units: token tile wv % KT, blocks wv / KT, + 4 / KT, ...
+    const int uk = wv % KT, uj = wv / KT;
+    const int ubase = (tt + uk) * nq * 4096 + uj * 1024;
+    uint32_t wd[WD][4][NW], sw[WD];
+    float xsr[WD][KT];
+    uint4 st[SD][KT];
+#define NC_PB_UNITS(S, SLOT)                                                                                       \
+    _Pragma("unroll") for (int u = 0; u < KT; u++) st[SLOT][u] = __builtin_bit_cast(                               \
+        uint4, __builtin_amdgcn_raw_buffer_load_b128(xres, lane * 16 + u * (4 / KT) * 1024, ubase + (S) * 4096, 0));
+#define NC_PB_WEIGHTS(S, SLOT)                                                                                     \
+    {                                                                                                              \
+        const int h_ = LAYOUT == LAYOUT_R64 ? ((S) & 1) : 0;                                                       \
+        const int qo_ = LAYOUT == LAYOUT_R64 ? ((S) >> 1) * kQ40ChunkBytes : (S) * r16_quad_bytes(Q8);             \
+        _Pragma("unroll") for (int j = 0; j < 4; j++) _Pragma("unroll") for (int x = 0; x < NW; x++)               \
+            wd[SLOT][j][x] = __builtin_amdgcn_raw_buffer_load_b32(                                                 \
+                wres, nvo + (LAYOUT == LAYOUT_R64 ? 1024 : 256) * j + 1024 * x, qo_ + 4096 * h_, 0);               \
+        sw[SLOT] = __builtin_amdgcn_raw_buffer_load_b16(wres, svo, qo_ + 512 * h_, 0);                             \
+        _Pragma("unroll") for (int k = 0; k < KT; k++) xsr[SLOT][k] = __builtin_bit_cast(                          \
+            float, __builtin_amdgcn_raw_buffer_load_b32(sres, lane * 4, ((tt + k) * nq + (S)) * 256, 0));          \
+    }
+    uint32_t one = 0x64006400u;  // two f16 1024
+    asm("" : "+v"(one));
+    p_v4f acc[KT];
 #pragma unroll
-    for (int i = 0; i < RT; i++)
+    for (int k = 0; k < KT; k++) acc[k] = p_v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    const p_v16f zero16 = {};
+    const p_v4f zero4 = {};
 #pragma unroll
-        for (int k = 0; k < 2; k++)
+    for (int b = 0; b < WD; b++) {
+        if (b < SD) NC_PB_UNITS(b, b)
+        if (b < WD - 1) NC_PB_WEIGHTS(b, b)
+    }
 #pragma unroll
-            for (int v = 0; v < 4; v++) acc[i][k][v] = 0.0f;
-    const long minus8 = (long)0xF8F8F8F8F8F8F8F8ull;
-    const p_v4i zero = {0, 0, 0, 0};
+    for (int u = 0; u < KT; u++) bs[0][u * (4 / KT) + uj][uk][lane] = st[0][u];
+    __syncthreads();
+    for (int s0 = 0; s0 < nq; s0 += WD) {
 #pragma unroll
-    for (int s = 0; s < D - 1; s++) NC_PQ_LOAD(s, s);
-    for (int q0 = 0; q0 < nq; q0 += D) {
+        for (int b = 0; b < WD; b++) {
+            const int s = s0 + b;
+            if (s >= nq) break;  // uniform over the workgroup
+            NC_PB_UNITS(s + SD, b % SD)  // that slot's stage is in LDS
+            NC_PB_WEIGHTS(s + WD - 1, (b + WD - 1) % WD)
+            const float ws = f16_to_f32((uint16_t)sw[b]);
+            p_h8 a[4];
 #pragma unroll
-        for (int s = 0; s < D; s++) {
-            const int qd = q0 + s;
-            NC_PQ_LOAD(qd + D - 1, (s + D - 1) % D);
-            if (qd < nq) {  // uniform
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    if (4 * qd + j >= p.nb) break;  // uniform
-                    long bx[2];
-                    p_v4i corr[2];
-                    float xsj[2];
-#pragma unroll
-                    for (int k = 0; k < 2; k++) {
-                        bx[k] = (long)((uint64_t)xa[s][k][j] | ((uint64_t)xb[s][k][j] << 32));
-                        corr[k] = __builtin_amdgcn_mfma_i32_16x16x32_i8(minus8, bx[k], zero, 0, 0, 0);
-                        xsj[k] = j == 0 ? xsv[s][k].x : j == 1 ? xsv[s][k].y : j == 2 ? xsv[s][k].z : xsv[s][k].w;
-                    }
-#pragma unroll
-                    for (int i = 0; i < RT; i++) {
-                        const uint32_t wn = nib[s][i][j];
-                        const long a = (long)((uint64_t)(wn & 0x0F0F0F0Fu) | ((uint64_t)((wn >> 4) & 0x0F0F0F0Fu) << 32));
-                        float ws[4];
-#pragma unroll
-                        for (int v = 0; v < 4; v++) {
-                            // R16: [g][j][v] halves; R64: [v][j] halves
-                            const uint32_t dw = LAYOUT == LAYOUT_R16 ? sw[s][i][2 * j + (v >> 1)] : sw[s][i][2 * v + (j >> 1)];
-                            const int hi = LAYOUT == LAYOUT_R16 ? (v & 1) : (j & 1);
-                            ws[v] = f16_to_f32((uint16_t)(hi ? dw >> 16 : dw & 0xffff));
-                        }
-#pragma unroll
-                        for (int k = 0; k < 2; k++) {
-                            const p_v4i d = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, bx[k], corr[k], 0, 0, 0);
-#pragma unroll
-                            for (int v = 0; v < 4; v++) acc[i][k][v] = acc[i][k][v] + (ws[v] * xsj[k]) * (float)d[v];
-                        }
-                    }
-                }
+            for (int j = 0; j < 4; j++) {
+                if constexpr (Q8) a[j] = unpack_q80(wd[b][j][0], wd[b][j][NW - 1], one);
+                else a[j] = unpack_q40(wd[b][j][0], one);
             }
+#pragma unroll
+            for (int k = 0; k < KT; k++) {
+                // the quad's matrix instructions of one token tile back to back, then its chains: the
+                // first results are there when the last one has issued, so neither waits
+                p_v4f d[4];
+                const p_v16f sc = __builtin_amdgcn_mfma_f32_16x16x1f32(ws, xsr[b][k], zero16, 0, 0, 0);
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    d[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[j], __builtin_bit_cast(p_h8, bs[b & 1][j][k][lane]),
+                                                                  zero4, 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+#pragma unroll
+                    for (int v = 0; v < 4; v++) acc[k][v] = acc[k][v] + sc[4 * j + v] * d[j][v];
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            // the other buffer was last read a stage ago, before the barrier that ended that stage
+#pragma unroll
+            for (int u = 0; u < KT; u++) bs[(b + 1) & 1][u * (4 / KT) + uj][uk][lane] = st[(b + 1) % SD][u];
+            __syncthreads();
         }
     }
-#undef NC_PQ_LOAD
+#undef NC_PB_UNITS
+#undef NC_PB_WEIGHTS
 #pragma unroll
-    for (int k = 0; k < 2; k++) {
-        const int n = tok0 + 16 * k + r;
+    for (int k = 0; k < KT; k++) {
+        const int n = (tt + k) * 16 + r, row = t16 * 16 + 4 * g;
         if (n >= p.N) continue;
+        float* o = p.out + (size_t)n * p.ld_out + row;
+        if (row + 3 < p.M && (p.ld_out & 3) == 0) {
+            *(float4*)o = make_float4(acc[k][0], acc[k][1], acc[k][2], acc[k][3]);
+        } else {
 #pragma unroll
-        for (int i = 0; i < RT; i++) {
-            const int row = row0 + 16 * i + 4 * g;
-            float* o = p.out + (size_t)n * p.ld_out + row;
-            if (row + 3 < p.M && (p.ld_out & 3) == 0) {
-                *(float4*)o = make_float4(acc[i][k][0], acc[i][k][1], acc[i][k][2], acc[i][k][3]);
-            } else {
-#pragma unroll
-                for (int v = 0; v < 4; v++)
-                    if (row + v < p.M) o[v] = acc[i][k][v];
-            }
+            for (int v = 0; v < 4; v++)
+                if (row + v < p.M) o[v] = acc[k][v];
         }
     }
 }
 
-// Row tiles per wave: 2 (32 x 32 wave tiles) when that gives every SIMD at least two waves
-// (2048 waves on 256 CUs), else 1 (16 x 32: twice the waves for the same work).
-static int prompt_row_tiles(int64_t rows, int N) {
-    return ((rows + 31) / 32) * ((N + 31) / 32) >= 2048 ? 2 : 1;
+template <int LAYOUT>
+static void launch_b32_prompt(const PromptGemm& p, hipStream_t st) {
+    const int64_t rt = (p.M + 15) / 16, n16 = (p.N + 15) / 16;
+    auto go = [&]<int KT, int WD, int SD>() {
+        const int tg = (int)((n16 + KT - 1) / KT);
+        const dim3 grid((unsigned)((rt + 3) / 4 * tg));
+        NC_LAUNCH((gemm_b32_prompt_kernel<LAYOUT, KT, WD, SD>), grid, dim3(256), 0, st, p, tg);
+    };
+    // Token tiles per wave: a wave unpacks its weights once for all of them, but needs company: one wave
+    // issues a VALU instruction every 8 cycles at most, four share a SIMD's rate.  Measured (us, Q4_0, K = 4096,
+    // 4 / 2 / 1 token tiles): 28672 rows x 256 tokens 144 / 180 / 259, x 64 (448 workgroups) 57 / 63 / 80;
+    // 6144 x 256 (384) 55 / 48 / 67; 6144 x 128 (384 with 2) 46 / 38 / 40; 4096 x 128 (256) 46 / 32 / 28.
+    const int64_t g4 = (rt + 3) / 4;
+    if (n16 > 2 && g4 * ((n16 + 3) / 4) >= 448) go.template operator()<4, 2, 1>();
+    else if (n16 > 1 && g4 * ((n16 + 1) / 2) >= 384) go.template operator()<2, 2, 1>();
+    else go.template operator()<1, 2, 2>();
 }
 
-int launch_gemm_prompt(const QMatDev& w, const int8_t* x, const float* xs, float* out, int ld_out, int N,
-                       hipStream_t st, const void* xm, const float* xsm) {
-    if (w.type != NC_TYPE_Q4_0 || (w.layout != LAYOUT_R16 && w.layout != LAYOUT_R64))
-        return fail(NC_EINVAL, "prompt matmul: Q4_0 matrices only");
-    if (!xm || !xsm) return fail(NC_EINVAL, "prompt matmul: repacked activations required");
-    if (N < 1 || (int64_t)N * w.cols >= (int64_t)1 << 31 || w.dev_bytes >= (int64_t)1 << 31)
+int launch_gemm_prompt(const QMatDev& w, float* out, int ld_out, int N, hipStream_t st, const void* xh,
+                       const float* xsm) {
+    const bool q40 = w.type == NC_TYPE_Q4_0 && (w.layout == LAYOUT_R16 || w.layout == LAYOUT_R64);
+    if (!q40 && !(w.type == NC_TYPE_Q8_0 && w.layout == LAYOUT_Q80))
+        return fail(NC_EINVAL, "prompt matmul: Q4_0 and Q8_0 matrices only");
+    if (!xh || !xsm) return fail(NC_EINVAL, "prompt matmul: repacked activations required");
+    if (N < 1 || (int64_t)N * w.cols >= (int64_t)1 << 30 || w.dev_bytes >= (int64_t)1 << 31)
         return fail(NC_ERANGE, "prompt matmul: operands exceed 2 GiB");
     PromptGemm p;
     p.w = w.dev;
-    p.w_bytes = w.dev_bytes;
     p.groups = (int)w.groups;
-    p.tiles16 = (int)(w.layout == LAYOUT_R16 ? w.tiles : 4 * w.tiles);
+    p.tiles16 = (int)(w.layout == LAYOUT_R64 ? 4 * w.tiles : w.tiles);
     p.M = (int)w.rows;
     p.nb = (int)(w.cols / 32);
     p.N = N;
     p.ld_out = ld_out;
-    p.x = x;
-    p.xs = xs;
-    p.xm = (const uint2*)xm;
-    p.xsm = (const float4*)xsm;
+    p.xh = (const uint8_t*)xh;
+    p.xsm = xsm;
     p.out = out;
-    if (prompt_row_tiles(w.rows, N) == 2) {
-        const dim3 grid((unsigned)((w.rows + 63) / 64), (unsigned)((N + 63) / 64));
-        if (w.layout == LAYOUT_R16) NC_LAUNCH((gemm_q4_0_prompt_kernel<LAYOUT_R16, 2, 2>), grid, dim3(256), 0, st, p);
-        else NC_LAUNCH((gemm_q4_0_prompt_kernel<LAYOUT_R64, 2, 2>), grid, dim3(256), 0, st, p);
-    } else {
-        const dim3 grid((unsigned)((w.rows + 63) / 64), (unsigned)((N + 31) / 32));
-        if (w.layout == LAYOUT_R16) NC_LAUNCH((gemm_q4_0_prompt_kernel<LAYOUT_R16, 2, 1>), grid, dim3(256), 0, st, p);
-        else NC_LAUNCH((gemm_q4_0_prompt_kernel<LAYOUT_R64, 2, 1>), grid, dim3(256), 0, st, p);
-    }
+    if (w.layout == LAYOUT_Q80) launch_b32_prompt<LAYOUT_Q80>(p, st);
+    else if (w.layout == LAYOUT_R16) launch_b32_prompt<LAYOUT_R16>(p, st);
+    else launch_b32_prompt<LAYOUT_R64>(p, st);
     NC_HIP(hipGetLastError());
     return NC_OK;
 }
@@ -235,6 +245,12 @@ int launch_gemm_prompt(const QMatDev& w, const int8_t* x, const float* xs, float
 // 4g..4g+3.  A wave covers 32 rows x 32 tokens, a workgroup 64 x 64; weights stay in the verify
 // layouts (R16K: 16-row tiles, chunks of 4 super-blocks; R64: 64-row tiles, one super-block per
 // chunk), each chunk 9 slots of [64 lanes x 16 B], slot 0 the header (d, dmin, 12 scale bytes).
+// Row tiles per wave: 2 (32 x 32 wave tiles) when that gives every SIMD at least two waves
+// (2048 waves on 256 CUs), else 1 (16 x 32: twice the waves for the same work).
+static int prompt_row_tiles(int64_t rows, int N) {
+    return ((rows + 31) / 32) * ((N + 31) / 32) >= 2048 ? 2 : 1;
+}
+
 struct PromptGemmK {
     const uint8_t* w = nullptr;
     int64_t w_bytes = 0;
@@ -505,6 +521,44 @@ __global__ void prompt_repack_kernel(const int8_t* x, const float* xs, int N, in
         }
         xam[id2] = make_float4(sa[0], sa[1], sa[2], sa[3]);
     }
+}
+
+// The same as f16 for gemm_b32_prompt_kernel: xh unit (tile t, block b of 4 nq, lane (g, c)) = token 16t +
+// c's elements 0, 2, 16, 18, 1, 3, 17, 19 + 4g of the block, xsm (t, quad, lane (j, c)) its scale of
+// block 4 quad + j; zero past N and past the row's blocks.  One thread per unit lane, then per scale.
+__global__ void prompt_repack_f16_kernel(const int8_t* x, const float* xs, int N, int nb, uint4* xh, float* xsm) {
+    const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int n16 = (N + 15) / 16, nbp = (nb + 3) / 4 * 4, K = 32 * nb;
+    const int64_t nx = (int64_t)n16 * nbp * 64;
+    if (id < nx) {
+        const int lane = (int)(id & 63), g = lane >> 4, c = lane & 15;
+        const int64_t tb = id >> 6;
+        const int b = (int)(tb % nbp), n = (int)(tb / nbp) * 16 + c;
+        p_h8 v = {};
+        if (n < N && b < nb) {
+            const int8_t* e = x + (size_t)n * K + 32 * b + 4 * g;
+            const char4 lo = *(const char4*)e, hi = *(const char4*)(e + 16);
+            v = p_h8{(_Float16)lo.x, (_Float16)lo.z, (_Float16)hi.x, (_Float16)hi.z,
+                     (_Float16)lo.y, (_Float16)lo.w, (_Float16)hi.y, (_Float16)hi.w};
+        }
+        xh[id] = __builtin_bit_cast(uint4, v);
+        return;
+    }
+    const int64_t id2 = id - nx;
+    if (id2 >= (int64_t)n16 * nbp * 16) return;
+    const int c = (int)(id2 & 15), j = (int)(id2 >> 4) & 3;
+    const int64_t tq = id2 >> 6;
+    const int b = (int)(tq % (nbp / 4)) * 4 + j, n = (int)(tq / (nbp / 4)) * 16 + c;
+    xsm[id2] = n < N && b < nb ? xs[(size_t)n * nb + b] : 0.0f;
+}
+
+int launch_prompt_repack_f16(const int8_t* x, const float* xs, int N, int K, void* xh, float* xsm, hipStream_t st) {
+    const int nb = K / 32;
+    const int64_t total = (int64_t)((N + 15) / 16) * ((nb + 3) / 4 * 4) * 80;
+    NC_LAUNCH(prompt_repack_f16_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, x, xs, N, nb,
+              (uint4*)xh, xsm);
+    NC_HIP(hipGetLastError());
+    return NC_OK;
 }
 
 int launch_prompt_repack(const int8_t* x, const float* xs, int N, int K, void* xm, float* xsm, hipStream_t st,

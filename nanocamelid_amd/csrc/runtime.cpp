@@ -1157,6 +1157,7 @@ static int sample_session_rows(nc_session* s, int row0, int rows, float temp, co
 static bool prompt_matrix_ok(const QMatDev& q) {
     if (q.type == NC_TYPE_Q4_0) return q.layout == LAYOUT_R16 || q.layout == LAYOUT_R64;
     if (q.type == NC_TYPE_Q4_K) return q.layout == LAYOUT_R16K || q.layout == LAYOUT_R64;
+    if (q.type == NC_TYPE_Q8_0) return q.dev_bytes < (int64_t)1 << 31;  // larger ones in 16-token slices
     return false;
 }
 
@@ -1168,7 +1169,7 @@ static int slice_tokens(const QMatDev& q, int n) { return q.type == NC_TYPE_Q6_K
 // values of Q4_0 and the mins of Q4_K and Q5_K).
 static bool needs_block_sums(const QMatDev& q) { return q.type != NC_TYPE_Q6_K && q.type != NC_TYPE_Q8_0; }
 
-// Prompt passes take every layer matrix on a prompt kernel, or Q5_K, Q6_K and Q8_0 ones in 16-row slices.
+// Prompt passes take every layer matrix on a prompt kernel, or Q5_K and Q6_K ones on the verify kernels.
 static bool prompt_path_ok(const nc_model* m) {
     for (const LayerDev& L : m->layers)
         for (const QMatDev* q : L.all())
@@ -1178,14 +1179,16 @@ static bool prompt_path_ok(const nc_model* m) {
     return true;
 }
 
-// Prompt matmul of n tokens (Q4_0 or Q4_K) over activations repacked into xm / xsm (/ xam).
+// Prompt matmul of n tokens (Q4_0, Q8_0 or Q4_K) over activations repacked into xm / xsm (/ xam).
 static int prompt_matmul(const QMatDev& w, const int8_t* xq, const float* xs, float* out, int ld_out, int n,
                          hipStream_t st, int8_t* xm, float* xsm, float* xam) {
-    const bool k = w.type == NC_TYPE_Q4_K;
-    int rc = launch_prompt_repack(xq, xs, n, (int)w.cols, xm, xsm, st, k ? xam : nullptr);
-    if (rc) return rc;
-    return k ? launch_gemm_prompt_q4k(w, out, ld_out, n, st, xm, xsm, xam)
-             : launch_gemm_prompt(w, xq, xs, out, ld_out, n, st, xm, xsm);
+    int rc;
+    if (w.type == NC_TYPE_Q4_K) {
+        if ((rc = launch_prompt_repack(xq, xs, n, (int)w.cols, xm, xsm, st, xam))) return rc;
+        return launch_gemm_prompt_q4k(w, out, ld_out, n, st, xm, xsm, xam);
+    }
+    if ((rc = launch_prompt_repack_f16(xq, xs, n, (int)w.cols, xm, xsm, st))) return rc;
+    return launch_gemm_prompt(w, out, ld_out, n, st, xm, xsm);
 }
 
 static int ensure_prompt_bufs(nc_session* s) {
@@ -1201,7 +1204,7 @@ static int ensure_prompt_bufs(nc_session* s) {
         (rc = dev_alloc(s->allocs, &s->p_q, R * c.attention_output_width)) ||
         (rc = dev_alloc(s->allocs, &s->p_scores, (size_t)kPromptGroup * c.head_count * s->ctx_stride)) ||
         (rc = dev_alloc(s->allocs, &s->p_toks, (size_t)s->max_ctx)) ||
-        (rc = dev_alloc(s->allocs, &s->p_pos, R / kPromptGroup)) || (rc = dev_alloc(s->allocs, &s->p_xm, R * s->maxw)) ||
+        (rc = dev_alloc(s->allocs, &s->p_pos, R / kPromptGroup)) || (rc = dev_alloc(s->allocs, &s->p_xm, 2 * R * prompt_cols(s->maxw))) ||
         (rc = dev_alloc(s->allocs, &s->p_xsm, R * ((s->maxw + 127) / 128) * 4)) ||
         (rc = dev_alloc(s->allocs, &s->p_xam, R * ((s->maxw + 127) / 128) * 4)))
         return rc;
@@ -1211,7 +1214,7 @@ static int ensure_prompt_bufs(nc_session* s) {
 
 // Prompt matmul of the pass's activations (repacked first into MFMA operand order).
 // A prompt pass's matmul into rows of stride ld (default: the matrix's rows): the MFMA prompt
-// kernels, or for Q5_K, Q6_K and Q8_0 matrices (no prompt kernel) the verify kernel on 16-row slices.
+// kernels, or for Q5_K and Q6_K matrices (no prompt kernel) the verify kernel.
 static int prompt_gemm(nc_session* s, const QMatDev& w, const int8_t* xq, const float* xs, float* out, int n,
                        int ld = 0) {
     if (ld == 0) ld = (int)w.rows;
@@ -1429,7 +1432,7 @@ int nc_ctx_create(int device, nc_ctx** out) {
         c->tp_cap = temperature_scratch_floats(16);
         e = hipMalloc((void**)&c->tp_scratch, c->tp_cap * sizeof(float));
     }
-    if (e == hipSuccess) e = hipMalloc((void**)&c->pxm, kPromptRows * kCtxScratchCols);
+    if (e == hipSuccess) e = hipMalloc((void**)&c->pxm, 2 * kPromptRows * (kCtxScratchCols + 128));
     if (e == hipSuccess) e = hipMalloc((void**)&c->pxsm, kPromptRows * (kCtxScratchCols / 128 + 1) * 4 * sizeof(float));
     if (e == hipSuccess) e = hipMalloc((void**)&c->pxam, kPromptRows * (kCtxScratchCols / 128 + 1) * 4 * sizeof(float));
     if (e != hipSuccess) {

@@ -7,7 +7,7 @@ import pytest
 import nanocamelid_amd as nc
 from oracle import oracle as O
 from tests import gguf_writer as GW
-from tests.gpu_util import q8_activations, random_q8_0
+from tests.gpu_util import q8_activations, random_q4_0, random_q8_0
 
 pytestmark = pytest.mark.gpu
 
@@ -45,3 +45,15 @@ def test_q6_k_tile_edges(ctx, M, K):
 def test_q8_0_tile_edges(ctx, M, K):
     w = random_q8_0(M, K, seed=M + K)
     check(ctx, nc.NC_TYPE_Q8_0, w, O.matmul_q8_0, M, K, [1, 2, 3, 4, 5, 6, 7, 8, 9, 16, 17, 50], 4)
+
+
+# the prompt matmul's wave tiles: 16 x 32 (few workgroups), 16 x 64 and 32 x 64 (many), on 16-row tiles and, from
+# 65536 rows of Q4_0, on 64-row tiles; K: one block, cut quads, an odd number of quads; ragged rows and tokens
+@pytest.mark.parametrize("qtype", ["q4_0", "q8_0"])
+@pytest.mark.parametrize("M,K,batches", [(17, 32, [17, 33, 64]), (200, 416, [40, 130, 300]), (16401, 96, [129, 66]),
+                                         (32785, 288, [130]), (65553, 96, [20, 65]), (20, 8224, [31, 49])])
+def test_prompt_block_matmul_wave_tiles(ctx, qtype, M, K, batches):
+    if qtype == "q4_0":
+        check(ctx, nc.NC_TYPE_Q4_0, random_q4_0(M, K, seed=M), O.matmul_q4_0, M, K, batches, 5)
+    else:
+        check(ctx, nc.NC_TYPE_Q8_0, random_q8_0(M, K, seed=M), O.matmul_q8_0, M, K, batches, 6)
