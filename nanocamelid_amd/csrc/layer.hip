@@ -909,11 +909,18 @@ enum AttnTier {
     AT_FUSED_1_512, AT_FUSED_3_256, AT_FUSED_4_256, AT_FUSED_5_256, AT_FUSED_3_512,  // one kernel
     AT_PV_32_256_X1, AT_PV_4_512, AT_PV_8_512, AT_PV_16_512, AT_PV_32_512,           // scores, then
     AT_PV_8_256, AT_PV_16_256, AT_PV_32_256,                                         // softmax + V
+    AT_TILES,                                                                        // 16-query tiles
     AT_TOO_LONG
 };
 
 static int attention_tier(const AttnParams& a) {
     const int len = a.max_pos + 1;  // the longest score row of the pass
+    // Tiles of 16 queries once a pass has work for most of the chip: 1024 units at head dim 128 (32 rows x 32
+    // heads, one 8B layer at positions 0 / 3000 / 7500: 195 / 298 / 500 -> 179 / 295 / 475 us; 256 rows
+    // 596 / 1170 / 2509 -> 387 / 662 / 1108), 2048 at 64 (64 x 32: 159 / 228 / 412 -> 129 / 225 / 379).  Below,
+    // its 16-row workgroups leave CUs idle: 1536 units at head dim 64 144 / 211 / 326 -> 129 / 220 / 368, 512 at
+    // 128 (16 rows, 8000 positions) 202 -> 304 us for the attention alone.
+    if (a.inv && len <= 16384 && (int64_t)a.N * a.H * a.hd >= 1024 * 128) return AT_TILES;
     if (len <= 1536) {
         // one kernel per pass: each (row, head) unit scores its own keys (rows up to 1536
         // positions: the units of a KV head, all on one XCD, re-read its keys from that XCD's
@@ -960,6 +967,7 @@ int launch_attention(const AttnParams& a, hipStream_t st) {
     if (a.split) return launch_attention_split(a, st);
     const int tier = attention_tier(a);
     if (tier == AT_TOO_LONG) return fail(NC_ERANGE, "attention: context longer than 16384 positions");
+    if (tier == AT_TILES) return launch_attention_tiles(a, st);
     const dim3 grid(a.N * a.H);
     if (tier <= AT_FUSED_3_512) {
 #define NC_FUSED(E, T)                                                                               \

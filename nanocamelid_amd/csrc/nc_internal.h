@@ -173,6 +173,7 @@ struct AttnParams {
     const int32_t* d_pos = nullptr;
     int N = 0, H = 0, Hkv = 0, hd = 0, max_ctx = 0, max_pos = 0;
     float scale = 0.f;
+    float* inv = nullptr;     // [N][H] 1 / softmax sum (launch_attention_tiles; null: per-unit kernels only)
     // split-position order (NC_ATTN_SPLIT): per (row, head, 64-position chunk) partials
     bool split = false;
     float* part_o = nullptr;   // [N][H][nchunks][hd]
@@ -180,6 +181,8 @@ struct AttnParams {
     int nchunks = 0;
 };
 int launch_attention(const AttnParams& a, hipStream_t stream);
+// The same outputs by tiles of 16 queries (attn_tile.hip), for passes with many (row, head) units.
+int launch_attention_tiles(const AttnParams& a, hipStream_t stream);
 // Launch variant of launch_attention: passes with equal values launch the same kernels with the
 // same grids and blocks (the kernels read the rows' positions from d_pos, not from max_pos), so
 // a captured pass replays correctly at every start position of its variant.
@@ -208,9 +211,7 @@ int launch_prompt_qkv_rope(const float* y, int N, int start, int aw, int kw, int
 int launch_prompt_residual(const float* y, float* hidden, int N, int d, hipStream_t stream);
 int launch_prompt_swiglu_q8(const float* y, int N, int F, int8_t* xq, float* xs, int32_t* xs8, hipStream_t stream,
                             bool split = false);
-int launch_prompt_positions(int32_t* d, int start, int stride, int count, hipStream_t stream);
 constexpr int kPromptRows = 256;   // tokens per prompt pass
-constexpr int kPromptGroup = 64;   // rows per attention launch inside a prompt pass (score buffer rows)
 constexpr int kPromptMin = 32;     // shorter prompts run as verify-sized passes
 int launch_argmax_final(const float* part_val, const int32_t* part_idx, int N, int ntiles, uint32_t* preds,
                         hipStream_t stream);

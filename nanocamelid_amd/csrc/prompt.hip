@@ -665,17 +665,4 @@ int launch_prompt_swiglu_q8(const float* y, int N, int F, int8_t* xq, float* xs,
     return NC_OK;
 }
 
-// Start positions of the attention row groups of a prompt pass: d[i] = start + i * stride.
-__global__ void prompt_positions_kernel(int32_t* d, int start, int stride, int count) {
-    const int i = threadIdx.x;
-    if (i < count) d[i] = start + i * stride;
-}
-
-int launch_prompt_positions(int32_t* d, int start, int stride, int count, hipStream_t st) {
-    if (count < 1 || count > 256) return fail(NC_EINVAL, "prompt positions: 1..256 groups");
-    NC_LAUNCH(prompt_positions_kernel, dim3(1), dim3(256), 0, st, d, start, stride, count);
-    NC_HIP(hipGetLastError());
-    return NC_OK;
-}
-
 }  // namespace nc

@@ -117,11 +117,13 @@ struct nc_session {
     int32_t* p_xs8 = nullptr;    // [R][maxw/32]
     float* p_y = nullptr;        // [R][max(q|k|v rows, 2F, d)] matmul outputs
     float* p_q = nullptr;        // [R][aw]
-    float* p_scores = nullptr;   // [kPromptGroup][H][ctx_stride]
+    float* p_scores = nullptr;   // [kPromptRows][H][ctx_stride]
     uint32_t* p_toks = nullptr;  // [max_ctx] the prompt's ids
-    int32_t* p_pos = nullptr;    // [R / kPromptGroup] start positions of the attention row groups
+    int32_t* p_pos = nullptr;    // start position of the pass
     int8_t* p_xm = nullptr;      // matmul activations repacked in MFMA operand order
     float* p_xsm = nullptr;
+    float* attn_inv = nullptr;   // [max_batch][H] 1 / softmax sum of the tiled attention
+    float* p_inv = nullptr;      // 1 / softmax sum of each (row, head)
     float* p_xam = nullptr;      // their block sums (Q4_K)
     std::vector<void*> allocs;
 };
@@ -939,6 +941,7 @@ static int pass_body(nc_session* s, int n, int64_t start_pos, bool head) {
         a.split = s->ctx->attn_order == NC_ATTN_SPLIT;
         a.part_o = s->attn_part_o;
         a.part_ml = s->attn_part_ml;
+        a.inv = s->attn_inv;
         a.nchunks = s->attn_chunks;
         stage_mark(s, ST_ATTENTION);
         if ((rc = launch_attention(a, st))) return rc;
@@ -1030,6 +1033,7 @@ static AttnParams pass_attention_shape(const nc_session* s, int n, int64_t start
     a.max_pos = (int)(start_pos + n - 1);
     a.split = s->ctx->attn_order == NC_ATTN_SPLIT;
     a.nchunks = s->attn_chunks;
+    a.inv = s->attn_inv;
     return a;
 }
 
@@ -1202,9 +1206,10 @@ static int ensure_prompt_bufs(nc_session* s) {
         (rc = dev_alloc(s->allocs, &s->p_xq, R * s->maxw)) || (rc = dev_alloc(s->allocs, &s->p_xs, R * (s->maxw / 32))) ||
         (rc = dev_alloc(s->allocs, &s->p_xs8, R * (s->maxw / 32))) || (rc = dev_alloc(s->allocs, &s->p_y, R * yw)) ||
         (rc = dev_alloc(s->allocs, &s->p_q, R * c.attention_output_width)) ||
-        (rc = dev_alloc(s->allocs, &s->p_scores, (size_t)kPromptGroup * c.head_count * s->ctx_stride)) ||
+        (rc = dev_alloc(s->allocs, &s->p_scores, R * c.head_count * s->ctx_stride)) ||
+        (rc = dev_alloc(s->allocs, &s->p_inv, R * c.head_count)) ||
         (rc = dev_alloc(s->allocs, &s->p_toks, (size_t)s->max_ctx)) ||
-        (rc = dev_alloc(s->allocs, &s->p_pos, R / kPromptGroup)) || (rc = dev_alloc(s->allocs, &s->p_xm, 2 * R * prompt_cols(s->maxw))) ||
+        (rc = dev_alloc(s->allocs, &s->p_pos, (size_t)1)) || (rc = dev_alloc(s->allocs, &s->p_xm, 2 * R * prompt_cols(s->maxw))) ||
         (rc = dev_alloc(s->allocs, &s->p_xsm, R * ((s->maxw + 127) / 128) * 4)) ||
         (rc = dev_alloc(s->allocs, &s->p_xam, R * ((s->maxw + 127) / 128) * 4)))
         return rc;
@@ -1259,17 +1264,16 @@ static int prompt_gateup(nc_session* s, const LayerDev& L, int n, int F) {
 // One prompt pass over n <= kPromptRows ids p_toks[off..off+n) at positions start..: the
 // layers of run_pass (run_layer_range_batch, inference.rs:3747-4111) with the MFMA prompt
 // matmul and the epilogues as separate kernels; no head (prefill_pass_batch discards the
-// prompt's logits).  Attention runs in row groups of kPromptGroup (the score rows).
+// prompt's logits).
 static int run_prompt_pass(nc_session* s, int off, int n, int64_t start) {
     nc_model* m = s->m;
     const nc_model_config& c = m->cfg;
     const int d = (int)c.embedding_length, aw = (int)c.attention_output_width, kw = (int)c.kv_width;
     const int F = (int)c.feed_forward_length, hd = (int)c.head_dim, Hkv = (int)c.head_count_kv;
     hipStream_t st = s->stream;
-    const int ngroups = (n + kPromptGroup - 1) / kPromptGroup;
     int rc;
     if ((rc = launch_embed(m->tok_emb, s->p_toks + off, n, d, s->p_hidden, st)) ||
-        (rc = launch_prompt_positions(s->p_pos, (int)start, kPromptGroup, ngroups, st)))
+        (rc = launch_set_pass_state(s->p_pos, (int)start, nullptr, nullptr, 0, st)))
         return rc;
     const size_t layer_kv = (size_t)Hkv * s->ctx_stride * hd;
     for (int64_t li = 0; li < c.block_count; li++) {
@@ -1281,26 +1285,24 @@ static int run_prompt_pass(nc_session* s, int off, int n, int64_t start) {
             (rc = launch_prompt_qkv_rope(s->p_y, n, (int)start, aw, kw, hd, (int)c.rope_dimension_count / 2,
                                          s->rope_tab, s->p_q, kc, vc, (int)s->ctx_stride, st)))
             return rc;
-        for (int gi = 0; gi < ngroups; gi++) {
-            const int g0 = gi * kPromptGroup, ng = std::min(kPromptGroup, n - g0);
-            AttnParams a;
-            a.q = s->p_q + (size_t)g0 * aw;
-            a.kcache = kc;
-            a.vcache = vc;
-            a.scores = s->p_scores;
-            a.xq = s->p_xq + (size_t)g0 * aw;
-            a.xs = s->p_xs + (size_t)g0 * (aw / 32);
-            a.xs8 = s->p_xs8 + (size_t)g0 * (aw / 32);
-            a.d_pos = s->p_pos + gi;
-            a.N = ng;
-            a.H = (int)c.head_count;
-            a.Hkv = Hkv;
-            a.hd = hd;
-            a.max_ctx = (int)s->ctx_stride;
-            a.max_pos = (int)(start + g0 + ng - 1);
-            a.scale = 1.0f / std::sqrt((float)hd);  // inference.rs:3927
-            if ((rc = launch_attention(a, st))) return rc;
-        }
+        AttnParams a;
+        a.q = s->p_q;
+        a.kcache = kc;
+        a.vcache = vc;
+        a.scores = s->p_scores;
+        a.inv = s->p_inv;
+        a.xq = s->p_xq;
+        a.xs = s->p_xs;
+        a.xs8 = s->p_xs8;
+        a.d_pos = s->p_pos;
+        a.N = n;
+        a.H = (int)c.head_count;
+        a.Hkv = Hkv;
+        a.hd = hd;
+        a.max_ctx = (int)s->ctx_stride;
+        a.max_pos = (int)(start + n - 1);
+        a.scale = 1.0f / std::sqrt((float)hd);  // inference.rs:3927
+        if ((rc = launch_attention(a, st))) return rc;
         if ((rc = prompt_gemm(s, L.wo, s->p_xq, s->p_xs, s->p_y, n)) ||
             (rc = launch_prompt_residual(s->p_y, s->p_hidden, n, d, st)) ||
             (rc = launch_rmsnorm_q8(s->p_hidden, L.ffn_norm, n, d, c.rms_norm_epsilon, s->p_xq, s->p_xs, s->p_xs8, st)) ||
@@ -1835,6 +1837,7 @@ int nc_session_create(nc_model* m, int64_t max_ctx, int32_t max_batch, nc_sessio
         (rc = dev_alloc(s->allocs, &s->scores, (size_t)B * c.head_count * s->ctx_stride)) ||
         (rc = dev_alloc(s->allocs, &s->attn_part_o, (size_t)B * c.head_count * s->attn_chunks * c.head_dim)) ||
         (rc = dev_alloc(s->allocs, &s->attn_part_ml, (size_t)B * c.head_count * s->attn_chunks * 2)) ||
+        (rc = dev_alloc(s->allocs, &s->attn_inv, (size_t)B * c.head_count)) ||
         (rc = dev_alloc(s->allocs, &s->logits, (size_t)B * c.vocab_size)) ||
         (rc = dev_alloc(s->allocs, &s->probs, (size_t)B * c.vocab_size)) ||
         (rc = dev_alloc(s->allocs, &s->qbuf, (size_t)B * c.vocab_size)) ||

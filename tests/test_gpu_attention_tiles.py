@@ -1,0 +1,37 @@
+"""The tiled attention of passes with many (row, head) units, at the edges of its 16-query tiles and
+16- and 256-position steps: bit-exact against the oracle's sequential attention."""
+import numpy as np
+import pytest
+
+import nanocamelid_amd as nc
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+# heads, KV heads, head dim and the chunk lengths of one prompt, each a pass of >= 1024 * 128 / hd units: rows
+# that cut a tile (35, 70, 101), tiles across two heads' rows, eight and one heads per KV head, starts
+# off the 16- and 256-position steps
+@pytest.mark.parametrize("H,Hkv,hd,chunks", [(32, 4, 128, [35, 70, 256, 33]), (32, 32, 128, [101, 48]),
+                                             (32, 8, 64, [70, 190, 67, 256]), (64, 8, 64, [35, 33, 200])])
+def test_tiled_attention_vs_oracle(H, Hkv, hd, chunks):
+    ctx = nc.Context(0)
+    spec = dict(layers=2, embedding_length=H * hd, head_count=H, head_count_kv=Hkv, feed_forward_length=256,
+                vocab_size=300, context_length=1024, tied=1, norm_mode=1)
+    img = nc.synth_gguf(**spec, seed=H + Hkv + hd)
+    gs = nc.Session(nc.Model(ctx, data=img), sum(chunks) + 16, 16)
+    os_ = O.Session(O.Model(data=img.tobytes(), nthreads=8), sum(chunks) + 16, 16)
+    pos = 0
+    for n in chunks:
+        toks = nc.uniform_prompt(pos + n, n, 300)
+        gs.prefill_pass_batch(toks, pos, want_logits=False)
+        for i in range(0, n, 16):
+            os_.prefill_pass_batch(toks[i:i + 16], pos + i)
+        pos += n
+    # layer 0's tiles feed layer 1's keys and values, which these logits read
+    batch = nc.uniform_prompt(7, 5, 300)
+    _, _, _, preds = gs.verify_greedy(batch, pos)
+    opreds, _, ologits = os_.verify_greedy(batch, pos, want_logits=True)
+    assert np.array_equal(preds, opreds)
+    for i in range(5):
+        assert np.array_equal(gs.logits(i).view(np.uint32), ologits[i].view(np.uint32)), i
