@@ -235,16 +235,28 @@ __device__ __forceinline__ int dot32_bcast_scaled(int acc, float& c, int xp, int
     return acc;
 }
 
+// A Q4_0 block's 32 weights as 8 dwords of signed bytes 16 * (nib - 8) (low nibbles, then high): the
+// nibble in a byte's upper half, its sign bit flipped, is that value, for as many operations as
+// masking out the unsigned nibbles.  The dot comes out times 16, exactly, and is shifted back; no sum of
+// the activations has to be loaded or broadcast to correct an offset.
+__device__ __forceinline__ void signed_q40(const uint4& v, int (&lo)[4], int (&hi)[4]) {
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        lo[i] = (int)(((w[i] << 4) & 0xF0F0F0F0u) ^ 0x80808080u);
+        hi[i] = (int)((w[i] & 0xF0F0F0F0u) ^ 0x80808080u);
+    }
+}
+
 // Term of token n (compile-time) for one block: t = (ws * xs) * (float)sum (nib - 8) * x.
 template <int n, bool Q8 = false>
 __device__ __forceinline__ float term_q40(const int* xp, const int* meta, const int (&lo)[4], const int (&hi)[4],
                                           float ws) {
-    // -8 * sum x: sum (nib-8)*x = sum nib*x - 8 sum x (Q8_0 weights are signed)
-    int d = Q8 ? 0 : bcast_i<8 + (n & 7)>(meta[n >> 3]);
+    int d = 0;
     float c;                                       // x_scale * ws (IEEE product, commutative)
     d = dot32_bcast_scaled<8 * (n & 1), n & 7>(d, c, xp[n >> 1], meta[n >> 3], ws, lo[0], lo[1], lo[2], lo[3], hi[0],
                                                 hi[1], hi[2], hi[3]);
-    return c * (float)d;  // == (ws * xs) * d
+    return c * (float)(Q8 ? d : d >> 4);  // == (ws * xs) * dot (Q4_0 weights come times 16)
 }
 
 // R64: a ring of D rounds of weights, scales and activations is kept in flight per wave.
@@ -258,13 +270,12 @@ __device__ __forceinline__ void terms_q40(float (&t)[NMAX], const int* xp, const
         (([&] {
              constexpr int n0 = 2 * P, n1 = 2 * P + 1;
              if constexpr (n1 < NMAX) {
-                 int d0 = Q8 ? 0 : bcast_i<8 + (n0 & 7)>(meta[n0 >> 3]);
-                 int d1 = Q8 ? 0 : bcast_i<8 + (n1 & 7)>(meta[n1 >> 3]);
+                 int d0 = 0, d1 = 0;
                  float c0, c1;  // x_scale * ws (meta[n0 >> 3] == meta[n1 >> 3]: n0, n1 differ in bit 0)
                  dot32_bcast_pair_scaled<n0 & 7, n1 & 7>(d0, d1, c0, c1, xp[P], meta[n0 >> 3], ws, lo[0], lo[1],
                                                          lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]);
-                 t[n0] = c0 * (float)d0;
-                 t[n1] = c1 * (float)d1;
+                 t[n0] = c0 * (float)(Q8 ? d0 : d0 >> 4);
+                 t[n1] = c1 * (float)(Q8 ? d1 : d1 >> 4);
              } else {
                  t[n0] = term_q40<n0, Q8>(xp, meta, lo, hi, ws);
              }
@@ -292,11 +303,11 @@ __global__ __launch_bounds__(64 * S) void gemm_q4_0_kernel(GemmParams p) {
 #pragma unroll
     for (int t = 0; t < TPW; t++) acc[t] = 0.0f;
     // per-lane activation addresses: pair q -> token 2q + (j16 >> 3), dword j16 & 7;
-    // meta: lanes 0..7 read x_scale, lanes 8..15 read -8*sum(x) of token 8q + (j16 & 7)
+    // meta: x_scale of token 8q + (j16 & 7)
     const int* xbase = (const int*)p.x + (j16 & 7);
     const int xtok = j16 >> 3;
     const int mtok = j16 & 7;
-    const int* mbase = j16 >= 8 ? p.xs8 : (const int*)p.xs;
+    const int* mbase = (const int*)p.xs;
     const int nrounds = (nb + RB - 1) / RB;
 
     uint4 rw[D][U];
@@ -341,10 +352,8 @@ __global__ __launch_bounds__(64 * S) void gemm_q4_0_kernel(GemmParams p) {
                 for (int u = 0; u < U; u++) {
                     if (b0 + u < nb) {  // uniform
                         const uint4 v = rw[k][u];
-                        const int lo[4] = {(int)(v.x & 0x0F0F0F0Fu), (int)(v.y & 0x0F0F0F0Fu),
-                                           (int)(v.z & 0x0F0F0F0Fu), (int)(v.w & 0x0F0F0F0Fu)};
-                        const int hi[4] = {(int)((v.x >> 4) & 0x0F0F0F0Fu), (int)((v.y >> 4) & 0x0F0F0F0Fu),
-                                           (int)((v.z >> 4) & 0x0F0F0F0Fu), (int)((v.w >> 4) & 0x0F0F0F0Fu)};
+                        int lo[4], hi[4];
+                        signed_q40(v, lo, hi);
                         const uint32_t sw = u < 2 ? rs[k].x : rs[k].y;
                         const float ws = f16_to_f32((uint16_t)((u & 1) ? (sw >> 16) : (sw & 0xffff)));
                         // every token of the instantiation, without branches (tokens >= N read
@@ -652,23 +661,15 @@ __global__ __launch_bounds__(64 * (S * TPG + CW)) void gemm_q4_0_r16_kernel(Gemm
         __builtin_amdgcn_make_buffer_rsrc((void*)wt, 0, p.groups * CB, 0x00020000);
     const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc((void*)p.x, 0, N * p.K, 0x00020000);
     const __amdgpu_buffer_rsrc_t sres = __builtin_amdgcn_make_buffer_rsrc((void*)p.xs, 0, N * nb * 4, 0x00020000);
-    const __amdgpu_buffer_rsrc_t s8res = __builtin_amdgcn_make_buffer_rsrc((void*)p.xs8, 0, N * nb * 4, 0x00020000);
     // a quad's nibbles, then its 64 scales ([row / 4][block][row % 4]: this lane's is (j, i16))
     const int wvo = lane * 16, svo = 2 * (16 * (i16 >> 2) + 4 * j + (i16 & 3));
-    int xvo[NP], mvo[NM], mt[NM];
+    int xvo[NP], mvo[NM];
 #pragma unroll
     for (int q = 0; q < NP; q++) xvo[q] = (2 * q + xtok) * p.K + 32 * j + 4 * (i16 & 7);
 #pragma unroll
     for (int q = 0; q < NM; q++) {
         mvo[q] = ((8 * q + mtok) * nb + j) * 4;
-        mt[q] = min(8 * q + mtok, N - 1);
     }
-    // Block scales: lanes 0-7 of a row take xs, lanes 8-15 xs8.  For 3..8 rows two buffer
-    // loads and a select measured faster than one load through a per-lane pointer; for
-    // other widths the single clamped load is faster.
-    constexpr bool kMetaBuf = Q8 || (NMAX >= 3 && NMAX <= 8);
-    const bool meta_s = Q8 || i16 < 8;
-    const int* mbase = meta_s ? (const int*)p.xs : p.xs8;
 #define NC_R16_LOAD(R, SLOT)                                                                         \
     do {                                                                                             \
         const int qd0_ = min(min((R), nrounds - 1) * QR + wave * U, qmax);                           \
@@ -683,19 +684,7 @@ __global__ __launch_bounds__(64 * (S * TPG + CW)) void gemm_q4_0_r16_kernel(Gemm
             _Pragma("unroll") for (int q = 0; q < NP; q++) rx[SLOT][u][q] = (int)                     \
                 __builtin_amdgcn_raw_buffer_load_b32(xres, xvo[q] + 128 * (qd0_ + u), 0, 0);         \
             _Pragma("unroll") for (int q = 0; q < NM; q++) {                                         \
-                if constexpr (kMetaBuf) {                                                            \
-                    const int mo_ = mvo[q] + 16 * (qd0_ + u);                                        \
-                    const int ms_ = (int)__builtin_amdgcn_raw_buffer_load_b32(sres, mo_, 0, 0);      \
-                    if constexpr (Q8) {                                                              \
-                        rm[SLOT][u][q] = ms_;                                                        \
-                    } else {                                                                         \
-                        const int m8_ = (int)__builtin_amdgcn_raw_buffer_load_b32(s8res, mo_, 0, 0); \
-                        rm[SLOT][u][q] = meta_s ? ms_ : m8_;                                         \
-                    }                                                                                \
-                } else {                                                                             \
-                    const int b_ = min(4 * (qd0_ + u) + j, nb - 1);                                  \
-                    rm[SLOT][u][q] = mbase[(size_t)mt[q] * nb + b_];                                 \
-                }                                                                                    \
+                rm[SLOT][u][q] = (int)__builtin_amdgcn_raw_buffer_load_b32(sres, mvo[q] + 16 * (qd0_ + u), 0, 0); \
             }                                                                                        \
         }                                                                                            \
     } while (0)
@@ -722,12 +711,7 @@ __global__ __launch_bounds__(64 * (S * TPG + CW)) void gemm_q4_0_r16_kernel(Gemm
                             lo[0] = (int)v.x, lo[1] = (int)v.y, lo[2] = (int)v.z, lo[3] = (int)v.w;
                             hi[0] = (int)v1.x, hi[1] = (int)v1.y, hi[2] = (int)v1.z, hi[3] = (int)v1.w;
                         } else {
-                            const uint32_t w4[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                            for (int i = 0; i < 4; i++) {
-                                lo[i] = (int)(w4[i] & 0x0F0F0F0Fu);
-                                hi[i] = (int)((w4[i] >> 4) & 0x0F0F0F0Fu);
-                            }
+                            signed_q40(v, lo, hi);
                         }
                         const float ws = f16_to_f32((uint16_t)rs[k][u]);
                         float* dst = buf + ((size_t)((wave * U + u) * 4 + j) * NMAX) * 16 + i16;

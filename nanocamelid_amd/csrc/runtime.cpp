@@ -1169,9 +1169,12 @@ static bool prompt_matrix_ok(const QMatDev& q) {
 // groups share a launch), the others 16.
 static int slice_tokens(const QMatDev& q, int n) { return q.type == NC_TYPE_Q6_K ? n : 16; }
 
-// Whether the verify kernels of a matrix read the activations' block sums (the offset of the unsigned
-// values of Q4_0 and the mins of Q4_K and Q5_K).
-static bool needs_block_sums(const QMatDev& q) { return q.type != NC_TYPE_Q6_K && q.type != NC_TYPE_Q8_0; }
+// Whether the verify kernels of a matrix read the activations' block sums: for the mins of Q4_K and
+// Q5_K, and for the offset of the unsigned Q4_0 nibbles on the int8 MFMA path.
+static bool needs_block_sums(const nc_ctx* ctx, const QMatDev& q) {
+    return q.type == NC_TYPE_Q4_K || q.type == NC_TYPE_Q5_K ||
+           (q.type == NC_TYPE_Q4_0 && ctx->gemm_kernel == NC_GEMM_KERNEL_MFMA);
+}
 
 // Prompt passes take every layer matrix on a prompt kernel, or Q5_K and Q6_K ones on the verify kernels.
 static bool prompt_path_ok(const nc_model* m) {
@@ -1556,7 +1559,7 @@ int nc_matmul_quantized_batch(nc_ctx* ctx, const nc_qmat* w, const int8_t* x_i8,
     for (int i = 0; i < batch_size; i += slice) {
         const int nb = std::min(slice, batch_size - i);
         int rc = NC_OK;
-        if (needs_block_sums(w->m) &&
+        if (needs_block_sums(ctx, w->m) &&
             ((rc = ensure_xsum(ctx, (size_t)nb * (cols / 32))) ||
              (rc = launch_block_sums(x_i8 + (size_t)i * cols, nb, (int)cols, ctx->xsum, st))))
             return rc;
