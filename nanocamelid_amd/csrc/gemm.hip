@@ -169,6 +169,32 @@ __device__ __forceinline__ int dot32_bcast(int acc, int xp, int w0, int w1, int 
     return acc;
 }
 
+// The two 32-value dots of a K-quant pair: a0 += low-half weights . lanes 0-7 of xp, a1 += high-half
+// weights . lanes 8-15; the chains alternate, so neither waits on its accumulator.
+__device__ __forceinline__ void dot64_bcast(int& a0, int& a1, int xp, const int (&lo)[8], const int (&hi)[8]) {
+    asm("s_nop 1\n\t"
+        "v_dot4c_i32_i8_dpp %0, %2, %3 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
+        "v_dot4c_i32_i8_dpp %1, %2, %11 row_newbcast:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_dot4c_i32_i8_dpp %0, %2, %4 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
+        "v_dot4c_i32_i8_dpp %1, %2, %12 row_newbcast:9 row_mask:0xf bank_mask:0xf\n\t"
+        "v_dot4c_i32_i8_dpp %0, %2, %5 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
+        "v_dot4c_i32_i8_dpp %1, %2, %13 row_newbcast:10 row_mask:0xf bank_mask:0xf\n\t"
+        "v_dot4c_i32_i8_dpp %0, %2, %6 row_newbcast:3 row_mask:0xf bank_mask:0xf\n\t"
+        "v_dot4c_i32_i8_dpp %1, %2, %14 row_newbcast:11 row_mask:0xf bank_mask:0xf\n\t"
+        "v_dot4c_i32_i8_dpp %0, %2, %7 row_newbcast:4 row_mask:0xf bank_mask:0xf\n\t"
+        "v_dot4c_i32_i8_dpp %1, %2, %15 row_newbcast:12 row_mask:0xf bank_mask:0xf\n\t"
+        "v_dot4c_i32_i8_dpp %0, %2, %8 row_newbcast:5 row_mask:0xf bank_mask:0xf\n\t"
+        "v_dot4c_i32_i8_dpp %1, %2, %16 row_newbcast:13 row_mask:0xf bank_mask:0xf\n\t"
+        "v_dot4c_i32_i8_dpp %0, %2, %9 row_newbcast:6 row_mask:0xf bank_mask:0xf\n\t"
+        "v_dot4c_i32_i8_dpp %1, %2, %17 row_newbcast:14 row_mask:0xf bank_mask:0xf\n\t"
+        "v_dot4c_i32_i8_dpp %0, %2, %10 row_newbcast:7 row_mask:0xf bank_mask:0xf\n\t"
+        "v_dot4c_i32_i8_dpp %1, %2, %18 row_newbcast:15 row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 2"
+        : "+v"(a0), "+v"(a1)
+        : "v"(xp), "v"(lo[0]), "v"(lo[1]), "v"(lo[2]), "v"(lo[3]), "v"(lo[4]), "v"(lo[5]), "v"(lo[6]), "v"(lo[7]),
+          "v"(hi[0]), "v"(hi[1]), "v"(hi[2]), "v"(hi[3]), "v"(hi[4]), "v"(hi[5]), "v"(hi[6]), "v"(hi[7]));
+}
+
 template <int J>
 __device__ __forceinline__ int bcast_i(int v) {
     return __builtin_amdgcn_mov_dpp(v, 0x150 + J, 0xf, 0xf, false);
@@ -1056,10 +1082,18 @@ __global__ __launch_bounds__(64 * S) void gemm_q4_k_kernel(GemmParams p) {
 // row r) add them in super-block order.  Loads are unconditional buffer loads: weights at a
 // scalar chunk offset (clamped to the padded quads), activations and meta at per-lane offsets
 // range-checked against [N][K] and [N][K/32] (a token past N reads 0 and is never stored).
-template <int NMAX, int S, int D>
+//
+// Q5: Q5_K super-blocks, chunks of 11 slots (slots 1-2 the 32 high-bit bytes, slots 3-10 the nibbles):
+// the high bit is OR'd into the unpacked nibble, the rest is the same.
+//
+// p.xs8 null (operator calls, whose activations come without block sums): the workgroup sums its
+// activations' blocks itself, into LDS beside the terms, while its first weights arrive.  A separate launch for
+// them cost 2 us of device and 3 us of host time before a 9 us matmul.
+template <int NMAX, int S, int D, bool Q5 = false>
 __global__ __launch_bounds__(64 * S) void gemm_q4_k_r16_kernel(GemmParams p) {
     static_assert(16 * NMAX <= 64 * S, "chain threads must fit the workgroup");
-    extern __shared__ float lds[];  // [2][4*S][NMAX][16] super-block terms
+    constexpr int NSLOT = Q5 ? 11 : 9, QS = Q5 ? 3 : 1, CHUNK = NSLOT * 1024;
+    extern __shared__ float lds[];  // [2][4*S][NMAX][16] super-block terms, then [N][nb] block sums
     const int tile = blockIdx.x;
     const int wave = wave_id_uniform();
     const int lane = threadIdx.x & 63;
@@ -1068,21 +1102,24 @@ __global__ __launch_bounds__(64 * S) void gemm_q4_k_r16_kernel(GemmParams p) {
     const int nquads = (nsb + 3) / 4;    // padded to p.groups quads per tile
     const int nrounds = (nquads + S - 1) / S;
     const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(p.w + (size_t)tile * p.groups * kQ4KChunkBytes), 0, p.groups * kQ4KChunkBytes, 0x00020000);
+        (void*)(p.w + (size_t)tile * p.groups * CHUNK), 0, p.groups * CHUNK, 0x00020000);
     const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc((void*)p.x, 0, N * p.K, 0x00020000);
     const __amdgpu_buffer_rsrc_t sres = __builtin_amdgcn_make_buffer_rsrc((void*)p.xs, 0, N * nb * 4, 0x00020000);
-    const __amdgpu_buffer_rsrc_t s8res = __builtin_amdgcn_make_buffer_rsrc((void*)p.xs8, 0, N * nb * 4, 0x00020000);
+    const bool own_sums = p.xs8 == nullptr;  // uniform
+    const __amdgpu_buffer_rsrc_t s8res =
+        __builtin_amdgcn_make_buffer_rsrc((void*)p.xs8, 0, own_sums ? 0 : N * nb * 4, 0x00020000);
+    float* sums = lds + 2 * 4 * S * NMAX * 16;
     const int wvo = lane * 16;
     const int xvo = q * 256 + j * 4;          // + n*K + c*64 + quad*1024
     const int mvo = q * 32 + (j & 7) * 4;     // + n*nb*4 + quad*128
     const bool meta_s = j < 8;
-    uint4 rw[D][9];
+    uint4 rw[D][NSLOT];
     int ax[D][NMAX][4], am[D][NMAX];
 #define NC_K16_LOAD(R, SLOT)                                                                         \
     do {                                                                                             \
         const int g_ = min(min((R), nrounds - 1) * S + wave, p.groups - 1);                          \
-        _Pragma("unroll") for (int i = 0; i < 9; i++) rw[SLOT][i] = __builtin_bit_cast(               \
-            uint4, __builtin_amdgcn_raw_buffer_load_b128(wres, wvo, g_ * kQ4KChunkBytes + i * 1024, 0)); \
+        _Pragma("unroll") for (int i = 0; i < NSLOT; i++) rw[SLOT][i] = __builtin_bit_cast(           \
+            uint4, __builtin_amdgcn_raw_buffer_load_b128(wres, wvo, g_ * CHUNK + i * 1024, 0)); \
         _Pragma("unroll") for (int n = 0; n < NMAX; n++) {                                           \
             _Pragma("unroll") for (int c = 0; c < 4; c++) ax[SLOT][n][c] = (int)                      \
                 __builtin_amdgcn_raw_buffer_load_b32(xres, xvo + n * p.K + c * 64 + g_ * 1024, 0, 0); \
@@ -1094,6 +1131,16 @@ __global__ __launch_bounds__(64 * S) void gemm_q4_k_r16_kernel(GemmParams p) {
     } while (0)
 #pragma unroll
     for (int k = 0; k < D - 1; k++) NC_K16_LOAD(k, k);
+    if (own_sums) {
+        for (int i = threadIdx.x; i < N * nb; i += 64 * S) {
+            const int* x = (const int*)(p.x + (size_t)(i / nb) * p.K) + 8 * (i % nb);
+            int sum = 0;
+#pragma unroll
+            for (int e = 0; e < 8; e++) sum = __builtin_amdgcn_sdot4(x[e], 0x01010101, sum, false);
+            sums[i] = (float)sum;
+        }
+        __syncthreads();
+    }
     float acc = 0.0f;
     const int cn = threadIdx.x >> 4, cr = threadIdx.x & 15;  // chain thread: token, row
     for (int r0 = 0; r0 < nrounds; r0 += D) {
@@ -1122,35 +1169,46 @@ __global__ __launch_bounds__(64 * S) void gemm_q4_k_r16_kernel(GemmParams p) {
                     sc[jj] = d * (float)sv;
                     mn[jj] = dmin * (float)mv;
                 }
+                // per token, as floats: lanes j < 8 of a row x_scale, lanes 8 + j the block sum A_j
+                float xm[NMAX];
+                const int sb = 4 * (r * S + wave) + q;
+#pragma unroll
+                for (int n = 0; n < NMAX; n++) {
+                    float a = (float)-(am[k][n] >> 3);  // from -8 * sum
+                    if (own_sums) a = sums[min(n, N - 1) * nb + 8 * min(sb, nsb - 1) + (j & 7)];
+                    xm[n] = meta_s ? __int_as_float(am[k][n]) : a;
+                }
                 float part[NMAX];
 #pragma unroll
                 for (int n = 0; n < NMAX; n++) part[n] = 0.0f;
                 auto pair_step = [&]<int PR>() {
-                    const uint4 q0 = v[1 + 2 * PR], q1 = v[2 + 2 * PR];
+                    constexpr int jl = 2 * PR, jh = 2 * PR + 1;
+                    const uint4 q0 = v[QS + 2 * PR], q1 = v[QS + 1 + 2 * PR];
                     const uint32_t qw[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
                     int lo[8], hi[8];
 #pragma unroll
                     for (int i = 0; i < 8; i++) {
                         lo[i] = (int)(qw[i] & 0x0F0F0F0Fu);
                         hi[i] = (int)((qw[i] >> 4) & 0x0F0F0F0Fu);
+                        if constexpr (Q5) {  // high bits: bit j of byte l belongs to sub-block j's value l
+                            const uint4 h4 = v[1 + (i >> 2)];
+                            const uint32_t h = (i & 3) == 0 ? h4.x : (i & 3) == 1 ? h4.y : (i & 3) == 2 ? h4.z : h4.w;
+                            lo[i] |= (int)(((h >> jl) & 0x01010101u) << 4);
+                            hi[i] |= (int)(((h >> jh) & 0x01010101u) << 4);
+                        }
                     }
-                    constexpr int jl = 2 * PR, jh = 2 * PR + 1;
                     [&]<int... Ns>(std::integer_sequence<int, Ns...>) {
                         (([&] {
                              constexpr int n = Ns;
-                             // W = sum(nib * x) over the pair's low / high 32 elements: x dwords
+                             // W = sum(q * x) over the pair's low / high 32 elements: x dwords
                              // 16*PR + i (lanes i) and 16*PR + 8 + i (lanes 8 + i) of ax[.][n][PR]
-                             const int wl = dot32_bcast<0>(0, ax[k][n][PR], lo[0], lo[1], lo[2], lo[3], lo[4], lo[5],
-                                                           lo[6], lo[7]);
-                             const int wh = dot32_bcast<8>(0, ax[k][n][PR], hi[0], hi[1], hi[2], hi[3], hi[4], hi[5],
-                                                           hi[6], hi[7]);
-                             const float xl = bcast_f<jl>(__int_as_float(am[k][n]));
-                             const float xh = bcast_f<jh>(__int_as_float(am[k][n]));
-                             const int al = bcast_i<8 + jl>(am[k][n]) / -8;  // A_j = sum of x
-                             const int ah = bcast_i<8 + jh>(am[k][n]) / -8;
+                             int wl = 0, wh = 0;
+                             dot64_bcast(wl, wh, ax[k][n][PR], lo, hi);
+                             const float xl = bcast_f<jl>(xm[n]), xh = bcast_f<jh>(xm[n]);
+                             const float al = bcast_f<8 + jl>(xm[n]), ah = bcast_f<8 + jh>(xm[n]);
                              // q8.rs:1372-1375: sum += xs * (sc*W - mn*A), low then high half
-                             part[n] = part[n] + xl * (sc[jl] * (float)wl - mn[jl] * (float)al);
-                             part[n] = part[n] + xh * (sc[jh] * (float)wh - mn[jh] * (float)ah);
+                             part[n] = part[n] + xl * (sc[jl] * (float)wl - mn[jl] * al);
+                             part[n] = part[n] + xh * (sc[jh] * (float)wh - mn[jh] * ah);
                          }()),
                          ...);
                     }(std::make_integer_sequence<int, NMAX>{});
@@ -1556,17 +1614,24 @@ int launch_k(int S, const QMatDev& w, const GemmParams& p, hipStream_t st, hipEv
 // Q4_K on 16-row tiles: 8 waves (one quad of super-blocks each per round) when K has at least
 // 8 quads, else 4 (enough chain threads for 16 tokens); a ring of 2 rounds, 1 at 16 rows
 // (registers).
-template <int NMAX>
+template <int NMAX, bool Q5 = false>
 int launch_k16(const QMatDev& w, const GemmParams& p, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
     constexpr int D = NMAX <= 9 ? 2 : 1;
     auto go = [&]<int S>() {
-        const size_t lds = (size_t)2 * 4 * S * NMAX * 16 * sizeof(float);
+        const size_t lds = q4k_r16_lds_bytes(w, p.N, !p.xs8);
         if (ev0)
-            hipExtLaunchKernelGGL((gemm_q4_k_r16_kernel<NMAX, S, D>), dim3(p.ntiles), dim3(64 * S), lds, st, ev0, ev1, 0,
-                                  p);
+            hipExtLaunchKernelGGL((gemm_q4_k_r16_kernel<NMAX, S, D, Q5>), dim3(p.ntiles), dim3(64 * S), lds, st, ev0, ev1,
+                                  0, p);
         else
-            NC_LAUNCH((gemm_q4_k_r16_kernel<NMAX, S, D>), dim3(p.ntiles), dim3(64 * S), lds, st, p);
+            NC_LAUNCH((gemm_q4_k_r16_kernel<NMAX, S, D, Q5>), dim3(p.ntiles), dim3(64 * S), lds, st, p);
     };
+    if constexpr (Q5) {
+        if (p.epi == EPI_SWIGLU_Q8) return fail(NC_EINVAL, "gemm: 16-row Q5_K tiles have no SwiGLU epilogue");
+        if (w.groups >= 8) go.template operator()<8>();
+        else go.template operator()<4>();
+        NC_HIP(hipGetLastError());
+        return NC_OK;
+    }
     if constexpr (NMAX <= 9) {
         // The interleaved gate,up as four-tile groups with the SwiGLU epilogue on the pair-split
         // kernel (3B, N = 5: 14.9 us against 15.4 for the 64-row kernel in the verify step).
@@ -1583,6 +1648,8 @@ int launch_k16(const QMatDev& w, const GemmParams& p, hipStream_t st, hipEvent_t
         // quad lanes; read at each launch, so a sweep or a test can switch it within a process
         const char* ps_env = getenv("NC_Q4K_PS");
         const int forced = ps_env ? atoi(ps_env) : 0;
+        if (!p.xs8 && (p.epi == EPI_SWIGLU_Q8 || forced))
+            return fail(NC_EINVAL, "gemm: the pair-split kernel reads block sums");
         if (p.epi == EPI_SWIGLU_Q8) {
             if (p.ntiles % 4) return fail(NC_EINVAL, "gemm: interleaved gate,up needs whole 64-row groups");
             ps.template operator()<1, 4>();
@@ -1607,6 +1674,11 @@ int launch_k16(const QMatDev& w, const GemmParams& p, hipStream_t st, hipEvent_t
     }
     NC_HIP(hipGetLastError());
     return NC_OK;
+}
+
+template <int NMAX>
+int launch_k16_q5(const QMatDev& w, const GemmParams& p, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
+    return launch_k16<NMAX, true>(w, p, st, ev0, ev1);
 }
 
 }  // namespace
@@ -1658,6 +1730,9 @@ int launch_gemm(const QMatDev& w, const GemmParams& p0, hipStream_t st, hipEvent
         NC_GEMM_FOR_NMAX(launch_r16, p.N, w, p, st, ev0, ev1)
     }
     if (w.layout == LAYOUT_R16K) {
+        if (w.type == NC_TYPE_Q5_K) {
+            NC_GEMM_FOR_NMAX(launch_k16_q5, p.N, w, p, st, ev0, ev1)
+        }
         NC_GEMM_FOR_NMAX(launch_k16, p.N, w, p, st, ev0, ev1)
     }
     if (w.layout == LAYOUT_Q80) {

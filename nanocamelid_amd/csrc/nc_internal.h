@@ -95,7 +95,7 @@ void repack_q4_0_r16(const uint8_t* src, int64_t rows_src, int64_t cols, uint8_t
 int64_t q40_r16_layout_bytes(int64_t rows, int64_t cols);
 int64_t q40_layout_bytes(int64_t rows, int64_t cols);
 int64_t q4k_layout_bytes(int64_t rows, int64_t cols);
-int64_t q4k_r16_layout_bytes(int64_t rows, int64_t cols);
+int64_t q4k_r16_layout_bytes(int64_t rows, int64_t cols, int nslot = 9);
 // Q4_K on 16-row tiles: per (tile, quad of 4 super-blocks) 9 x [64 lanes x 16 B], lane
 // 16*q + r = super-block 4*quad + q of row r.  half >= 0: rows of an interleaved gate (0) or up
 // (1) matrix, placed in 64-row groups as the Q4_0 repacks do.
@@ -103,7 +103,7 @@ int64_t q80_layout_bytes(int64_t rows, int64_t cols);
 void repack_q8_0(const uint8_t* src, int64_t rows_src, int64_t cols, uint8_t* dst, int64_t groups, int64_t row_off,
                  int half);
 void repack_q4_k_r16(const uint8_t* src, int64_t rows_src, int64_t cols, uint8_t* dst, int64_t groups,
-                     int64_t row_off, int half = -1);
+                     int64_t row_off, int half = -1, int nslot = 9);
 
 // ---------------------------------------------------------------- GEMM launch
 enum Epi : int {
@@ -119,7 +119,8 @@ struct GemmParams {
     int ntiles = 0, units = 0, groups = 0, M = 0, K = 0, N = 0;
     const int8_t* x = nullptr;     // [N][K]
     const float* xs = nullptr;     // [N][K/32]
-    const int32_t* xs8 = nullptr;  // [N][K/32] -8 * (sum of the 32 int8 values of each block)
+    const int32_t* xs8 = nullptr;  // [N][K/32] -8 * (sum of the 32 int8 values of each block), or null
+                                   // (only where the kernel reads no sums or makes its own)
     int epi = EPI_STORE;
     float* out = nullptr;
     int ld_out = 0;
@@ -144,6 +145,12 @@ struct GemmParams {
 // ev0/ev1: optional events stamped at the kernel's own start and end (timing).
 int launch_gemm(const QMatDev& w, const GemmParams& p, hipStream_t stream, hipEvent_t ev0 = nullptr,
                 hipEvent_t ev1 = nullptr);
+// LDS of the 16-row K-quant kernel for n tokens (S = 8 waves from 8 quads on, else 4): two rounds of terms,
+// and the activations' block sums when it makes its own.
+inline size_t q4k_r16_lds_bytes(const QMatDev& w, int n, bool own_sums) {
+    const size_t nmax = n <= 9 ? n : 16, S = w.groups >= 8 ? 8 : 4;
+    return 2 * 4 * S * nmax * 16 * sizeof(float) + (own_sums ? (size_t)n * w.units * 8 * sizeof(float) : 0);
+}
 int launch_blockdots(const QMatDev& w, const int8_t* x, int32_t* dots, int N, hipStream_t stream);
 // Q6_K matmul of any number of tokens (plain outputs or the head's logits + argmax partials)
 int launch_gemm_q6k(const QMatDev& w, const GemmParams& p, hipStream_t stream);

@@ -160,8 +160,8 @@ int64_t q40_layout_bytes(int64_t rows, int64_t cols) {
     return tiles * groups * kQ40ChunkBytes;
 }
 int64_t q4k_layout_bytes(int64_t rows, int64_t cols) { return (rows + 63) / 64 * (cols / 256) * kQ4KChunkBytes; }
-int64_t q4k_r16_layout_bytes(int64_t rows, int64_t cols) {
-    return (rows + 15) / 16 * ((cols / 256 + 3) / 4) * kQ4KChunkBytes;
+int64_t q4k_r16_layout_bytes(int64_t rows, int64_t cols, int nslot) {
+    return (rows + 15) / 16 * ((cols / 256 + 3) / 4) * 1024 * nslot;
 }
 
 static inline int64_t dst_row(int64_t r, int64_t row_off, int half) {
@@ -254,15 +254,15 @@ void repack_q4_k(const uint8_t* src, int64_t rows_src, int64_t cols, uint8_t* ds
 }
 
 void repack_q4_k_r16(const uint8_t* src, int64_t rows_src, int64_t cols, uint8_t* dst, int64_t groups,
-                     int64_t row_off, int half) {
+                     int64_t row_off, int half, int nslot) {
     const int64_t nsb = cols / 256;
     parallel_for(rows_src, 0, [&](int64_t lo, int64_t hi) {
         for (int64_t r = lo; r < hi; r++) {
             const int64_t R = dst_row(r, row_off, half), t = R / 16, rr = R % 16;
             for (int64_t s = 0; s < nsb; s++) {
-                const uint8_t* blk = src + (r * nsb + s) * 144;
-                uint8_t* chunk = dst + (t * groups + s / 4) * kQ4KChunkBytes + (16 * (s % 4) + rr) * 16;
-                for (int i = 0; i < 9; i++) std::memcpy(chunk + i * 1024, blk + i * 16, 16);
+                const uint8_t* blk = src + (r * nsb + s) * 16 * nslot;
+                uint8_t* chunk = dst + (t * groups + s / 4) * 1024 * nslot + (16 * (s % 4) + rr) * 16;
+                for (int i = 0; i < nslot; i++) std::memcpy(chunk + i * 1024, blk + i * 16, 16);
             }
         }
     });
@@ -345,6 +345,9 @@ static int upload_matrix(int type, int64_t rows, int64_t cols, const std::vector
     }();
     out.layout = type == NC_TYPE_Q4_0 && (rows + 63) / 64 < r16_max ? LAYOUT_R16 : LAYOUT_R64;
     if (type == NC_TYPE_Q4_K && (rows + 63) / 64 < (single ? 256 : 1024)) out.layout = LAYOUT_R16K;
+    // Q5_K: the same for single matrices; an interleaved gate/up pair keeps the 64-row SwiGLU epilogue
+    if (type == NC_TYPE_Q5_K && single && (rows + 63) / 64 < 256) out.layout = LAYOUT_R16K;
+    const int nslot = type == NC_TYPE_Q5_K ? 11 : 9;
     out.units = type == NC_TYPE_Q4_0 ? cols / 32 : cols / 256;
     if (out.layout == LAYOUT_R16) {
         out.tiles = (rows + 15) / 16;
@@ -353,7 +356,7 @@ static int upload_matrix(int type, int64_t rows, int64_t cols, const std::vector
     } else if (out.layout == LAYOUT_R16K) {
         out.tiles = (rows + 15) / 16;
         out.groups = (out.units + 3) / 4;
-        out.dev_bytes = q4k_r16_layout_bytes(rows, cols);
+        out.dev_bytes = q4k_r16_layout_bytes(rows, cols, nslot);
     } else {
         out.tiles = (rows + 63) / 64;
         out.groups = type == NC_TYPE_Q4_0 ? (out.units + 7) / 8 : 0;
@@ -367,9 +370,9 @@ static int upload_matrix(int type, int64_t rows, int64_t cols, const std::vector
     std::vector<uint8_t> host(out.dev_bytes, 0);
     for (const auto& p : parts) {
         if (out.layout == LAYOUT_R16) repack_q4_0_r16(p.src, p.rows, cols, host.data(), out.groups, p.row_off, p.half);
-        else if (out.layout == LAYOUT_R16K) repack_q4_k_r16(p.src, p.rows, cols, host.data(), out.groups, p.row_off, p.half);
+        else if (out.layout == LAYOUT_R16K) repack_q4_k_r16(p.src, p.rows, cols, host.data(), out.groups, p.row_off, p.half, nslot);
         else if (type == NC_TYPE_Q4_0) repack_q4_0(p.src, p.rows, cols, host.data(), out.groups, p.row_off, p.half);
-        else repack_q4_k(p.src, p.rows, cols, host.data(), p.row_off, p.half, type == NC_TYPE_Q5_K ? 11 : 9);
+        else repack_q4_k(p.src, p.rows, cols, host.data(), p.row_off, p.half, nslot);
     }
     NC_HIP(hipMalloc((void**)&out.dev, out.dev_bytes));
     NC_HIP(hipMemcpy(out.dev, host.data(), out.dev_bytes, hipMemcpyHostToDevice));
@@ -1171,7 +1174,10 @@ static int slice_tokens(const QMatDev& q, int n) { return q.type == NC_TYPE_Q6_K
 
 // Whether the verify kernels of a matrix read the activations' block sums: for the mins of Q4_K and
 // Q5_K, and for the offset of the unsigned Q4_0 nibbles on the int8 MFMA path.
-static bool needs_block_sums(const nc_ctx* ctx, const QMatDev& q) {
+// A plain K-quant matmul of n tokens on 16-row tiles sums for itself where the sums fit in 64 KB of LDS
+// beside its terms.
+static bool needs_block_sums(const nc_ctx* ctx, const QMatDev& q, int n) {
+    if (q.layout == LAYOUT_R16K && !getenv("NC_Q4K_PS") && q4k_r16_lds_bytes(q, n, true) <= 65536) return false;
     return q.type == NC_TYPE_Q4_K || q.type == NC_TYPE_Q5_K ||
            (q.type == NC_TYPE_Q4_0 && ctx->gemm_kernel == NC_GEMM_KERNEL_MFMA);
 }
@@ -1559,15 +1565,15 @@ int nc_matmul_quantized_batch(nc_ctx* ctx, const nc_qmat* w, const int8_t* x_i8,
     for (int i = 0; i < batch_size; i += slice) {
         const int nb = std::min(slice, batch_size - i);
         int rc = NC_OK;
-        if (needs_block_sums(ctx, w->m) &&
-            ((rc = ensure_xsum(ctx, (size_t)nb * (cols / 32))) ||
-             (rc = launch_block_sums(x_i8 + (size_t)i * cols, nb, (int)cols, ctx->xsum, st))))
+        const bool sums = needs_block_sums(ctx, w->m, nb);
+        if (sums && ((rc = ensure_xsum(ctx, (size_t)nb * (cols / 32))) ||
+                     (rc = launch_block_sums(x_i8 + (size_t)i * cols, nb, (int)cols, ctx->xsum, st))))
             return rc;
         GemmParams p;
         p.kernel = ctx->gemm_kernel;
         p.x = x_i8 + (size_t)i * cols;
         p.xs = x_scales + (size_t)i * (cols / 32);
-        p.xs8 = ctx->xsum;
+        p.xs8 = sums ? ctx->xsum : nullptr;
         p.N = nb;
         p.epi = EPI_STORE;
         p.out = out + (size_t)i * rows;

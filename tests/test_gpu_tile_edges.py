@@ -7,7 +7,7 @@ import pytest
 import nanocamelid_amd as nc
 from oracle import oracle as O
 from tests import gguf_writer as GW
-from tests.gpu_util import q8_activations, random_q4_0, random_q8_0
+from tests.gpu_util import q8_activations, random_q4_0, random_q4_k, random_q5_k, random_q8_0
 
 pytestmark = pytest.mark.gpu
 
@@ -57,3 +57,16 @@ def test_prompt_block_matmul_wave_tiles(ctx, qtype, M, K, batches):
         check(ctx, nc.NC_TYPE_Q4_0, random_q4_0(M, K, seed=M), O.matmul_q4_0, M, K, batches, 5)
     else:
         check(ctx, nc.NC_TYPE_Q8_0, random_q8_0(M, K, seed=M), O.matmul_q8_0, M, K, batches, 6)
+
+
+# K-quant matrices on 16-row tiles (and from 16384 rows on 64-row ones): one super-block, cut quads, both wave
+# counts (4, and 8 from 29 super-blocks), operator calls whose kernel sums the activations itself and, at 16 tokens
+# of a long row, ones that take a separate launch
+@pytest.mark.parametrize("qtype", ["q4_k", "q5_k"])
+@pytest.mark.parametrize("M,K", [(1, 256), (17, 1280), (100, 768), (40, 7680), (33, 8192), (16400, 256)])
+def test_k_quant_tile_edges(ctx, qtype, M, K):
+    batches = [1, 2, 3, 4, 5, 6, 7, 8, 9, 16, 18]
+    if qtype == "q4_k":
+        check(ctx, nc.NC_TYPE_Q4_K, random_q4_k(M, K, seed=M + K), O.matmul_q4_k, M, K, batches, 7)
+    else:
+        check(ctx, nc.NC_TYPE_Q5_K, random_q5_k(M, K, seed=M + K), O.matmul_q5_k, M, K, batches, 8)
