@@ -196,21 +196,16 @@ int launch_attention_tiles(const AttnParams& a, hipStream_t stream);
 int64_t attention_variant(const AttnParams& a);
 
 // ---------------------------------------------------------------- prompt (prefill) path
-// Q4_0 / Q8_0 batch matmul for any number of tokens on the matrix cores: out[n * ld_out + row] over
-// xh / xsm, the activations as f16 in operand order with their scales (launch_prompt_repack_f16; xh:
-// 16 * ceil(N/16) * prompt_cols(K) * 2 bytes, xsm: 16 * ceil(N/16) * prompt_cols(K) / 32 floats).
+// Batch matmuls for any number of tokens on the matrix cores: out[n * ld_out + row] over the activations
+// as f16 in operand order (launch_prompt_repack; xh: 16 * ceil(N/16) * prompt_cols(K) * 2 bytes, xsm and, for
+// the K-quants only, xam: 16 * ceil(N/16) * prompt_cols(K) / 32 floats).
 int launch_gemm_prompt(const QMatDev& w, float* out, int ld_out, int N, hipStream_t stream, const void* xh,
-                       const float* xsm);
-int launch_prompt_repack_f16(const int8_t* x, const float* xs, int N, int K, void* xh, float* xsm, hipStream_t stream);
-inline int64_t prompt_cols(int64_t cols) { return (cols + 127) / 128 * 128; }  // whole quads of blocks
-// The int8 form for the K-quant prompt matmuls (xm: 16 * ceil(N/16) * K bytes, xsm as above).
-int launch_prompt_repack(const int8_t* x, const float* xs, int N, int K, void* xm, float* xsm, hipStream_t stream,
+                       const float* xsm);  // Q4_0 (R16, R64), Q8_0
+int launch_gemm_prompt_k(const QMatDev& w, float* out, int ld_out, int N, hipStream_t stream, const void* xh,
+                         const float* xsm, const float* xam);  // Q4_K, Q5_K (R16K, R64)
+int launch_prompt_repack(const int8_t* x, const float* xs, int N, int K, void* xh, float* xsm, hipStream_t stream,
                          float* xam = nullptr);
-// (xam, as xsm: the float sums of each 32-value block's int8 values, Q4_K's A_j)
-// Q4_K batch matmul for any number of tokens on int8 MFMA (R16K and R64 layouts) over
-// activations repacked with their block sums
-int launch_gemm_prompt_q4k(const QMatDev& w, float* out, int ld_out, int N, hipStream_t stream, const void* xm,
-                           const float* xsm, const float* xam);
+inline int64_t prompt_cols(int64_t cols) { return (cols + 127) / 128 * 128; }  // whole quads of blocks
 // The verify GEMMs' epilogues as separate kernels over a prompt matmul's f32 output y.
 int launch_prompt_qkv_rope(const float* y, int N, int start, int aw, int kw, int hd, int rope_half,
                            const float* rope_tab, float* q_out, float* kcache, float* vcache, int max_ctx,

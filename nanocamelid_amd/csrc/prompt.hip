@@ -23,8 +23,6 @@
 
 namespace nc {
 
-typedef int p_v4i __attribute__((ext_vector_type(4)));
-
 typedef float p_v4f __attribute__((ext_vector_type(4)));
 typedef float p_v16f __attribute__((ext_vector_type(16)));
 typedef _Float16 p_h2 __attribute__((ext_vector_type(2)));
@@ -231,34 +229,29 @@ int launch_gemm_prompt(const QMatDev& w, float* out, int ld_out, int N, hipStrea
     return NC_OK;
 }
 
-// ---------------------------------------------------------------- Q4_K prompt matmul
+// ---------------------------------------------------------------- Q4_K and Q5_K prompt matmul
 // matmul_q4_k_batch (inference.rs:2006-2132, x86 path :2083-2130) for many tokens: per row and
 // token, super-blocks in order, each the f32 sum from 0.0 over its eight 32-value sub-blocks j of
 //   xs_j * (sc_j * (float)W_j - mn_j * (float)A_j),   sc_j = d * s_j, mn_j = dmin * m_j
-// (q8.rs:1339-1376 dot_q8_scaled_preloaded, scales by q4_k_scale_min q8.rs:2009-2018), with
-// W_j = sum nib * x (unsigned nibbles) and A_j = sum x of the sub-block; that super-block sum is
-// added to the row's sum.  W_j comes from v_mfma_i32_16x16x32_i8 on the raw nibbles (K = 32 = one
-// sub-block): sub-block 2p is the low nibbles of bytes 32p..32p+31, 2p + 1 the high nibbles, so
-// lane (g, r)'s dwords at bytes 32p + 4g and 32p + 16 + 4g give both A operands.  A_j as a float
-// comes with the repacked activations (xam).  Lane (g, r) decodes its row's scales and mins of
-// sub-blocks 2g and 2g + 1 into a per-wave LDS table from which the D lanes (g, c) read rows
-// 4g..4g+3.  A wave covers 32 rows x 32 tokens, a workgroup 64 x 64; weights stay in the verify
+// (q8.rs:1339-1376 dot_q8_scaled_preloaded, scales by q4_k_scale_min q8.rs:2009-2018; Q5_K likewise,
+// q8.rs:1551-1594), with W_j = sum q * x (unsigned values) and A_j = sum x of the sub-block; that
+// super-block sum is added to the row's sum.  W_j arrives as an exact f32 from f16 MFMA, mn_j * A_j from a
+// one-term f32 MFMA, as in the kernel above; four VALU operations per output and sub-block remain.
+// Sub-block 2p is the low nibbles of bytes 32p..32p+31, 2p + 1 the high nibbles.  Lane (g, r)
+// decodes its row's scales and mins of sub-blocks 2g and 2g + 1 into a per-wave LDS table.  Same tiles,
+// stages (half a super-block) and activation staging as gemm_b32_prompt_kernel; weights stay in the verify
 // layouts (R16K: 16-row tiles, chunks of 4 super-blocks; R64: 64-row tiles, one super-block per
-// chunk), each chunk 9 slots of [64 lanes x 16 B], slot 0 the header (d, dmin, 12 scale bytes).
-// Row tiles per wave: 2 (32 x 32 wave tiles) when that gives every SIMD at least two waves
-// (2048 waves on 256 CUs), else 1 (16 x 32: twice the waves for the same work).
-static int prompt_row_tiles(int64_t rows, int N) {
-    return ((rows + 31) / 32) * ((N + 31) / 32) >= 2048 ? 2 : 1;
-}
-
+// chunk), each chunk 9 (Q5_K 11) slots of [64 lanes x 16 B]: header (d, dmin, 12 scale bytes), Q5_K's two
+// slots of high-bit bytes, nibbles.
+// Q4_K, 250 / 256 tokens, against int8 MFMA with conversions and 32 x 32 wave tiles: 8192 x 3072 58 -> 56 us,
+// 3072 x 8192 92 -> 73, 16384 x 3072 108 -> 97.  Q5_K 14336 x 4096 took 16-token slices (16 x 62 us), now 137.
 struct PromptGemmK {
     const uint8_t* w = nullptr;
-    int64_t w_bytes = 0;
     int nsb = 0, groups = 0, tiles16 = 0;  // super-blocks per row; R16K chunks per tile; 16-row tiles stored
     int M = 0, N = 0, ld_out = 0;
-    const uint2* xm = nullptr;    // activations in MFMA operand order (prompt_repack_kernel)
-    const float4* xsm = nullptr;  // x_scale of each sub-block, 4 per float4
-    const float4* xam = nullptr;  // (float) sum of each sub-block's int8 values, 4 per float4
+    const uint8_t* xh = nullptr;  // as PromptGemm
+    const float* xsm = nullptr;   // [N/16][nq][16 tokens] float4: a quad's x_scales
+    const float* xam = nullptr;   // [N/16][nq][64 lanes]: (float) sum of block lane / 16's values, token lane % 16
     float* out = nullptr;         // out[n * ld_out + row]
 };
 
@@ -277,256 +270,216 @@ __device__ __forceinline__ void q4k_scale_min_dev(int j, uint32_t s0, uint32_t s
     }
 }
 
-template <int LAYOUT, int RT>
-__global__ __launch_bounds__(256) void gemm_q4_k_prompt_kernel(PromptGemmK p) {
-    __shared__ __align__(16) float tab[4][2][8][2][16];  // per wave: [tile][sub-block][sc, mn][row]
+template <int LAYOUT, bool Q5, int KT, int SD>
+__global__ __launch_bounds__(256, KT == 4 ? 3 : 4) void gemm_k_prompt_kernel(PromptGemmK p, int tgroups) {
+    constexpr int NSLOT = Q5 ? 11 : 9, QS = Q5 ? 3 : 1, CHUNK = 1024 * NSLOT, WD = 2;
+    __shared__ __align__(16) uint4 bs[2][4][KT][64];
+    __shared__ __align__(16) float xss[2][KT][64];
+    __shared__ __align__(16) float tab[4][8][2][16];  // per wave: [sub-block][sc, mn][row]
     const int lane = threadIdx.x & 63, wv = wave_id_uniform();
     const int g = lane >> 4, r = lane & 15;
-    // RT = 2: a wave covers 32 rows x 32 tokens, a workgroup 64 x 64; RT = 1 (matrices whose
-    // 32 x 32 tiles would leave a SIMD one wave): 16 rows x 32 tokens, a workgroup 64 x 32
-    const int row0 = RT == 2 ? blockIdx.x * 64 + (wv & 1) * 32 : blockIdx.x * 64 + wv * 16;
-    const int tok0 = RT == 2 ? blockIdx.y * 64 + (wv >> 1) * 32 : blockIdx.y * 32;
-    if (row0 >= p.M || tok0 >= p.N) return;  // wave-uniform; the kernel has no barriers
-    const int n16 = (p.N + 15) / 16, nq = 2 * p.nsb;  // 16-token tiles, quads of sub-blocks
-    int tt[2];
-#pragma unroll
-    for (int k = 0; k < 2; k++) tt[k] = min(tok0 / 16 + k, n16 - 1);
-    const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc((void*)p.w, 0, (int)p.w_bytes, 0x00020000);
-    const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc((void*)p.xm, 0, n16 * p.nsb * 256 * 16, 0x00020000);
+    const int t16 = blockIdx.x / tgroups * 4 + wv, tt = blockIdx.x % tgroups * KT;  // row tile, first token tile
+    const int nq = 2 * p.nsb, n16 = (p.N + 15) / 16;
+    const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc((void*)p.xh, 0, n16 * nq * 4096, 0x00020000);
     const __amdgpu_buffer_rsrc_t sres = __builtin_amdgcn_make_buffer_rsrc((void*)p.xsm, 0, n16 * nq * 256, 0x00020000);
     const __amdgpu_buffer_rsrc_t ares = __builtin_amdgcn_make_buffer_rsrc((void*)p.xam, 0, n16 * nq * 256, 0x00020000);
-    // chunk offset of (16-row tile i, super-block sb) and this lane's part of a slot
-    auto chunk = [&](int i, int sb) -> int {
-        if constexpr (LAYOUT == LAYOUT_R16K) {
-            const int t16 = min(row0 / 16 + i, p.tiles16 - 1);  // storage is padded to 16 rows
-            return (t16 * p.groups + sb / 4) * kQ4KChunkBytes + 256 * (sb & 3);
-        } else {
-            return ((row0 / 64) * p.nsb + sb) * kQ4KChunkBytes + ((row0 & 63) + 16 * i) * 16;
-        }
-    };
-    // one stage = half a super-block (sub-blocks 4h..4h+3): per tile the nibble dwords of two
-    // pairs and the header; per token tile four B operands, the x_scales and the sums
-    uint32_t hd[2][RT][4], nb0[2][RT][2], nb1[2][RT][2], xa[2][2][4], xb[2][2][4];
-    float4 xsv[2][2], xav[2][2];
-#define NC_PK_LOAD(ST, SLOT)                                                                                    \
-    do {                                                                                                        \
-        const int st_ = min((ST), nq - 1), sb_ = st_ >> 1, h_ = st_ & 1;                                        \
-        _Pragma("unroll") for (int i = 0; i < RT; i++) {                                                         \
-            const int c_ = chunk(i, sb_);                                                                       \
-            const uint4 hv_ = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(wres, r * 16, c_, 0)); \
-            hd[SLOT][i][0] = hv_.x; hd[SLOT][i][1] = hv_.y; hd[SLOT][i][2] = hv_.z; hd[SLOT][i][3] = hv_.w;     \
-            _Pragma("unroll") for (int pp = 0; pp < 2; pp++) {                                                  \
-                const int pr_ = 2 * h_ + pp;                                                                    \
-                nb0[SLOT][i][pp] = __builtin_amdgcn_raw_buffer_load_b32(wres, r * 16 + 4 * g, c_ + (2 * pr_ + 1) * 1024, 0); \
-                nb1[SLOT][i][pp] = __builtin_amdgcn_raw_buffer_load_b32(wres, r * 16 + 4 * g, c_ + (2 * pr_ + 2) * 1024, 0); \
-            }                                                                                                   \
-        }                                                                                                       \
-        _Pragma("unroll") for (int k = 0; k < 2; k++) {                                                         \
-            _Pragma("unroll") for (int j = 0; j < 4; j++) {                                                     \
-                const uint2 v_ = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(                \
-                    xres, lane * 8, (tt[k] * 8 * p.nsb + 4 * st_ + j) * 512, 0));                               \
-                xa[SLOT][k][j] = v_.x;                                                                          \
-                xb[SLOT][k][j] = v_.y;                                                                          \
-            }                                                                                                   \
-            xsv[SLOT][k] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(sres, r * 16, (tt[k] * nq + st_) * 256, 0)); \
-            xav[SLOT][k] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(ares, r * 16, (tt[k] * nq + st_) * 256, 0)); \
-        }                                                                                                       \
-    } while (0)
-    float acc[RT][2][4], part[RT][2][4];
+    // the row tile's storage (clamped into the padded rows)
+    const int ts = min(t16, p.tiles16 - 1);
+    const int tile_bytes = (LAYOUT == LAYOUT_R16K ? p.groups : p.nsb) * CHUNK;
+    const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(p.w + (size_t)(LAYOUT == LAYOUT_R16K ? ts : ts >> 2) * tile_bytes), 0, tile_bytes, 0x00020000);
+    const int hvo = LAYOUT == LAYOUT_R16K ? r * 16 : (16 * (ts & 3) + r) * 16, nvo = hvo + 4 * g;
+    const int uk = wv % KT, uj = wv / KT;  // this wave's share of a stage's units
+    const int ubase = (tt + uk) * nq * 4096 + uj * 1024;
+    uint32_t wd[WD][2][2], hdn[6];
+    float xar[WD][KT], xst[SD];
+    uint4 st[SD][KT];
+#define NC_PK_UNITS(S, SLOT)                                                                                       \
+    {                                                                                                              \
+        _Pragma("unroll") for (int u = 0; u < KT; u++) st[SLOT][u] = __builtin_bit_cast(                           \
+            uint4, __builtin_amdgcn_raw_buffer_load_b128(xres, lane * 16 + u * (4 / KT) * 1024, ubase + (S) * 4096, 0)); \
+        xst[SLOT] = __builtin_bit_cast(                                                                            \
+            float, __builtin_amdgcn_raw_buffer_load_b32(sres, lane * 4, ((tt + uk) * nq + (S)) * 256, 0));         \
+    }
+#define NC_PK_WEIGHTS(S, SLOT, HEAD)                                                                               \
+    {                                                                                                              \
+        const int sb_ = (S) >> 1;                                                                                  \
+        const int co_ = LAYOUT == LAYOUT_R16K ? (sb_ >> 2) * CHUNK + 256 * (sb_ & 3) : sb_ * CHUNK;                \
+        _Pragma("unroll") for (int pp = 0; pp < 2; pp++) _Pragma("unroll") for (int x = 0; x < 2; x++)             \
+            wd[SLOT][pp][x] = __builtin_amdgcn_raw_buffer_load_b32(                                                \
+                wres, nvo + 1024 * (2 * pp + x), co_ + (QS + 4 * ((S) & 1)) * 1024, 0);                            \
+        if (HEAD) {                                                                                                \
+            const uint4 h_ = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(wres, hvo, co_, 0));  \
+            hdn[0] = h_.x, hdn[1] = h_.y, hdn[2] = h_.z, hdn[3] = h_.w;                                            \
+            if (Q5) {                                                                                              \
+                hdn[4] = __builtin_amdgcn_raw_buffer_load_b32(wres, nvo + 1024, co_, 0);                           \
+                hdn[5] = __builtin_amdgcn_raw_buffer_load_b32(wres, nvo + 2048, co_, 0);                           \
+            }                                                                                                      \
+        }                                                                                                          \
+        _Pragma("unroll") for (int k = 0; k < KT; k++) xar[SLOT][k] = __builtin_bit_cast(                          \
+            float, __builtin_amdgcn_raw_buffer_load_b32(ares, lane * 4, ((tt + k) * nq + (S)) * 256, 0));          \
+    }
+    uint32_t one = 0x64006400u;  // two f16 1024
+    asm("" : "+v"(one));
+    p_v4f acc[KT], part[KT];
 #pragma unroll
-    for (int i = 0; i < RT; i++)
+    for (int k = 0; k < KT; k++) acc[k] = p_v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    const p_v16f zero16 = {};
+    const p_v4f zero4 = {};
 #pragma unroll
-        for (int k = 0; k < 2; k++)
+    for (int b = 0; b < SD; b++) NC_PK_UNITS(b, b)
+    NC_PK_WEIGHTS(0, 0, true)
 #pragma unroll
-            for (int v = 0; v < 4; v++) acc[i][k][v] = 0.0f;
-    const p_v4i zero = {0, 0, 0, 0};
-    float(*wt)[8][2][16] = tab[wv];
-    NC_PK_LOAD(0, 0);
-    for (int s0 = 0; s0 < nq; s0 += 2) {
+    for (int u = 0; u < KT; u++) bs[0][u * (4 / KT) + uj][uk][lane] = st[0][u];
+    xss[0][uk][lane] = xst[0];
+    __syncthreads();
+    uint32_t h0 = 0, h1 = 0;
+    for (int s0 = 0; s0 < nq; s0 += 2) {  // nq is even: a super-block per turn
 #pragma unroll
-        for (int s = 0; s < 2; s++) {
-            const int st = s0 + s;  // s == st & 1 (nq is even)
-            NC_PK_LOAD(st + 1, (s + 1) & 1);
-            if (s == 0) {
+        for (int b = 0; b < 2; b++) {
+            const int s = s0 + b;
+            if (b == 0) {
                 // this lane's row r, sub-blocks 2g and 2g + 1: scales and mins into the table
+                const float d = f16_to_f32((uint16_t)(hdn[0] & 0xffff)), dmin = f16_to_f32((uint16_t)(hdn[0] >> 16));
 #pragma unroll
-                for (int i = 0; i < RT; i++) {
-                    const float d = f16_to_f32((uint16_t)(hd[0][i][0] & 0xffff));
-                    const float dmin = f16_to_f32((uint16_t)(hd[0][i][0] >> 16));
-#pragma unroll
-                    for (int e = 0; e < 2; e++) {
-                        uint32_t sv, mv;
-                        q4k_scale_min_dev(2 * g + e, hd[0][i][1], hd[0][i][2], hd[0][i][3], &sv, &mv);
-                        wt[i][2 * g + e][0][r] = d * (float)sv;
-                        wt[i][2 * g + e][1][r] = dmin * (float)mv;
-                    }
+                for (int e = 0; e < 2; e++) {
+                    uint32_t sv, mv;
+                    q4k_scale_min_dev(2 * g + e, hdn[1], hdn[2], hdn[3], &sv, &mv);
+                    tab[wv][2 * g + e][0][r] = d * (float)sv;
+                    tab[wv][2 * g + e][1][r] = dmin * (float)mv;
                 }
+                if (Q5) h0 = hdn[4], h1 = hdn[5];
                 __builtin_amdgcn_wave_barrier();
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                 __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
-                for (int i = 0; i < RT; i++)
-#pragma unroll
-                    for (int k = 0; k < 2; k++)
-#pragma unroll
-                        for (int v = 0; v < 4; v++) part[i][k][v] = 0.0f;
+                for (int k = 0; k < KT; k++) part[k] = p_v4f{0.0f, 0.0f, 0.0f, 0.0f};
             }
+            NC_PK_UNITS(s + SD, b % SD)  // that slot's stage is in LDS
+            NC_PK_WEIGHTS(s + 1, (b + 1) & 1, b == 1)
+            p_h8 a[4];
 #pragma unroll
-            for (int jj = 0; jj < 4; jj++) {
-                const int j = 4 * s + jj, pp = jj >> 1, hi = jj & 1;  // sub-block j of the super-block
-                long bx[2];
-                float xsj[2], xaj[2];
+            for (int j = 0; j < 4; j++) {
+                const uint32_t w0 = wd[b][j >> 1][0], w1 = wd[b][j >> 1][1];
+                const int sh = j & 1 ? 4 : 0;
+                uint32_t u[4] = {w0 >> sh, w1 >> sh, w0 >> (8 + sh), w1 >> (8 + sh)};
 #pragma unroll
-                for (int k = 0; k < 2; k++) {
-                    bx[k] = (long)((uint64_t)xa[s][k][jj] | ((uint64_t)xb[s][k][jj] << 32));
-                    const float4 xs4 = xsv[s][k], xa4 = xav[s][k];
-                    xsj[k] = jj == 0 ? xs4.x : jj == 1 ? xs4.y : jj == 2 ? xs4.z : xs4.w;
-                    xaj[k] = jj == 0 ? xa4.x : jj == 1 ? xa4.y : jj == 2 ? xa4.z : xa4.w;
-                }
-#pragma unroll
-                for (int i = 0; i < RT; i++) {
-                    const uint32_t w0 = hi ? (nb0[s][i][pp] >> 4) : nb0[s][i][pp];
-                    const uint32_t w1 = hi ? (nb1[s][i][pp] >> 4) : nb1[s][i][pp];
-                    const long a = (long)((uint64_t)(w0 & 0x0F0F0F0Fu) | ((uint64_t)(w1 & 0x0F0F0F0Fu) << 32));
-                    const float4 sc4 = *(const float4*)&wt[i][j][0][4 * g];
-                    const float4 mn4 = *(const float4*)&wt[i][j][1][4 * g];
-                    const float scv[4] = {sc4.x, sc4.y, sc4.z, sc4.w}, mnv[4] = {mn4.x, mn4.y, mn4.z, mn4.w};
-#pragma unroll
-                    for (int k = 0; k < 2; k++) {
-                        const p_v4i dw = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, bx[k], zero, 0, 0, 0);
-#pragma unroll
-                        for (int v = 0; v < 4; v++) {
-                            const float av = scv[v] * (float)dw[v];
-                            const float bv = mnv[v] * xaj[k];
-                            part[i][k][v] = part[i][k][v] + xsj[k] * (av - bv);
-                        }
+                for (int i = 0; i < 4; i++) {
+                    u[i] = (u[i] & 0x000F000Fu) | one;
+                    if constexpr (Q5) {  // bit 4 b + j of a byte of h0 / h1 is the value's bit 4
+                        const uint32_t h = (i & 1 ? h1 : h0) >> (8 * (i >> 1));
+                        const int bit = 4 * b + j;
+                        u[i] |= (bit < 4 ? h << (4 - bit) : h >> (bit - 4)) & 0x00100010u;
                     }
+                    const p_h2 v = __builtin_bit_cast(p_h2, u[i]);
+                    u[i] = __builtin_bit_cast(uint32_t, v - (p_h2){(_Float16)1024.0f, (_Float16)1024.0f});
                 }
+                a[j] = __builtin_bit_cast(p_h8, make_uint4(u[0], u[1], u[2], u[3]));
             }
-            if (s == 1) {
+            const float mnv = tab[wv][4 * b + g][1][r];  // A operand of the outer product: (sub-block, row)
+            p_v4f sc[4];
 #pragma unroll
-                for (int i = 0; i < RT; i++)
+            for (int j = 0; j < 4; j++) sc[j] = *(const p_v4f*)&tab[wv][4 * b + j][0][4 * g];
 #pragma unroll
-                    for (int k = 0; k < 2; k++)
+            for (int k = 0; k < KT; k++) {
+                p_v4f d[4];
+                const p_v16f bo = __builtin_amdgcn_mfma_f32_16x16x1f32(mnv, xar[b][k], zero16, 0, 0, 0);
+                const p_v4f xs4 = *(const p_v4f*)&xss[b][k][4 * r];
 #pragma unroll
-                        for (int v = 0; v < 4; v++) acc[i][k][v] = acc[i][k][v] + part[i][k][v];
-                // every lane has read this super-block's table before the next one is written
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                for (int j = 0; j < 4; j++)
+                    d[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[j], __builtin_bit_cast(p_h8, bs[b][j][k][lane]), zero4,
+                                                                  0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+#pragma unroll
+                    for (int v = 0; v < 4; v++)
+                        part[k][v] = part[k][v] + xs4[j] * (sc[j][v] * d[j][v] - bo[4 * j + v]);
+                // the next token tile's products start after these sums (all would be live at once otherwise)
+                if (k + 1 < KT) asm volatile("" : "+v"(part[k]), "+v"(xar[b][k + 1]));
             }
+            if (b == 1) {
+#pragma unroll
+                for (int k = 0; k < KT; k++)
+#pragma unroll
+                    for (int v = 0; v < 4; v++) acc[k][v] = acc[k][v] + part[k][v];
+            }
+            // the other buffer was last read a stage ago, before the barrier that ended that stage; the
+            // wave's own table is rewritten after it too
+#pragma unroll
+            for (int u = 0; u < KT; u++) bs[(b + 1) & 1][u * (4 / KT) + uj][uk][lane] = st[(b + 1) % SD][u];
+            xss[(b + 1) & 1][uk][lane] = xst[(b + 1) % SD];
+            __syncthreads();
         }
     }
-#undef NC_PK_LOAD
+#undef NC_PK_UNITS
+#undef NC_PK_WEIGHTS
 #pragma unroll
-    for (int k = 0; k < 2; k++) {
-        const int n = tok0 + 16 * k + r;
+    for (int k = 0; k < KT; k++) {
+        const int n = (tt + k) * 16 + r, row = t16 * 16 + 4 * g;
         if (n >= p.N) continue;
+        float* o = p.out + (size_t)n * p.ld_out + row;
+        if (row + 3 < p.M && (p.ld_out & 3) == 0) {
+            *(float4*)o = make_float4(acc[k][0], acc[k][1], acc[k][2], acc[k][3]);
+        } else {
 #pragma unroll
-        for (int i = 0; i < RT; i++) {
-            const int row = row0 + 16 * i + 4 * g;
-            float* o = p.out + (size_t)n * p.ld_out + row;
-            if (row + 3 < p.M && (p.ld_out & 3) == 0) {
-                *(float4*)o = make_float4(acc[i][k][0], acc[i][k][1], acc[i][k][2], acc[i][k][3]);
-            } else {
-#pragma unroll
-                for (int v = 0; v < 4; v++)
-                    if (row + v < p.M) o[v] = acc[i][k][v];
-            }
+            for (int v = 0; v < 4; v++)
+                if (row + v < p.M) o[v] = acc[k][v];
         }
     }
 }
 
-int launch_gemm_prompt_q4k(const QMatDev& w, float* out, int ld_out, int N, hipStream_t st, const void* xm,
-                           const float* xsm, const float* xam) {
-    if (w.type != NC_TYPE_Q4_K || (w.layout != LAYOUT_R16K && w.layout != LAYOUT_R64))
-        return fail(NC_EINVAL, "Q4_K prompt matmul: Q4_K matrices only");
-    if (!xm || !xsm || !xam) return fail(NC_EINVAL, "Q4_K prompt matmul: repacked activations required");
-    if (N < 1 || (int64_t)N * w.cols >= (int64_t)1 << 31 || w.dev_bytes >= (int64_t)1 << 31)
-        return fail(NC_ERANGE, "Q4_K prompt matmul: operands exceed 2 GiB");
+template <int LAYOUT, bool Q5>
+static void launch_k_prompt(const PromptGemmK& p, hipStream_t st) {
+    const int64_t g4 = (p.M + 63) / 64, n16 = (p.N + 15) / 16;
+    auto go = [&]<int KT, int SD>() {
+        const int tg = (int)((n16 + KT - 1) / KT);
+        NC_LAUNCH((gemm_k_prompt_kernel<LAYOUT, Q5, KT, SD>), dim3((unsigned)(g4 * tg)), dim3(256), 0, st, p, tg);
+    };
+    // As launch_b32_prompt, with more work per output to spread over waves.  Measured (us, Q4_K, 4 / 2 / 1 token
+    // tiles): 16384 x 3072 x 256 tokens (1024 workgroups with 4) 97 / 101 / 135, 8192 x 3072 x 250 (512 with 4) 58 /
+    // 56 / 74, x 128 (512 with 2) 47 / 39 / 43, x 64 (256) 45 / 32 / 28; 3072 x 8192 x 256 (384 with 2) 108 / 83 / 73.
+    if (n16 > 2 && g4 * ((n16 + 3) / 4) >= 1024) go.template operator()<4, 1>();
+    else if (n16 > 1 && g4 * ((n16 + 1) / 2) >= 512) go.template operator()<2, 1>();
+    else go.template operator()<1, 2>();
+}
+
+int launch_gemm_prompt_k(const QMatDev& w, float* out, int ld_out, int N, hipStream_t st, const void* xh,
+                         const float* xsm, const float* xam) {
+    if ((w.type != NC_TYPE_Q4_K && w.type != NC_TYPE_Q5_K) || (w.layout != LAYOUT_R16K && w.layout != LAYOUT_R64))
+        return fail(NC_EINVAL, "K-quant prompt matmul: Q4_K and Q5_K matrices only");
+    if (!xh || !xsm || !xam) return fail(NC_EINVAL, "K-quant prompt matmul: repacked activations required");
+    if (N < 1 || (int64_t)N * w.cols >= (int64_t)1 << 30 || w.dev_bytes >= (int64_t)1 << 31)
+        return fail(NC_ERANGE, "K-quant prompt matmul: operands exceed 2 GiB");
     PromptGemmK p;
     p.w = w.dev;
-    p.w_bytes = w.dev_bytes;
     p.nsb = (int)(w.cols / 256);
     p.groups = (int)w.groups;
     p.tiles16 = (int)(w.layout == LAYOUT_R16K ? w.tiles : 4 * w.tiles);
     p.M = (int)w.rows;
     p.N = N;
     p.ld_out = ld_out;
-    p.xm = (const uint2*)xm;
-    p.xsm = (const float4*)xsm;
-    p.xam = (const float4*)xam;
+    p.xh = (const uint8_t*)xh;
+    p.xsm = xsm;
+    p.xam = xam;
     p.out = out;
-    if (prompt_row_tiles(w.rows, N) == 2) {
-        const dim3 grid((unsigned)((w.rows + 63) / 64), (unsigned)((N + 63) / 64));
-        if (w.layout == LAYOUT_R16K) NC_LAUNCH((gemm_q4_k_prompt_kernel<LAYOUT_R16K, 2>), grid, dim3(256), 0, st, p);
-        else NC_LAUNCH((gemm_q4_k_prompt_kernel<LAYOUT_R64, 2>), grid, dim3(256), 0, st, p);
+    if (w.type == NC_TYPE_Q5_K) {
+        if (w.layout == LAYOUT_R16K) launch_k_prompt<LAYOUT_R16K, true>(p, st);
+        else launch_k_prompt<LAYOUT_R64, true>(p, st);
     } else {
-        const dim3 grid((unsigned)((w.rows + 63) / 64), (unsigned)((N + 31) / 32));
-        if (w.layout == LAYOUT_R16K) NC_LAUNCH((gemm_q4_k_prompt_kernel<LAYOUT_R16K, 1>), grid, dim3(256), 0, st, p);
-        else NC_LAUNCH((gemm_q4_k_prompt_kernel<LAYOUT_R64, 1>), grid, dim3(256), 0, st, p);
+        if (w.layout == LAYOUT_R16K) launch_k_prompt<LAYOUT_R16K, false>(p, st);
+        else launch_k_prompt<LAYOUT_R64, false>(p, st);
     }
     NC_HIP(hipGetLastError());
     return NC_OK;
 }
 
-// Activations in MFMA operand order for the prompt matmul: xm unit (tile t, block b, lane
-// (g, c)) = token 16t + c's bytes 32b + 4g..+3 and 32b + 16 + 4g..+3 (zero past N), so a wave
-// reads a block's B operand as 512 contiguous bytes; xsm (t, quad q, c) = token 16t + c's scales
-// of blocks 4q..4q+3 (zero past the row).  Units of x first, then of the scales.
-__global__ void prompt_repack_kernel(const int8_t* x, const float* xs, int N, int nb, uint2* xm, float4* xsm,
-                                     float4* xam) {
-    const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int n16 = (N + 15) / 16, nq = (nb + 3) / 4, K = 32 * nb;
-    const int64_t nx = (int64_t)n16 * nb * 64;
-    if (id < nx) {
-        const int lane = (int)(id & 63), g = lane >> 4, c = lane & 15;
-        const int64_t tb = id >> 6;
-        const int b = (int)(tb % nb), n = (int)(tb / nb) * 16 + c;
-        uint2 v = make_uint2(0u, 0u);
-        if (n < N) {
-            const int8_t* row = x + (size_t)n * K + 32 * b + 4 * g;
-            v.x = *(const uint32_t*)row;
-            v.y = *(const uint32_t*)(row + 16);
-        }
-        xm[id] = v;
-        return;
-    }
-    const int64_t id2 = id - nx;
-    if (id2 >= (int64_t)n16 * nq * 16) return;
-    const int c = (int)(id2 & 15);
-    const int64_t tq = id2 >> 4;
-    const int q = (int)(tq % nq), n = (int)(tq / nq) * 16 + c;
-    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (n < N) {
-        const float* sr = xs + (size_t)n * nb + 4 * q;
-        v.x = sr[0];
-        if (4 * q + 1 < nb) v.y = sr[1];
-        if (4 * q + 2 < nb) v.z = sr[2];
-        if (4 * q + 3 < nb) v.w = sr[3];
-    }
-    xsm[id2] = v;
-    if (xam) {  // (float) sum of each block's int8 values (exact: |sum| <= 32 * 128)
-        float sa[4] = {0.f, 0.f, 0.f, 0.f};
-        if (n < N) {
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                if (4 * q + e >= nb) break;
-                const int* blk = (const int*)(x + (size_t)n * K + 32 * (4 * q + e));
-                int sum = 0;
-#pragma unroll
-                for (int d = 0; d < 8; d++) sum = __builtin_amdgcn_sdot4(blk[d], 0x01010101, sum, false);
-                sa[e] = (float)sum;
-            }
-        }
-        xam[id2] = make_float4(sa[0], sa[1], sa[2], sa[3]);
-    }
-}
-
-// The same as f16 for gemm_b32_prompt_kernel: xh unit (tile t, block b of 4 nq, lane (g, c)) = token 16t +
-// c's elements 0, 2, 16, 18, 1, 3, 17, 19 + 4g of the block, xsm (t, quad, lane (j, c)) its scale of
-// block 4 quad + j; zero past N and past the row's blocks.  One thread per unit lane, then per scale.
-__global__ void prompt_repack_f16_kernel(const int8_t* x, const float* xs, int N, int nb, uint4* xh, float* xsm) {
+// Activations in operand order as f16: xh unit (tile t, block b of 4 nq, lane (g, c)) = token 16t +
+// c's elements 0, 2, 16, 18, 1, 3, 17, 19 + 4g of the block, zero past N and past the row's blocks.  xam null:
+// xsm (t, quad, lane (j, c)) = its scale of block 4 quad + j; else (K-quants) xsm (t, quad, c, j) and xam (t,
+// quad, lane (j, c)) = the float sum of the block's values (exact).  One thread per unit lane, then per scale.
+__global__ void prompt_repack_kernel(const int8_t* x, const float* xs, int N, int nb, uint4* xh, float* xsm,
+                                     float* xam) {
     const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int n16 = (N + 15) / 16, nbp = (nb + 3) / 4 * 4, K = 32 * nb;
     const int64_t nx = (int64_t)n16 * nbp * 64;
@@ -549,24 +502,25 @@ __global__ void prompt_repack_f16_kernel(const int8_t* x, const float* xs, int N
     const int c = (int)(id2 & 15), j = (int)(id2 >> 4) & 3;
     const int64_t tq = id2 >> 6;
     const int b = (int)(tq % (nbp / 4)) * 4 + j, n = (int)(tq / (nbp / 4)) * 16 + c;
-    xsm[id2] = n < N && b < nb ? xs[(size_t)n * nb + b] : 0.0f;
+    const bool live = n < N && b < nb;
+    xsm[xam ? tq * 64 + 4 * c + j : id2] = live ? xs[(size_t)n * nb + b] : 0.0f;
+    if (xam) {
+        int sum = 0;
+        if (live) {
+            const int* e = (const int*)(x + (size_t)n * K + 32 * b);
+#pragma unroll
+            for (int d = 0; d < 8; d++) sum = __builtin_amdgcn_sdot4(e[d], 0x01010101, sum, false);
+        }
+        xam[id2] = (float)sum;
+    }
 }
 
-int launch_prompt_repack_f16(const int8_t* x, const float* xs, int N, int K, void* xh, float* xsm, hipStream_t st) {
+int launch_prompt_repack(const int8_t* x, const float* xs, int N, int K, void* xh, float* xsm, hipStream_t st,
+                         float* xam) {
     const int nb = K / 32;
     const int64_t total = (int64_t)((N + 15) / 16) * ((nb + 3) / 4 * 4) * 80;
-    NC_LAUNCH(prompt_repack_f16_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, x, xs, N, nb,
-              (uint4*)xh, xsm);
-    NC_HIP(hipGetLastError());
-    return NC_OK;
-}
-
-int launch_prompt_repack(const int8_t* x, const float* xs, int N, int K, void* xm, float* xsm, hipStream_t st,
-                         float* xam) {
-    const int nb = K / 32, n16 = (N + 15) / 16, nq = (nb + 3) / 4;
-    const int64_t total = (int64_t)n16 * nb * 64 + (int64_t)n16 * nq * 16;
-    NC_LAUNCH(prompt_repack_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, x, xs, N, nb,
-                       (uint2*)xm, (float4*)xsm, (float4*)xam);
+    NC_LAUNCH(prompt_repack_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, x, xs, N, nb, (uint4*)xh,
+              xsm, xam);
     NC_HIP(hipGetLastError());
     return NC_OK;
 }

@@ -1164,7 +1164,8 @@ static int sample_session_rows(nc_session* s, int row0, int rows, float temp, co
 static bool prompt_matrix_ok(const QMatDev& q) {
     if (q.type == NC_TYPE_Q4_0) return q.layout == LAYOUT_R16 || q.layout == LAYOUT_R64;
     if (q.type == NC_TYPE_Q4_K) return q.layout == LAYOUT_R16K || q.layout == LAYOUT_R64;
-    if (q.type == NC_TYPE_Q8_0) return q.dev_bytes < (int64_t)1 << 31;  // larger ones in 16-token slices
+    if (q.type == NC_TYPE_Q8_0 || q.type == NC_TYPE_Q5_K)
+        return q.dev_bytes < (int64_t)1 << 31;  // larger ones in 16-token slices
     return false;
 }
 
@@ -1182,7 +1183,7 @@ static bool needs_block_sums(const nc_ctx* ctx, const QMatDev& q, int n) {
            (q.type == NC_TYPE_Q4_0 && ctx->gemm_kernel == NC_GEMM_KERNEL_MFMA);
 }
 
-// Prompt passes take every layer matrix on a prompt kernel, or Q5_K and Q6_K ones on the verify kernels.
+// Prompt passes take every layer matrix on a prompt kernel, or the verify kernels.
 static bool prompt_path_ok(const nc_model* m) {
     for (const LayerDev& L : m->layers)
         for (const QMatDev* q : L.all())
@@ -1192,16 +1193,14 @@ static bool prompt_path_ok(const nc_model* m) {
     return true;
 }
 
-// Prompt matmul of n tokens (Q4_0, Q8_0 or Q4_K) over activations repacked into xm / xsm (/ xam).
+// Prompt matmul of n tokens (any type but Q6_K) over activations repacked into xm / xsm (/ xam).
 static int prompt_matmul(const QMatDev& w, const int8_t* xq, const float* xs, float* out, int ld_out, int n,
                          hipStream_t st, int8_t* xm, float* xsm, float* xam) {
     int rc;
-    if (w.type == NC_TYPE_Q4_K) {
-        if ((rc = launch_prompt_repack(xq, xs, n, (int)w.cols, xm, xsm, st, xam))) return rc;
-        return launch_gemm_prompt_q4k(w, out, ld_out, n, st, xm, xsm, xam);
-    }
-    if ((rc = launch_prompt_repack_f16(xq, xs, n, (int)w.cols, xm, xsm, st))) return rc;
-    return launch_gemm_prompt(w, out, ld_out, n, st, xm, xsm);
+    const bool k = w.type == NC_TYPE_Q4_K || w.type == NC_TYPE_Q5_K;
+    if ((rc = launch_prompt_repack(xq, xs, n, (int)w.cols, xm, xsm, st, k ? xam : nullptr))) return rc;
+    return k ? launch_gemm_prompt_k(w, out, ld_out, n, st, xm, xsm, xam)
+             : launch_gemm_prompt(w, out, ld_out, n, st, xm, xsm);
 }
 
 static int ensure_prompt_bufs(nc_session* s) {
@@ -1228,7 +1227,7 @@ static int ensure_prompt_bufs(nc_session* s) {
 
 // Prompt matmul of the pass's activations (repacked first into MFMA operand order).
 // A prompt pass's matmul into rows of stride ld (default: the matrix's rows): the MFMA prompt
-// kernels, or for Q5_K and Q6_K matrices (no prompt kernel) the verify kernel.
+// kernels, or for Q6_K matrices (no prompt kernel) the verify kernel.
 static int prompt_gemm(nc_session* s, const QMatDev& w, const int8_t* xq, const float* xs, float* out, int n,
                        int ld = 0) {
     if (ld == 0) ld = (int)w.rows;

@@ -49,6 +49,16 @@ def test_q8_0_tile_edges(ctx, M, K):
 
 # the prompt matmul's wave tiles: 16 x 32 (few workgroups), 16 x 64 and 32 x 64 (many), on 16-row tiles and, from
 # 65536 rows of Q4_0, on 64-row tiles; K: one block, cut quads, an odd number of quads; ragged rows and tokens
+@pytest.mark.parametrize("qtype", ["q4_k", "q5_k"])
+@pytest.mark.parametrize("M,K,batches", [(17, 256, [17, 33, 64]), (200, 1280, [40, 130, 300]), (16401, 512, [129, 66]),
+                                         (16000, 256, [260, 40])])
+def test_prompt_k_quant_matmul_wave_tiles(ctx, qtype, M, K, batches):
+    if qtype == "q4_k":
+        check(ctx, nc.NC_TYPE_Q4_K, random_q4_k(M, K, seed=M), O.matmul_q4_k, M, K, batches, 9)
+    else:
+        check(ctx, nc.NC_TYPE_Q5_K, random_q5_k(M, K, seed=M), O.matmul_q5_k, M, K, batches, 10)
+
+
 @pytest.mark.parametrize("qtype", ["q4_0", "q8_0"])
 @pytest.mark.parametrize("M,K,batches", [(17, 32, [17, 33, 64]), (200, 416, [40, 130, 300]), (16401, 96, [129, 66]),
                                          (32785, 288, [130]), (65553, 96, [20, 65]), (20, 8224, [31, 49])])
