@@ -177,11 +177,18 @@ constexpr int kChainMargin = 256;  // ulps between a guess and the true state th
 
 // Step 2 for one thread: its E terms added in order from the guess g; x receives the end
 // value.  Returns whether moving the run to the true start might not translate it exactly:
-// the guess or the end lies within kChainMargin ulps of a binade edge, the run leaves the
+// the guess or the end lies within MARGIN ulps of a binade edge, the run leaves the
 // guess's binade, a step rounds an exact tie, or the binade is too small for the test.
 // s0_neg: the chain started below zero, so a zero guess is a cancellation, not an exact start.
-template <int E>
-__device__ __forceinline__ bool chain_run_sensitive(const float (&a)[E], float g, bool s0_neg, float& x_out) {
+// MARGIN: the ulps by which the true start may differ from the guess.  The chain's accumulated rounding grows
+// with its length (about 2,500 ulps over 128,256 softmax terms of which few are large), and a start further off
+// than the margin near a binade edge costs a sequential evaluation; each binade edge makes the runs
+// within the margin sensitive.
+// floor1: the true start is known to be at least 1 (a term of 1 came before: the chain never falls), so a guess
+// in [1, 2) cannot be off below its binade.
+template <int E, int MARGIN = kChainMargin>
+__device__ __forceinline__ bool chain_run_sensitive(const float (&a)[E], float g, bool s0_neg, float& x_out,
+                                                    bool floor1 = false) {
     const uint32_t bg = __float_as_uint(g);
     const int eg = (int)(bg >> 23);  // sign and exponent: the binade test below includes the sign
     const int ea = eg & 0xff;
@@ -210,7 +217,8 @@ __device__ __forceinline__ bool chain_run_sensitive(const float (&a)[E], float g
     // g == 0 with s0 >= 0: every earlier term and s0 are 0, so the start is exact and the run
     // is the truth
     return !absorbed & ((bg != 0) | s0_neg) &
-           ((ea < 25) | ((int)(bx >> 23) != eg) | (mg < kChainMargin) | (mx + kChainMargin >= (1 << 23)) | tie);
+           ((ea < 25) | ((int)(bx >> 23) != eg) | ((mg < MARGIN) & !(floor1 & (eg == 127))) |
+            (mx + MARGIN >= (1 << 23)) | tie);
 }
 
 // The walk's serial part, run by one lane: adds rows[0 .. cnt) in order to S (a row holds the
@@ -262,7 +270,7 @@ __device__ __forceinline__ float chain_walk_rows(const WalkRow<E>* rows, int cnt
 // neighbourhood only makes segments sensitive.  a_lds: n floats of LDS used by the walk and
 // the fallback.  Every thread of the block must call it; returns s_{n-1} to all threads.
 // FIND: sc.first also receives the first index i (0 .. n-1) with s_i >= 0, or INT_MAX.
-template <int E, int T, bool FIND = false>
+template <int E, int T, bool FIND = false, int MARGIN = kChainMargin>
 __device__ float exact_chain_sum(const float (&a)[E], ChainScratch<T>& sc, float* a_lds, float s0 = 0.0f) {
     static_assert(E >= 1 && E <= 32, "terms per thread");
     const int t = threadIdx.x;
@@ -278,7 +286,7 @@ __device__ float exact_chain_sum(const float (&a)[E], ChainScratch<T>& sc, float
 
     // 2. the segment evaluated from the guess, with the tie and binade tests
     float x;
-    const bool sens = chain_run_sensitive<E>(a, g, s0 < 0.0f, x);
+    const bool sens = chain_run_sensitive<E, MARGIN>(a, g, s0 < 0.0f, x);
     const double d = (double)x - (double)g;
 
     // 3. uncorrected starts C_t, with the sensitive count scanned in the same pass

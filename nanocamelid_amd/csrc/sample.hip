@@ -59,6 +59,8 @@ __device__ inline uint64_t fixed_weight(float w) { return w > 0.0f ? (uint64_t)(
 constexpr int kSmT = 1024;             // threads per row
 constexpr int kSmE = 16;               // chain terms per thread per segment
 constexpr int kSmSeg = kSmT * kSmE;    // terms per exact-chain segment
+constexpr int kSmMargin = 2048;        // chain_run_sensitive margin within a segment from its exact start
+constexpr int kTpMargin = 4096;        // and over a whole row from the double prefix
 
 __device__ inline float wave_max(float v) {
 #pragma unroll
@@ -68,7 +70,7 @@ __device__ inline float wave_max(float v) {
 
 // The order-free passes (max, e_j, p_j = e_j * (1/S)) run on kTpCh workgroups per row.  The
 // exact sequential sum S runs its kSmSeg-term segments on one workgroup each (the evaluation
-// of exact_chain_sum spread over the segments: tps_run, tps_walk, tps_verify, tps_finish) when
+// of exact_chain_sum spread over the segments: tps_run, tps_verify, tps_finish) when
 // the row has at most kTpSegMax segments, else on one workgroup per row, segment after
 // segment.  e_j is kept in the output row between the passes.
 constexpr int kTpCh = 64;
@@ -78,7 +80,6 @@ constexpr int kTpEntCap = 256;  // sensitive runs listed per segment
 
 struct TpSegInfo {
     double dtot;      // sum of the segment's run increments (runs evaluated from the guesses)
-    double shift_in;  // correction of the last sensitive run before the segment (0: none)
     int nsens;        // sensitive runs in the segment (more than kTpEntCap: not listed)
     int bad;          // a boundary check inside the segment failed
     float first;      // verified start of the segment's first run
@@ -94,9 +95,9 @@ struct TpEnt {
 struct TpRowScratch {
     float cmax[kTpCh];  // chunk maxima
     float inv, S;       // 1 / S and S
-    int ok;             // the walk listed every sensitive run
     int fast;           // S came from the parallel evaluation (else from the sequential fallback)
     double csum[kTpCh];                      // chunk sums of e in double (the guesses' prefix)
+    int cone[kTpCh];                         // whether the chunk holds a maximum, whose e is 1
     TpSegInfo seg[kTpSegMax];
     TpEnt ent[kTpSegMax * kTpEntCap];
     double crun[kTpSegMax * kSmT];  // uncorrected start of each run, relative to its segment
@@ -119,13 +120,25 @@ __device__ inline int tp_chunk(int V) {
     return c;
 }
 
+// Whether elements lo..hi-1 of a row can be taken four at a time (16-byte loads).
+__device__ inline bool tp_quads(const float* row, int lo, int hi) {
+    return (reinterpret_cast<uintptr_t>(row + lo) & 15) == 0 && ((hi - lo) & 3) == 0;
+}
+
 __global__ __launch_bounds__(kTpT) void tp_max_kernel(const float* logits, int64_t ld_in, int V, float* scratch) {
     __shared__ float wm[kTpT / 64];
     const int row = blockIdx.y, c = blockIdx.x, t = threadIdx.x;
     const float* l = logits + (size_t)row * ld_in;
     const int lo = min(c * tp_chunk(V), V), hi = min(lo + tp_chunk(V), V);
     float mx = -INFINITY;
-    for (int i = lo + t; i < hi; i += kTpT) mx = fmaxf(mx, l[i]);
+    if (tp_quads(l, lo, hi)) {
+        for (int i = lo + 4 * t; i < hi; i += 4 * kTpT) {
+            const float4 v = *(const float4*)(l + i);
+            mx = fmaxf(fmaxf(fmaxf(fmaxf(mx, v.x), v.y), v.z), v.w);
+        }
+    } else {
+        for (int i = lo + t; i < hi; i += kTpT) mx = fmaxf(mx, l[i]);
+    }
     mx = wave_max(mx);
     if ((t & 63) == 0) wm[t >> 6] = mx;
     __syncthreads();
@@ -151,10 +164,21 @@ __global__ __launch_bounds__(kTpT) void tp_exp_kernel(const float* logits, int64
     float* e = probs + (size_t)row * ld_out;
     const int lo = min(c * tp_chunk(V), V), hi = min(lo + tp_chunk(V), V);
     double sum = 0.0;
-    for (int i = lo + t; i < hi; i += kTpT) {
-        const float v = expf_glibc((l[i] - mx) / temp);
-        e[i] = v;
-        sum += (double)v;
+    if (tp_quads(l, lo, hi) && tp_quads(e, lo, hi)) {
+#pragma unroll 2
+        for (int i = lo + 4 * t; i < hi; i += 4 * kTpT) {
+            const float4 x = *(const float4*)(l + i);
+            const float4 v = make_float4(expf_glibc((x.x - mx) / temp), expf_glibc((x.y - mx) / temp),
+                                         expf_glibc((x.z - mx) / temp), expf_glibc((x.w - mx) / temp));
+            *(float4*)(e + i) = v;
+            sum += ((double)v.x + (double)v.y) + ((double)v.z + (double)v.w);
+        }
+    } else {
+        for (int i = lo + t; i < hi; i += kTpT) {
+            const float v = expf_glibc((l[i] - mx) / temp);
+            e[i] = v;
+            sum += (double)v;
+        }
     }
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) sum += __shfl_xor(sum, o);
@@ -165,6 +189,7 @@ __global__ __launch_bounds__(kTpT) void tp_exp_kernel(const float* logits, int64
 #pragma unroll
         for (int w = 0; w < kTpT / 64; w++) c_sum += ws[w];
         R->csum[c] = c_sum;
+        R->cone[c] = R->cmax[c] == mx;
     }
 }
 
@@ -179,7 +204,7 @@ __device__ float tp_sum_segments(const float* e, int V, ChainScratch<kSmT>& sc, 
             const int i = base + t * kSmE + j;
             a[j] = i < V ? e[i] : 0.0f;
         }
-        sum = exact_chain_sum<kSmE, kSmT>(a, sc, a_lds, sum);
+        sum = exact_chain_sum<kSmE, kSmT, false, kSmMargin>(a, sc, a_lds, sum);
     }
     return sum;
 }
@@ -204,14 +229,18 @@ __global__ __launch_bounds__(kSmT) void tp_sum_kernel(const float* probs, int64_
 //               chunk sums before the segment plus the block scan), the runs from the guesses
 //               and their sensitivity, the uncorrected starts relative to the segment and the
 //               segment's list of sensitive runs;
-//   tps_walk    (one wave per row) step 4: the segment bases C_g (sums of the earlier
-//               segments' increments, in order), then the walk over every listed run of the
-//               row, which fixes each run's correction;
-//   tps_verify  (segment x row) step 5: every run recomputed from its corrected start and
-//               every boundary inside the segment checked;
-//   tps_finish  (one workgroup per row) the boundaries between segments; if any check
-//               failed, or a segment had more sensitive runs than it lists, S is evaluated
-//               segment after segment as tp_sum_kernel does.
+//   tps_verify  (segment x row) steps 4 and 5: the segment bases C_g (sums of the earlier segments'
+//               increments, in order); one wave walks every listed run of the row up to the
+//               workgroup's own segment, which fixes each run's correction (each workgroup for
+//               itself: a launch of its own and the corrections' way through memory took 3 us
+//               more); then every run is recomputed from its corrected start and every boundary
+//               inside the segment checked;
+//   tps_finish  the boundaries between segments; if any check failed, or a segment had more
+//               sensitive runs than it lists, S is evaluated segment after segment as
+//               tp_sum_kernel does.  With NORM, one workgroup per segment also scales its
+//               probabilities by 1 / S (in that rare case every one evaluates S).
+// 5 rows of 128256 (launches included): 30 us, where walk, verify, finish and norm as four launches and a margin of
+// 256 ulps, which rows of N(0, 2.5) logits overran on some binade edges, took 50 us, or 130 with such a row.
 // As in exact_chain_sum, the result is the sequential chain whenever it is accepted: the
 // verified starts equal the previous runs' ends at every boundary, so by induction the last
 // end is s_{V-1}.
@@ -239,6 +268,7 @@ __global__ __launch_bounds__(kSmT) void tps_run_kernel(const float* probs, int64
     __shared__ double dtot[kSmT / 64], dtot2[kSmT / 64];
     __shared__ int itot[kSmT / 64];
     __shared__ double s_base;
+    __shared__ int s_one;  // first run after a term of 1 (the row's maximum)
     const int g = blockIdx.x, row = blockIdx.y, t = threadIdx.x;
     TpRowScratch* R = tp_row(scratch, row);
     const float* e = probs + (size_t)row * ld;
@@ -247,9 +277,14 @@ __global__ __launch_bounds__(kSmT) void tps_run_kernel(const float* probs, int64
     tps_load_run(e, V, base + t * kSmE, a);
     if (t == 0) {
         double P = 0.0;
+        int one = kSmT;
         const int cb = base / tp_chunk(V);  // chunks tile the segments
-        for (int c = 0; c < cb; c++) P += R->csum[c];
+        for (int c = 0; c < cb; c++) {
+            P += R->csum[c];
+            if (R->cone[c]) one = 0;
+        }
         s_base = P;
+        s_one = one;
     }
     // 1. guess: the double prefix of every earlier term
     double run = 0.0;
@@ -257,9 +292,14 @@ __global__ __launch_bounds__(kSmT) void tps_run_kernel(const float* probs, int64
     for (int j = 0; j < kSmE; j++) run += (double)a[j];
     const double lp = block_excl_scan_f64<kSmT>(run, dtot);  // its barrier publishes s_base
     const float gs = (float)(s_base + lp);
+    bool here = false;
+#pragma unroll
+    for (int j = 0; j < kSmE; j++) here |= a[j] >= 1.0f;
+    if (here) atomicMin(&s_one, t + 1);
+    __syncthreads();
     // 2. the run from the guess
     float x;
-    const bool sens = chain_run_sensitive<kSmE>(a, gs, false, x);
+    const bool sens = chain_run_sensitive<kSmE, kTpMargin>(a, gs, false, x, t >= s_one);
     const double d = (double)x - (double)gs;
     // 3. uncorrected start relative to the segment, sensitive count before the run
     int off, total_s;
@@ -279,18 +319,24 @@ __global__ __launch_bounds__(kSmT) void tps_run_kernel(const float* probs, int64
     }
 }
 
-__global__ __launch_bounds__(64) void tps_walk_kernel(const float* probs, int64_t ld, int V, float* scratch) {
+__global__ __launch_bounds__(kSmT) void tps_verify_kernel(const float* probs, int64_t ld, int V, float* scratch) {
     constexpr int W = WalkRow<kSmE>::W;
     __shared__ WalkRow<kSmE> rows[64];
     __shared__ float walk_end[64];
     __shared__ double cbase[kTpSegMax + 1];
     __shared__ int eoff[kTpSegMax + 1];
     __shared__ double shifts[kTpSegMax * kTpEntCap];
+    __shared__ float last[kSmT];
     __shared__ int s_listed;
-    const int row = blockIdx.x, t = threadIdx.x;
+    const int gs = blockIdx.x, row = blockIdx.y, t = threadIdx.x;
     TpRowScratch* R = tp_row(scratch, row);
     const float* e = probs + (size_t)row * ld;
     const int nseg = (V + kSmSeg - 1) / kSmSeg;
+    float a[kSmE];
+    tps_load_run(e, V, gs * kSmSeg + t * kSmE, a);
+    const int r = gs * kSmT + t;
+    const int off = R->off[r];
+    const double crun = R->crun[r];
     if (t == 0) {
         double c = 0.0;
         int n = 0;
@@ -303,127 +349,110 @@ __global__ __launch_bounds__(64) void tps_walk_kernel(const float* probs, int64_
             listed = listed && ns <= kTpEntCap;
             n += min(ns, kTpEntCap);
         }
-        cbase[nseg] = c;
         eoff[nseg] = n;
         s_listed = listed ? 1 : 0;
     }
     __syncthreads();
-    if (!s_listed) {
-        if (t == 0) R->ok = 0;
-        return;
-    }
-    const int total = eoff[nseg];
-    float S = 0.0f;  // true chain value after the last walked run (lane 0)
-    for (int e0 = 0; e0 < total; e0 += 64) {
-        const int me = e0 + t;
-        const int cnt = min(64, total - e0);
-        double ce = 0.0;
-        if (me < total) {
-            int g = 0;
-            while (g + 1 < nseg && eoff[g + 1] <= me) g++;
-            const TpEnt& en = R->ent[g * kTpEntCap + (me - eoff[g])];
-            const double cs = cbase[g] + en.cstart;
-            ce = cbase[g] + en.cend;
-            double cprev = 0.0;  // uncorrected end of the previous listed run (the chain starts at 0)
-            if (me > 0) {
-                int gp = g;
-                while (eoff[gp] > me - 1) gp--;
-                cprev = cbase[gp] + R->ent[gp * kTpEntCap + (me - 1 - eoff[gp])].cend;
+    if (!s_listed) return;  // uniform over the row: tps_finish takes the sequential evaluation
+    if (t < 64) {
+        // wave 0; the LDS rows and walk ends of one wave complete in order
+        const int total = eoff[gs + 1];
+        float S = 0.0f;  // true chain value after the last walked run (lane 0)
+        for (int e0 = 0; e0 < total; e0 += 64) {
+            const int me = e0 + t;
+            const int cnt = min(64, total - e0);
+            double ce = 0.0;
+            if (me < total) {
+                int g = 0;
+                while (g + 1 < nseg && eoff[g + 1] <= me) g++;
+                const TpEnt& en = R->ent[g * kTpEntCap + (me - eoff[g])];
+                const double cs = cbase[g] + en.cstart;
+                ce = cbase[g] + en.cend;
+                double cprev = 0.0;  // uncorrected end of the previous listed run (the chain starts at 0)
+                if (me > 0) {
+                    int gp = g;
+                    while (eoff[gp] > me - 1) gp--;
+                    cprev = cbase[gp] + R->ent[gp * kTpEntCap + (me - 1 - eoff[gp])].cend;
+                }
+                rows[t].v[0] = (float)(cs - cprev);  // exact advance over the insensitive runs between
+                float er[kSmE];
+                tps_load_run(e, V, en.run * kSmE, er);
+#pragma unroll
+                for (int j = 0; j < kSmE; j++) rows[t].v[1 + j] = er[j];
+#pragma unroll
+                for (int j = kSmE + 1; j < W; j++) rows[t].v[j] = 0.0f;
             }
-            rows[t].v[0] = (float)(cs - cprev);  // exact advance over the insensitive runs between
-            const int i0 = en.run * kSmE;
-#pragma unroll
-            for (int j = 0; j < kSmE; j++) rows[t].v[1 + j] = i0 + j < V ? e[i0 + j] : 0.0f;
-#pragma unroll
-            for (int j = kSmE + 1; j < W; j++) rows[t].v[j] = 0.0f;
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            if (t == 0) S = chain_walk_rows<kSmE>(rows, cnt, S, walk_end);
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            if (me < total) shifts[me] = (double)walk_end[t] - ce;
+            __builtin_amdgcn_wave_barrier();
         }
-        __syncthreads();
-        if (t == 0) S = chain_walk_rows<kSmE>(rows, cnt, S, walk_end);
-        __syncthreads();
-        if (me < total) shifts[me] = (double)walk_end[t] - ce;
-        __syncthreads();  // rows and walk_end are rewritten by the next window
-    }
-    for (int g = t; g < nseg; g += 64) R->seg[g].shift_in = eoff[g] > 0 ? shifts[eoff[g] - 1] : 0.0;
-    for (int i = t; i < total; i += 64) {
-        int g = 0;
-        while (g + 1 < nseg && eoff[g + 1] <= i) g++;
-        R->ent[g * kTpEntCap + (i - eoff[g])].shift = shifts[i];
-    }
-    if (t == 0) R->ok = 1;
-}
-
-__global__ __launch_bounds__(kSmT) void tps_verify_kernel(const float* probs, int64_t ld, int V, float* scratch) {
-    __shared__ float last[kSmT];
-    __shared__ double s_cb;
-    __shared__ int s_ok;
-    const int g = blockIdx.x, row = blockIdx.y, t = threadIdx.x;
-    TpRowScratch* R = tp_row(scratch, row);
-    if (t == 0) {
-        s_ok = R->ok;
-        double c = 0.0;  // the walk's segment base, summed in the same order
-        for (int h = 0; h < g; h++) c += R->seg[h].dtot;
-        s_cb = c;
     }
     __syncthreads();
-    if (!s_ok) return;  // uniform: tps_finish takes the sequential evaluation
-    const float* e = probs + (size_t)row * ld;
-    const int base = g * kSmSeg;
-    float a[kSmE];
-    tps_load_run(e, V, base + t * kSmE, a);
-    const int r = g * kSmT + t;
-    const int off = R->off[r];
-    const double sh = off > 0 ? R->ent[g * kTpEntCap + off - 1].shift : R->seg[g].shift_in;
-    const float start = (float)((s_cb + R->crun[r]) + sh);
+    const int le = eoff[gs] + off;  // listed runs before this one
+    const float start = (float)((cbase[gs] + crun) + (le > 0 ? shifts[le - 1] : 0.0));
     float y = start;
 #pragma unroll
     for (int j = 0; j < kSmE; j++) y = y + a[j];
     last[t] = y;
-    bool bad = (g == 0 && t == 0) ? start != 0.0f : false;
+    bool bad = (gs == 0 && t == 0) ? start != 0.0f : false;
     __syncthreads();
     if (t > 0) bad |= start != last[t - 1];
     bad = __syncthreads_or(bad);
     if (t == 0) {
-        R->seg[g].bad = bad ? 1 : 0;
-        R->seg[g].first = start;
+        R->seg[gs].bad = bad ? 1 : 0;
+        R->seg[gs].first = start;
     }
-    if (t == kSmT - 1) R->seg[g].last = y;
+    if (t == kSmT - 1) R->seg[gs].last = y;
 }
 
-__global__ __launch_bounds__(kSmT) void tps_finish_kernel(const float* probs, int64_t ld, int V, float* scratch) {
+template <bool NORM>
+__global__ __launch_bounds__(kSmT) void tps_finish_kernel(float* probs, int64_t ld, int V, float* scratch) {
     __shared__ ChainScratch<kSmT> sc;
     __shared__ __align__(16) float a_lds[kSmSeg];
     __shared__ int s_ok;
     __shared__ float s_sum;
-    const int row = blockIdx.x, t = threadIdx.x;
+    const int row = blockIdx.y, t = threadIdx.x;
     TpRowScratch* R = tp_row(scratch, row);
+    float* e = probs + (size_t)row * ld;
     if (t == 0) {
         const int nseg = (V + kSmSeg - 1) / kSmSeg;
-        bool ok = R->ok != 0;
+        bool ok = true;
+        for (int g = 0; g < nseg; g++) ok = ok && R->seg[g].nsens <= kTpEntCap;
         for (int g = 0; ok && g < nseg; g++) ok = !R->seg[g].bad && (g == 0 || R->seg[g].first == R->seg[g - 1].last);
         s_ok = ok ? 1 : 0;
         s_sum = ok ? R->seg[nseg - 1].last : 0.0f;
     }
     __syncthreads();
     const bool ok = s_ok != 0;
-    const float sum = ok ? s_sum : tp_sum_segments(probs + (size_t)row * ld, V, sc, a_lds);
-    if (t == 0) {
-        R->inv = 1.0f / sum;
+    // the sequential evaluation reads the whole row, so there one workgroup does all of it
+    if (!ok && blockIdx.x > 0) return;
+    const float sum = ok ? s_sum : tp_sum_segments(e, V, sc, a_lds);
+    const float inv = 1.0f / sum;
+    if (blockIdx.x == 0 && t == 0) {
+        R->inv = inv;
         R->S = sum;
         R->fast = ok ? 1 : 0;
     }
-}
-
-// S and 1/S of every row, by the parallel segments when the row fits kTpSegMax of them.
-static void launch_tp_sum(const float* probs, int64_t ld, int rows, int V, float* rs, hipStream_t st) {
-    const int nseg = (V + kSmSeg - 1) / kSmSeg;
-    if (nseg > kTpSegMax) {
-        hipLaunchKernelGGL(tp_sum_kernel, dim3(rows), dim3(kSmT), 0, st, probs, ld, V, rs);
-        return;
+    if constexpr (NORM) {
+        // p_j = e_j * (1 / S) (inference.rs:3535-3539), in place
+        const int lo = ok ? blockIdx.x * kSmSeg : 0, hi = ok ? min(lo + kSmSeg, V) : V;
+        if (tp_quads(e, lo, hi)) {
+#pragma unroll 4
+            for (int i = lo + 4 * t; i < hi; i += 4 * kSmT) {
+                float4 v = *(const float4*)(e + i);
+                v.x = v.x * inv, v.y = v.y * inv, v.z = v.z * inv, v.w = v.w * inv;
+                *(float4*)(e + i) = v;
+            }
+        } else {
+            for (int i = lo + t; i < hi; i += kSmT) e[i] = e[i] * inv;
+        }
     }
-    hipLaunchKernelGGL(tps_run_kernel, dim3(nseg, rows), dim3(kSmT), 0, st, probs, ld, V, rs);
-    hipLaunchKernelGGL(tps_walk_kernel, dim3(rows), dim3(64), 0, st, probs, ld, V, rs);
-    hipLaunchKernelGGL(tps_verify_kernel, dim3(nseg, rows), dim3(kSmT), 0, st, probs, ld, V, rs);
-    hipLaunchKernelGGL(tps_finish_kernel, dim3(rows), dim3(kSmT), 0, st, probs, ld, V, rs);
 }
 
 // p_j = e_j * (1 / S) (inference.rs:3535-3539), in place.
@@ -433,6 +462,21 @@ __global__ __launch_bounds__(kTpT) void tp_norm_kernel(float* probs, int64_t ld_
     float* e = probs + (size_t)row * ld_out;
     const int lo = min(c * tp_chunk(V), V), hi = min(lo + tp_chunk(V), V);
     for (int i = lo + t; i < hi; i += kTpT) e[i] = e[i] * inv;
+}
+
+// S and 1/S of every row, by the parallel segments when the row fits kTpSegMax of them; NORM: and the
+// row scaled by 1/S.
+template <bool NORM>
+static void launch_tp_sum(float* probs, int64_t ld, int rows, int V, float* rs, hipStream_t st) {
+    const int nseg = (V + kSmSeg - 1) / kSmSeg;
+    if (nseg > kTpSegMax) {
+        hipLaunchKernelGGL(tp_sum_kernel, dim3(rows), dim3(kSmT), 0, st, probs, ld, V, rs);
+        if (NORM) hipLaunchKernelGGL(tp_norm_kernel, dim3(kTpCh, rows), dim3(kTpT), 0, st, probs, ld, V, rs);
+        return;
+    }
+    hipLaunchKernelGGL(tps_run_kernel, dim3(nseg, rows), dim3(kSmT), 0, st, probs, ld, V, rs);
+    hipLaunchKernelGGL(tps_verify_kernel, dim3(nseg, rows), dim3(kSmT), 0, st, probs, ld, V, rs);
+    hipLaunchKernelGGL(tps_finish_kernel<NORM>, dim3(NORM ? nseg : 1, rows), dim3(kSmT), 0, st, probs, ld, V, rs);
 }
 
 // ---------------------------------------------------------------- the reference's sampler
@@ -458,7 +502,7 @@ __global__ __launch_bounds__(kSmT) void lcg_walk_kernel(const float* probs, int6
             const int i = base + t * kSmE + j;
             a[j] = i < V ? e[i] : 0.0f;  // zeros past the row leave the chain and its sign unchanged
         }
-        q = exact_chain_sum<kSmE, kSmT, true>(a, sc, a_lds, q);
+        q = exact_chain_sum<kSmE, kSmT, true, kSmMargin>(a, sc, a_lds, q);
         if (sc.first != 0x7fffffff) {  // uniform: read after the routine's last barrier
             found = base + sc.first;
             break;
@@ -743,7 +787,7 @@ int launch_sample_logits(const float* logits, int64_t ld_in, int rows, int V, fl
     const dim3 grid(kTpCh, rows);
     hipLaunchKernelGGL(tp_max_kernel, grid, dim3(kTpT), 0, st, logits, ld_in, V, rs);
     hipLaunchKernelGGL(tp_exp_kernel, grid, dim3(kTpT), 0, st, logits, ld_in, probs, ld_p, V, temp, rs);
-    launch_tp_sum(probs, ld_p, rows, V, rs, st);
+    launch_tp_sum<false>(probs, ld_p, rows, V, rs, st);
     hipLaunchKernelGGL(lcg_walk_kernel, dim3(rows), dim3(kSmT), 0, st, probs, ld_p, V, rs, uu, out);
     NC_HIP(hipGetLastError());
     return NC_OK;
@@ -757,8 +801,7 @@ int launch_temperature_probs(const float* logits, int64_t ld_in, float* probs, i
     const dim3 grid(kTpCh, rows);
     hipLaunchKernelGGL(tp_max_kernel, grid, dim3(kTpT), 0, st, logits, ld_in, V, rs);
     hipLaunchKernelGGL(tp_exp_kernel, grid, dim3(kTpT), 0, st, logits, ld_in, probs, ld_out, V, temp, rs);
-    launch_tp_sum(probs, ld_out, rows, V, rs, st);
-    hipLaunchKernelGGL(tp_norm_kernel, grid, dim3(kTpT), 0, st, probs, ld_out, V, rs);
+    launch_tp_sum<true>(probs, ld_out, rows, V, rs, st);
     NC_HIP(hipGetLastError());
     return NC_OK;
 }
