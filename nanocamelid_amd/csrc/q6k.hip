@@ -12,12 +12,13 @@
 // off the element loop.
 //
 // Bound: VALU issue.  At 128256 x 4096 and 5 tokens the 41 M (wave, element, token) steps take
-// two full-rate operations and one DPP one (2.3 + 2.3 + 4.2 cycles measured), 0.15 ms on 1024
-// SIMDs at 2.4 GHz against 0.07 ms for the 0.43 GB of weights.  Lane (q, r) of a wave holds super-block
+// two full-rate operations and one DPP one (11.2 cycles for the three in a loop of nothing else, at
+// any occupancy), 0.19 ms on 1024 SIMDs at 2.4 GHz, and unpacking the elements 0.03 ms, against 0.09 ms
+// for the 0.43 GB of weights.  Lane (q, r) of a wave holds super-block
 // 4 * quad + q of row r (a 16-row tile), so weights load as 1 KB per wave instruction, a
 // 16-lane DPP row shares one super-block's activations, and v_mul_f32_dpp row_newbcast reads
 // each value from the lane that converted it: no per-lane activation loads or conversions.
-// Measured, 128256 x 4096 at 5 tokens: 258 us, where one lane per super-block with its own activation
+// Measured, 128256 x 4096 at 5 tokens: 254 us, where one lane per super-block with its own activation
 // loads and conversions, on code for 8 tokens with a branch per token, took 1767 us.
 //
 // Device layout (repack_q6_k): rows padded to 16-row tiles, super-blocks to quads; per (tile, quad)
@@ -107,33 +108,26 @@ __global__ __launch_bounds__(64 * W) void gemm_q6_k_kernel(GemmParams p, int nb,
                     for (int j = 0; j < 4; j++) {
                         const int e = 4 * e4 + j;
                         const float qf[4] = {q6_byte(v[0], j), q6_byte(v[1], j), q6_byte(v[2], j), q6_byte(v[3], j)};
-                        // products first, then the DPP products, then the adds: a VGPR a VALU wrote may
-                        // be read with DPP two issue slots later, so mixing them costs waits
-                        float pr[4][NMAX];
-                        constexpr int KS = NMAX <= 4 ? 4 : 2;
+                        // two k at a time: products, then the DPP products, then the adds.  All four at
+                        // once hold 20 more registers and took 216 -> 254 us at 4 tokens; left to the
+                        // scheduler, which mixes the three, 5 tokens took 250 -> 297 us.
 #pragma unroll
-                        for (int k0 = 0; k0 < 4; k0 += KS) {
-#pragma unroll
-                            for (int k = k0; k < k0 + KS; k++)
-#pragma unroll
-                                for (int t = 0; t < NMAX; t++) pr[k][t] = c[t][k] * qf[k];
-                            __builtin_amdgcn_sched_barrier(0);
+                        for (int k = 0; k < 4; k += 2) {
+                            float pa[NMAX], pb[NMAX];
 #pragma unroll
                             for (int t = 0; t < NMAX; t++) {
-                                if (k0 == 0) {
-                                    pr[0][t] = q6_bcast<M>(xf[t][e]) * pr[0][t];
-                                    pr[1][t] = q6_bcast<4 + M>(xf[t][e]) * pr[1][t];
-                                }
-                                if (k0 + KS == 4) {
-                                    pr[2][t] = q6_bcast<8 + M>(xf[t][e]) * pr[2][t];
-                                    pr[3][t] = q6_bcast<12 + M>(xf[t][e]) * pr[3][t];
-                                }
+                                pa[t] = c[t][k] * qf[k];
+                                pb[t] = c[t][k + 1] * qf[k + 1];
                             }
                             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                            for (int k = k0; k < k0 + KS; k++)
+                            for (int t = 0; t < NMAX; t++) {
+                                pa[t] = (k ? q6_bcast<8 + M>(xf[t][e]) : q6_bcast<M>(xf[t][e])) * pa[t];
+                                pb[t] = (k ? q6_bcast<12 + M>(xf[t][e]) : q6_bcast<4 + M>(xf[t][e])) * pb[t];
+                            }
+                            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                                for (int t = 0; t < NMAX; t++) s[t] = s[t] + pr[k][t];
+                            for (int t = 0; t < NMAX; t++) s[t] = (s[t] + pa[t]) + pb[t];
                         }
                     }
                 }
@@ -202,10 +196,12 @@ int launch_gemm_q6k(const QMatDev& w, const GemmParams& p0, hipStream_t st) {
     p.ntiles = (int)w.tiles;
     const int groups = (p.N + 7) / 8, per = (p.N + groups - 1) / groups;
     if (w.tiles * groups > 0x7fffffff) return fail(NC_ERANGE, "Q6_K matmul: rows x batch too large");
-    // waves per workgroup: a power of two up to the quads of a row, until the launch has four waves
-    // per SIMD
+    // waves per workgroup: a power of two up to the quads of a row; four, so that a wave is a small part
+    // of a SIMD's work and the last ones end together (128256 x 4096, one wave a group -> four: 119 ->
+    // 98 us at 1 token, 32768 x 4096 at 5 tokens 82 -> 79 us), eight where the launch is short of four
+    // waves per SIMD
     int W = 1;
-    while (W < 8 && W < nquads && w.tiles * groups * W < 4096) W *= 2;
+    while (W < 8 && W < nquads && (W < 4 || w.tiles * groups * W < 4096)) W *= 2;
     const dim3 grid((unsigned)(w.tiles * groups));
     const size_t lds = (size_t)4 * nquads * per * 16 * sizeof(float);
 #define NC_Q6K(NM)                                                                                                 \
