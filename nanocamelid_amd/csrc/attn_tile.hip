@@ -1,6 +1,10 @@
 // Attention for passes with many (row, head) units (prompt passes, wide verify passes at long
 // contexts), in the reference's order (apply_attention_head, inference.rs:4142-4292): scores, softmax
-// and the weighted V sum as three kernels over tiles of 16 queries that share a KV head.
+// and the weighted V sum as three kernels over tiles of 16 queries that share a KV head.  The scores kernel
+// also serves every smaller pass whose rows outgrow the one-kernel attention: from one row on it is at
+// least as fast as a lane per position with the keys staged in LDS was (64 heads x 9 rows at 8180 positions
+// 55 -> 33 us, 32 x 16 at 8000 69 -> 26, 32 x 4 at 4000 14.6 -> 7.2, 64 x 1 at 2500 8.0 -> 5.9, head dim 64
+// 32 x 1 at 4000 5.2 -> 5.0).
 //
 //   scores: s_p = (((-0 + q_0 k_0) + q_1 k_1) + ...) * scale, dims in order (dot :3542-3558);
 //   softmax: max, e_p = expf(s_p - max), sum = e_0 + e_1 + ... left to right (:3522-3540);
@@ -278,14 +282,32 @@ __global__ __launch_bounds__(4 * HD, 4) void attn_tile_pv_kernel(AttnParams a, c
     }
 }
 
-int launch_attention_tiles(const AttnParams& a, hipStream_t st) {
+template <int PT>
+static void launch_scores(const AttnParams& a, hipStream_t st) {
     const int tiles = (a.H / a.Hkv * a.N + 15) / 16;
-    constexpr int PT = 4;
-    // position groups of the scores rounded up to 512 positions, so that one grid serves a captured
-    // pass at 512 consecutive positions (a workgroup past the rows ends at once)
-    const dim3 grid(a.Hkv * tiles), sgrid(a.Hkv * tiles, (a.max_pos + 512) / 512 * (512 / (64 * PT)));
-    if (a.hd == 128) NC_LAUNCH((attn_tile_scores_kernel<128, PT>), sgrid, dim3(256), 0, st, a);
-    else NC_LAUNCH((attn_tile_scores_kernel<64, PT>), sgrid, dim3(256), 0, st, a);
+    // position groups rounded up to 512 positions, so that one grid serves a captured pass at 512
+    // consecutive positions (a workgroup past the rows ends at once)
+    const dim3 grid(a.Hkv * tiles, (a.max_pos + 512) / 512 * (512 / (64 * PT)));
+    if (a.hd == 128) NC_LAUNCH((attn_tile_scores_kernel<128, PT>), grid, dim3(256), 0, st, a);
+    else NC_LAUNCH((attn_tile_scores_kernel<64, PT>), grid, dim3(256), 0, st, a);
+}
+
+// 64 PT positions a workgroup: more of them spread the loads of the queries and leave a tile's waves in
+// step, as long as the launch fills the chip.  8 KV heads, head dim 128, us at PT 1 / 2 / 4: 1280 groups at
+// PT 4 (72 queries a KV head, 8180 positions) 41.9 / 35.8 / 32.7; 512 groups at PT 2 (16 queries) 13.4 / 11.7;
+// 160 groups at PT 2 (8 queries, 2500 positions) 5.9 / 8.2.
+int launch_attention_scores(const AttnParams& a, hipStream_t st) {
+    const int64_t g1 = (int64_t)a.Hkv * ((a.H / a.Hkv * a.N + 15) / 16) * ((a.max_pos + 512) / 512 * 8);
+    if (g1 >= 4 * 1024) launch_scores<4>(a, st);
+    else if (g1 >= 2 * 512) launch_scores<2>(a, st);
+    else launch_scores<1>(a, st);
+    NC_HIP(hipGetLastError());
+    return NC_OK;
+}
+
+int launch_attention_tiles(const AttnParams& a, hipStream_t st) {
+    const dim3 grid(a.Hkv * ((a.H / a.Hkv * a.N + 15) / 16));
+    if (int rc = launch_attention_scores(a, st)) return rc;
     NC_LAUNCH(attn_tile_softmax_kernel, grid, dim3(64 * (kTileWaves + 1)), 0, st, a, a.inv);
     if (a.hd == 128) NC_LAUNCH((attn_tile_pv_kernel<128>), grid, dim3(512), 0, st, a, a.inv);
     else NC_LAUNCH((attn_tile_pv_kernel<64>), grid, dim3(256), 0, st, a, a.inv);

@@ -275,79 +275,7 @@ int launch_embed(const float* table, const uint32_t* toks, int N, int d, float* 
 }
 
 // ---------------------------------------------------------------- attention
-// Phase 1: scores[n][h][p] = dot(q[n][h], k[p]) * scale for p <= pos_n
-// (inference.rs:4252-4257; dot_f32_scalar folds a*b from -0.0 in index order).
-// Workgroup = one KV head x 64 positions: the K tile is staged once in LDS (rows padded
-// to HD+4 floats so the per-lane row reads are bank-conflict free) and shared by the
-// G query-head waves; lane = position p reads its key row from LDS (4 floats a step).
-// RB rows' dot chains are interleaved (each chain is sequential in i, the rows are
-// independent); their q vectors sit in LDS and are read as wave-wide broadcasts.
-template <int HD, int RB>
-__global__ __launch_bounds__(512) void attn_scores_kernel(AttnParams a) {
-    constexpr int RS = HD + 4;
-    __shared__ float kt[64 * RS];
-    __shared__ __align__(16) float qs[8][RB][HD];  // [head in group][row][dim]
-    const int kvh = blockIdx.x;  // KV head fastest: one XCD per KV head (see attn_fused_kernel)
-    const int G = a.H / a.Hkv;
-    const int g = wave_id_uniform();
-    const int h = kvh * G + g;
-    const int lane = threadIdx.x & 63;
-    const int pos0 = a.d_pos[0];
-    const int last = pos0 + a.N - 1;
-    for (int tile = blockIdx.y; tile * 64 <= last; tile += gridDim.y) {
-        __syncthreads();  // previous tile's readers are done with kt
-        if (tile * 64 > pos0 + min(a.N, ((int)blockIdx.z + 1) * RB) - 1) break;  // no row of this block reaches it
-        const int rows = min(64, last + 1 - tile * 64);
-        // keys are stored as dim quads [HD/4][max_ctx][4]: quad c of the tile's rows is
-        // 16 * rows contiguous bytes
-        const float4* src = (const float4*)a.kcache + (size_t)kvh * (HD / 4) * a.max_ctx + (size_t)tile * 64;
-        for (int i = threadIdx.x; i < rows * (HD / 4); i += blockDim.x) {
-            const int c = i / rows, r = i % rows;
-            *(float4*)&kt[r * RS + c * 4] = src[(size_t)c * a.max_ctx + r];
-        }
-        __syncthreads();
-        const int p = tile * 64 + lane;
-        const float* krow = &kt[lane * RS];  // this lane's key row (stale for p > last: unused)
-        // this block's rows: n = blockIdx.z*RB .. +RB-1 whose window reaches this tile
-        // (n >= tile*64 - pos0; uniform over the block)
-        const int n_first = max((int)blockIdx.z * RB, tile * 64 - pos0);
-        for (int n0 = n_first; n0 < min(a.N, ((int)blockIdx.z + 1) * RB); n0 += RB) {
-            // this wave's head: q rows n0 .. n0+RB-1 into LDS (each wave owns its slice)
-#pragma unroll
-            for (int r = 0; r < RB; r++) {
-                const int n = min(n0 + r, a.N - 1);
-                const float* qrow = a.q + (size_t)n * a.H * HD + (size_t)h * HD;
-                for (int i = lane; i < HD; i += 64) qs[g][r][i] = qrow[i];
-            }
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            float dot[RB];
-#pragma unroll
-            for (int r = 0; r < RB; r++) dot[r] = -0.0f;
-#pragma unroll 4
-            for (int i = 0; i < HD; i += 4) {
-                const float4 kv = *(const float4*)&krow[i];
-#pragma unroll
-                for (int r = 0; r < RB; r++) {
-                    const float4 qv = *(const float4*)&qs[g][r][i];
-                    dot[r] = dot[r] + qv.x * kv.x;
-                    dot[r] = dot[r] + qv.y * kv.y;
-                    dot[r] = dot[r] + qv.z * kv.z;
-                    dot[r] = dot[r] + qv.w * kv.w;
-                }
-            }
-#pragma unroll
-            for (int r = 0; r < RB; r++) {
-                const int n = n0 + r;
-                if (n < a.N && p <= pos0 + n) a.scores[((size_t)n * a.H + h) * a.max_ctx + p] = dot[r] * a.scale;
-            }
-            __builtin_amdgcn_wave_barrier();  // readers done before the next group overwrites qs
-        }
-    }
-}
-
-// Phase 2 (fused), one workgroup of T threads per (row n, head h) unit: softmax over
+// After the scores (launch_attention_scores), one workgroup of T threads per (row n, head h) unit: softmax over
 // 0..=pos (inference.rs:3522-3540) then the weighted V sum (add_weighted_f32_scalar,
 // inference.rs:3603-3623) and the Q8_0 quantisation of the output for the wo matmul.
 //   max: order free (block reduction); e_p = expf(s_p - max) in parallel;
@@ -566,7 +494,7 @@ __global__ __launch_bounds__(T) void attn_softmax_pv_kernel(AttnParams a) {
 }
 
 // Attention of one (row n, head h) unit in one kernel, for rows of at most T*E <= 1536
-// positions: the scores (as attn_scores_kernel: dot from -0.0 over the head dims in order,
+// positions: the scores (dot_f32_scalar, inference.rs:4252-4257: dot from -0.0 over the head dims in order,
 // then * scale) go to LDS, then the softmax and the weighted V sum as attn_softmax_pv_kernel.
 // Thread t scores positions t, t + T, ..., so a wave's key loads are consecutive positions:
 // keys are stored as dim quads [HD/4][max_ctx][4], one 16-byte load brings 4 dims of a
@@ -915,16 +843,20 @@ enum AttnTier {
 
 static int attention_tier(const AttnParams& a) {
     const int len = a.max_pos + 1;  // the longest score row of the pass
-    // Tiles of 16 queries once a pass has work for most of the chip: 1024 units at head dim 128 (32 rows x 32
-    // heads, one 8B layer at positions 0 / 3000 / 7500: 195 / 298 / 500 -> 179 / 295 / 475 us; 256 rows
-    // 596 / 1170 / 2509 -> 387 / 662 / 1108), 2048 at 64 (64 x 32: 159 / 228 / 412 -> 129 / 225 / 379).  Below,
-    // its 16-row workgroups leave CUs idle: 1536 units at head dim 64 144 / 211 / 326 -> 129 / 220 / 368, 512 at
-    // 128 (16 rows, 8000 positions) 202 -> 304 us for the attention alone.
-    if (a.inv && len <= 16384 && (int64_t)a.N * a.H * a.hd >= 1024 * 128) return AT_TILES;
-    if (len <= 1536) {
-        // one kernel per pass: each (row, head) unit scores its own keys (rows up to 1536
-        // positions: the units of a KV head, all on one XCD, re-read its keys from that XCD's
-        // L2, which costs less than a second launch and the scores' round trip through memory)
+    // Tiles of 16 queries for the softmax and V sum too once a pass has work for most of the chip.  us a layer
+    // at positions 0 / 1200 / 3000 / 7500, units -> tiles: head dim 128, 1536 units (48 rows x 32 heads, 8B)
+    // 227 / 256 / 333 / 528 -> 199 / 251 / 345 / 524, 8192 units 597 / 640 / 958 / 1837 -> 392 / 504 / 670 / 1119;
+    // head dim 64, 2048 units (64 x 32, 1B) 159 / 186 / 219 / 390 -> 129 / 168 / 228 / 380.  Below, the 16-row
+    // workgroups leave CUs idle: 1024 units at 128 192 / 214 / 269 / 423 -> 178 / 224 / 297 / 478, 1536 at 64
+    // 129 / 180 / 211 / 326 -> 129 / 190 / 220 / 368.
+    if (a.inv && len <= 16384 && a.N * a.H >= (a.hd == 64 ? 2048 : 1536)) return AT_TILES;
+    // one kernel per pass: each (row, head) unit scores its own keys (the units of a KV head, all on
+    // one XCD, re-read them from that XCD's L2), which saves a launch and the scores' round trip through
+    // memory, until the dots themselves cost more than that.  Attention of a layer in us, one kernel / tiled
+    // scores, then softmax and V: head dim 128, 32 heads x 5 rows at 705 positions 18 / 18, at 1105 24 /
+    // 21, at 1505 29 / 25, 1 row at 1401 29 / 23; more units than CUs (64 heads x 9 rows) at 709 35 / 26, at
+    // 1409 71 / 40; head dim 64, 32 heads x 1 row at 701 12 / 16, x 5 rows at 1405 19 / 21.
+    if (len <= (a.hd == 64 ? 1536 : a.N * a.H <= 256 ? 1024 : 512)) {
         // positions per thread E matched to the row (fewer score slots past the row); rows of
         // at most 512 and of 1281..1536 positions on 512 threads (two waves per SIMD in the
         // score phase; measured faster there, slower for 513..1280)
@@ -949,15 +881,14 @@ static int attention_tier(const AttnParams& a) {
     return len <= 2048 ? AT_PV_8_256 : len <= 4096 ? AT_PV_16_256 : AT_PV_32_256;
 }
 
-// Score-kernel workgroups along the positions: the row's 64-position tiles rounded up to a
-// multiple of 8 (the kernel strides over the tiles and a workgroup past the last tile does
-// nothing), so that one grid serves 512 consecutive positions.
-static int score_tile_groups(const AttnParams& a) { return ((a.max_pos + 64) / 64 + 7) / 8 * 8; }
+// 512-position steps of the score kernel's grid: one grid serves 512 consecutive positions (a workgroup
+// past the rows does nothing).
+static int score_steps(const AttnParams& a) { return (a.max_pos + 512) / 512; }
 
 int64_t attention_variant(const AttnParams& a) {
     if (a.split) return ((int64_t)1 << 40) | (a.max_pos / kSplitChunk + 1);
     const int tier = attention_tier(a);
-    return ((int64_t)tier << 24) | (tier >= AT_PV_32_256_X1 ? score_tile_groups(a) : 0);
+    return ((int64_t)tier << 24) | (tier >= AT_PV_32_256_X1 ? score_steps(a) : 0);
 }
 
 int launch_attention(const AttnParams& a, hipStream_t st) {
@@ -978,36 +909,16 @@ int launch_attention(const AttnParams& a, hipStream_t st) {
             case AT_FUSED_1_512: NC_FUSED(1, 512)
             case AT_FUSED_3_256: NC_FUSED(3, 256)
             case AT_FUSED_4_256: NC_FUSED(4, 256)
-            case AT_FUSED_5_256: NC_FUSED(5, 256)
-            default: NC_FUSED(3, 512)
+            case AT_FUSED_5_256: NC_LAUNCH((attn_fused_kernel<5, 256, 64>), grid, dim3(256), 0, st, a); break;
+            default: NC_LAUNCH((attn_fused_kernel<3, 512, 64>), grid, dim3(512), 0, st, a);
         }
 #undef NC_FUSED
         NC_HIP(hipGetLastError());
         return NC_OK;
     }
-    // longer rows: scores by (KV head, 64-position tile) blocks that share each key tile
-    // between the query heads and rows of a group, then one kernel for softmax and V sum
-    // rows per block: one or two interleaved dot chains per lane; row groups are spread over
-    // blockIdx.z so that every SIMD gets a short chain instead of a few SIMDs getting long ones
-    const int rb = a.N >= 2 ? 2 : 1;
-    const int tiles = score_tile_groups(a);
-#define NC_SCORES(HD, RB)                                                                         \
-    NC_LAUNCH((attn_scores_kernel<HD, RB>), dim3(a.Hkv, tiles, (a.N + (RB)-1) / (RB)), dim3(64 * G), 0, \
-                       st, a);                                                                    \
-    break;
-#define NC_SCORES_HD(HD)            \
-    switch (rb) {                   \
-        case 1: NC_SCORES(HD, 1)    \
-        default: NC_SCORES(HD, 2)   \
-    }
-    if (a.hd == 128) {
-        NC_SCORES_HD(128)
-    } else {
-        NC_SCORES_HD(64)
-    }
-#undef NC_SCORES_HD
-#undef NC_SCORES
-    NC_HIP(hipGetLastError());
+    // longer rows: scores by tiles of 16 queries of a KV head, then one kernel per unit for softmax
+    // and V sum
+    if (int rc = launch_attention_scores(a, st)) return rc;
 #define NC_PV(E, T, PIPE, X)                                                                              \
     if (a.hd == 128) NC_LAUNCH((attn_softmax_pv_kernel<E, T, 128, PIPE, X>), grid, dim3(T), 0, st, a); \
     else NC_LAUNCH((attn_softmax_pv_kernel<E, T, 64, PIPE, X>), grid, dim3(T), 0, st, a);              \

@@ -190,6 +190,7 @@ struct AttnParams {
 int launch_attention(const AttnParams& a, hipStream_t stream);
 // The same outputs by tiles of 16 queries (attn_tile.hip), for passes with many (row, head) units.
 int launch_attention_tiles(const AttnParams& a, hipStream_t stream);
+int launch_attention_scores(const AttnParams& a, hipStream_t stream);  // a pass's scores, any number of units
 // Launch variant of launch_attention: passes with equal values launch the same kernels with the
 // same grids and blocks (the kernels read the rows' positions from d_pos, not from max_pos), so
 // a captured pass replays correctly at every start position of its variant.

@@ -35,3 +35,34 @@ def test_tiled_attention_vs_oracle(H, Hkv, hd, chunks):
     assert np.array_equal(preds, opreds)
     for i in range(5):
         assert np.array_equal(gs.logits(i).view(np.uint32), ologits[i].view(np.uint32)), i
+
+
+# rows just past the one-kernel attention (512, 1024 or 1536 positions by head dim and units) and the scores'
+# grid steps of 64, 128 and 256 positions a workgroup: one and eight heads per KV head, tiles of one, of 15 and of
+# 16 queries, the last prefill row a pass of 49 rows
+@pytest.mark.parametrize("H,Hkv,hd,start,rows", [(8, 1, 128, 1023, [1, 2, 3]), (8, 8, 128, 1021, [5, 16]),
+                                                 (8, 4, 64, 1533, [3, 8]), (32, 4, 128, 505, [9, 8, 1]),
+                                                 (32, 32, 64, 1535, [1, 2]), (32, 32, 64, 1537, [49, 3])])
+def test_tile_scores_vs_oracle(H, Hkv, hd, start, rows):
+    ctx = nc.Context(0)
+    img = nc.synth_gguf(layers=2, embedding_length=H * hd, head_count=H, head_count_kv=Hkv, feed_forward_length=256,
+                        vocab_size=300, context_length=2048, tied=1, norm_mode=1, seed=H + Hkv + hd + start)
+    end = start + sum(rows)
+    gs = nc.Session(nc.Model(ctx, data=img), end + 16, 16)
+    os_ = O.Session(O.Model(data=img.tobytes(), nthreads=8), end + 16, 16)
+    gs.fill_kv(end, 9)
+    os_.fill_kv(end, 9)
+    pos = start
+    for n in rows:
+        toks = nc.uniform_prompt(pos + n, n, 300)
+        if n > 16:
+            gs.prefill_pass_batch(toks, pos, want_logits=False)
+            for i in range(0, n, 16):
+                os_.prefill_pass_batch(toks[i:i + 16], pos + i)
+        else:
+            _, _, _, preds = gs.verify_greedy(toks, pos)
+            opreds, _, ologits = os_.verify_greedy(toks, pos, want_logits=True)
+            assert np.array_equal(preds, opreds)
+            for i in range(n):
+                assert np.array_equal(gs.logits(i).view(np.uint32), ologits[i].view(np.uint32)), (pos, i)
+        pos += n
