@@ -1590,7 +1590,8 @@ int nc_bench_matmul(nc_ctx* ctx, const nc_qmat* const* w, int32_t ncopies, const
     for (int i = 0; i < ncopies; i++)
         if (!w[i] || w[i]->m.rows != w[0]->m.rows || w[i]->m.cols != w[0]->m.cols)
             return fail(NC_EINVAL, "nc_bench_matmul: weight copies differ in shape");
-    if (batch_size > 16 && (!prompt_matrix_ok(w[0]->m) || prompt_slice_tokens(w[0]->m.cols) < 16))
+    if (batch_size > 16 && ((w[0]->m.type != NC_TYPE_Q4_0 && w[0]->m.type != NC_TYPE_Q4_K) ||
+                            !prompt_matrix_ok(w[0]->m) || prompt_slice_tokens(w[0]->m.cols) < 16))
         return fail(NC_EINVAL, "nc_bench_matmul: more than 16 tokens only for Q4_0 / Q4_K matrices of <= 1M columns");
     NC_HIP(hipSetDevice(ctx->device));
     hipStream_t st = ctx->stream;
