@@ -111,9 +111,8 @@ int nc_ctx_set_pass_launch(nc_ctx* ctx, int mode);
  * construction load_q4_0_matrix / decode_q4_k_blocks (src/model.rs:1369-1401,
  * src/model.rs:1270) that feeds QuantizedMatrix (src/model.rs:294-310).
  * type: NC_TYPE_Q4_0, NC_TYPE_Q4_K, NC_TYPE_Q5_K (matmul_q5_k_batch src/inference.rs:2513-2640),
- * NC_TYPE_Q8_0 (matmul_q8_0_batch src/inference.rs:1343-1383; both batches of 1..16 tokens, more
- * in 16-token slices) or NC_TYPE_Q6_K (the Q6_K output projection
- * of llama.cpp files, matmul_q6_k_batch src/inference.rs:1882-2000; batches of 1..16 tokens).
+ * NC_TYPE_Q8_0 (matmul_q8_0_batch src/inference.rs:1343-1383) or NC_TYPE_Q6_K (the Q6_K output
+ * projection of llama.cpp files, matmul_q6_k_batch src/inference.rs:1882-2000).
  * cols % 32 == 0 (Q4_K, Q5_K, Q6_K: % 256; Q6_K: cols <= 16384). */
 int nc_qmat_upload(nc_ctx* ctx, int type, int64_t rows, int64_t cols, const void* gguf_blocks_host,
                    nc_qmat** out);
@@ -128,9 +127,10 @@ int64_t nc_qmat_device_bytes(const nc_qmat* w);
  * x_i8 [batch][cols] int8, x_scales [batch][cols/32] f32, out [batch][rows] f32
  * (token-major, as write_batch_out src/inference.rs:1333-1341).  batch_size >= 1, no upper
  * limit (matmul_quantized_batch takes any batch): up to 16 tokens run on the verify kernels;
- * more run on the int8 MFMA prompt matmul (Q4_0; slices of up to 256 tokens through buffers
- * that nc_ctx_create allocates, 18 MiB) or as 16-token slices (Q4_K, Q6_K).  Calls that share
- * a context and overlap on different streams race on those buffers.
+ * more run on the f16 MFMA prompt matmul (every type but Q6_K; slices of up to 256 tokens through
+ * buffers that nc_ctx_create allocates, 36 MiB; Q5_K and Q8_0 matrices of 2 GiB or more as 16-token
+ * slices), or for Q6_K on the verify kernel in groups of up to 8 tokens.  Calls that share a
+ * context and overlap on different streams race on those buffers.
  * stream: a hipStream_t or NULL for the context's default stream. */
 int nc_matmul_quantized_batch(nc_ctx* ctx, const nc_qmat* w, const int8_t* x_i8, const float* x_scales,
                               float* out, int batch_size, int64_t rows, int64_t cols, void* stream);

@@ -1225,9 +1225,8 @@ static int ensure_prompt_bufs(nc_session* s) {
     return NC_OK;
 }
 
-// Prompt matmul of the pass's activations (repacked first into MFMA operand order).
 // A prompt pass's matmul into rows of stride ld (default: the matrix's rows): the MFMA prompt
-// kernels, or for Q6_K matrices (no prompt kernel) the verify kernel.
+// kernels (activations repacked into operand order first), or for Q6_K matrices (no prompt kernel) the verify kernel.
 static int prompt_gemm(nc_session* s, const QMatDev& w, const int8_t* xq, const float* xs, float* out, int n,
                        int ld = 0) {
     if (ld == 0) ld = (int)w.rows;
@@ -1326,8 +1325,8 @@ static int run_prompt_pass(nc_session* s, int off, int n, int64_t start) {
 }
 
 // prefill_tokens (main.rs:9415-9485): chunks of max_batch rows.  Returns the last row's
-// greedy prediction in *last_pred.  Q4_0 models run all but the last max_batch tokens (all of
-// them when no logits are wanted) as prompt passes of up to kPromptRows tokens; every token's
+// greedy prediction in *last_pred.  All but the last max_batch tokens (all of
+// them when no logits are wanted) run as prompt passes of up to kPromptRows tokens; every token's
 // arithmetic is the same in any chunking, so the KV cache and logits are the same bits.
 static int prefill_chunks(nc_session* s, const uint32_t* toks, int n, int64_t start_pos, uint32_t* last_pred,
                           bool last_logits = false) {
@@ -1557,7 +1556,7 @@ int nc_matmul_quantized_batch(nc_ctx* ctx, const nc_qmat* w, const int8_t* x_i8,
     if (batch_size < 1) return fail(NC_EINVAL, "nc_matmul_quantized_batch: batch must be >= 1");
     NC_HIP(hipSetDevice(ctx->device));
     hipStream_t st = stream ? (hipStream_t)stream : ctx->stream;
-    // more than 16 tokens: the MFMA prompt matmul (Q4_0), or 16-token slices (Q4_K)
+    // more than 16 tokens: the MFMA prompt matmul (every type but Q6_K)
     if (batch_size > 16 && prompt_matrix_ok(w->m) && prompt_slice_tokens(cols) >= 16)
         return ctx_prompt_matmul(ctx, w->m, x_i8, x_scales, out, batch_size, st);
     const int slice = slice_tokens(w->m, batch_size);
