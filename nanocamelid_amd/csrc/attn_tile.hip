@@ -22,6 +22,7 @@
 // sum 53 us at the last ones; the attention of the whole prompt 6.8 -> 2.3 ms a layer pair.
 #include "nc_internal.h"
 #include "nc_device.h"
+#include "nc_offsets.h"
 
 namespace nc {
 
@@ -53,7 +54,8 @@ __device__ __forceinline__ void tile_add16(t_v4f& acc, const t_v16f (&d)[4]) {
 
 // Scores.  Workgroup = one query tile x 64 * PT positions; wave w takes the 16-position tiles w, w + 4, ...
 // MFMA operands of dims 16 I + 4 j + e: A lane (j, r) = query r, B lane (j, c) = position c (key dim quads
-// [hd/4][ctx][4]), so register e of one 16-byte load each.  The wave's queries stay in registers.
+// [hd/4][ctx][4]), so register e of one 16-byte load each.  The wave's queries stay in registers.  A tile that holds
+// a position of the pass lies inside the cache (max_ctx is a multiple of 16), so no load is out of range.
 template <int HD, int PT>
 __global__ __launch_bounds__(256, 3) void attn_tile_scores_kernel(AttnParams a) {
     constexpr int NI = HD / 16;
@@ -184,7 +186,8 @@ __global__ __launch_bounds__(64 * (kTileWaves + 1)) void attn_tile_softmax_kerne
 
 // Weighted V sum and the Q8_0 quantisation of the output.  Workgroup = one query tile, wave w = output
 // dims 16w..16w+15.  MFMA operands of positions 16 P + 4 j + e: A lane (j, r) = prob of query r, B lane (j, c) =
-// value dim c (value position quads [ctx/4][hd][4]).  A ring of 4 steps of loads is in flight.
+// value dim c (value position quads [ctx/4][hd][4]).  A ring of 4 steps of loads is in flight; a step past the cache
+// loads its last one (max_ctx is a multiple of 16) and is not added.
 template <int HD>
 __global__ __launch_bounds__(4 * HD, 4) void attn_tile_pv_kernel(AttnParams a, const float* inv) {
     __shared__ __align__(16) float out[16][HD + 4];
@@ -205,13 +208,14 @@ __global__ __launch_bounds__(4 * HD, 4) void attn_tile_pv_kernel(AttnParams a, c
     const __amdgpu_buffer_rsrc_t vres = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(a.vcache + (size_t)kvh * a.max_ctx * HD), 0, a.max_ctx * HD * 4, 0x00020000);
     const int vvo = (j * HD + 16 * w + r) * 16;
-    const int steps = (longest + 15) / 16, pmax = (a.max_ctx - 4 - 4 * j) / 16;  // last step whose quad is in the row
+    const int steps = (longest + 15) / 16;
     constexpr int D = 4;
     t_v4f rp[D], rv[D];
 #define NC_TILE_LOAD(S, SLOT)                                                                                  \
     {                                                                                                          \
-        rp[SLOT] = *(const t_v4f*)(prow + 16 * min((S), pmax));                                                \
-        rv[SLOT] = __builtin_bit_cast(t_v4f, __builtin_amdgcn_raw_buffer_load_b128(vres, vvo, (S) * HD * 64, 0)); \
+        const int s_ = kv_step((S), a.max_ctx);                                                                \
+        rp[SLOT] = *(const t_v4f*)(prow + 16 * s_);                                                            \
+        rv[SLOT] = __builtin_bit_cast(t_v4f, __builtin_amdgcn_raw_buffer_load_b128(vres, vvo, s_ * HD * 64, 0)); \
     }
 #pragma unroll
     for (int k = 0; k < D - 1; k++) NC_TILE_LOAD(k, k)
@@ -297,6 +301,8 @@ static void launch_scores(const AttnParams& a, hipStream_t st) {
 // PT 4 (72 queries a KV head, 8180 positions) 41.9 / 35.8 / 32.7; 512 groups at PT 2 (16 queries) 13.4 / 11.7;
 // 160 groups at PT 2 (8 queries, 2500 positions) 5.9 / 8.2.
 int launch_attention_scores(const AttnParams& a, hipStream_t st) {
+    if (a.max_ctx % 16 || a.max_pos >= a.max_ctx)
+        return fail(NC_EINVAL, "attention: cache rows must be whole 16-position tiles that hold the pass");
     const int64_t g1 = (int64_t)a.Hkv * ((a.H / a.Hkv * a.N + 15) / 16) * ((a.max_pos + 512) / 512 * 8);
     if (g1 >= 4 * 1024) launch_scores<4>(a, st);
     else if (g1 >= 2 * 512) launch_scores<2>(a, st);

@@ -20,6 +20,7 @@
 // (g, c) = token c, rows 4g..4g+3.
 #include "nc_internal.h"
 #include "nc_device.h"
+#include "nc_offsets.h"
 
 namespace nc {
 
@@ -68,8 +69,8 @@ __device__ __forceinline__ p_h8 unpack_q80(uint32_t w0, uint32_t w1, uint32_t on
 // Workgroup = 4 waves x (16 rows x 16 KT tokens): the waves take consecutive row tiles of the same
 // tokens, whose activation units go through LDS (double-buffered stages of one quad of blocks, loaded
 // SD stages ahead into registers), so each is fetched once per workgroup; weights come straight from
-// memory, WD - 1 stages ahead.  Loads past a buffer's end return 0 and stages past the row are never
-// added, so no index is clamped.  blockIdx.x = token group + row group * token groups.
+// memory, WD - 1 stages ahead.  Token tiles and stages past the last one load the last one's (nc_offsets.h) and
+// are never stored or added.  blockIdx.x = token group + row group * token groups.
 template <int LAYOUT, int KT, int WD, int SD>
 __global__ __launch_bounds__(256, 4) void gemm_b32_prompt_kernel(PromptGemm p, int tgroups) {
     constexpr bool Q8 = LAYOUT == LAYOUT_Q80;
@@ -98,23 +99,26 @@ __global__ __launch_bounds__(256, 4) void gemm_b32_prompt_kernel(PromptGemm p, i
     }
     // this wave's share of a stage's units: token tile wv % KT, blocks wv / KT, + 4 / KT, ...
     const int uk = wv % KT, uj = wv / KT;
-    const int ubase = (tt + uk) * nq * 4096 + uj * 1024;
     uint32_t wd[WD][4][NW], sw[WD];
     float xsr[WD][KT];
     uint4 st[SD][KT];
 #define NC_PB_UNITS(S, SLOT)                                                                                       \
-    _Pragma("unroll") for (int u = 0; u < KT; u++) st[SLOT][u] = __builtin_bit_cast(                               \
-        uint4, __builtin_amdgcn_raw_buffer_load_b128(xres, lane * 16 + u * (4 / KT) * 1024, ubase + (S) * 4096, 0));
+    {                                                                                                              \
+        const int uo_ = prompt_unit(tt + uk, (S), n16, nq) * 4096 + uj * 1024;                                     \
+        _Pragma("unroll") for (int u = 0; u < KT; u++) st[SLOT][u] = __builtin_bit_cast(                           \
+            uint4, __builtin_amdgcn_raw_buffer_load_b128(xres, lane * 16 + u * (4 / KT) * 1024, uo_, 0));          \
+    }
 #define NC_PB_WEIGHTS(S, SLOT)                                                                                     \
     {                                                                                                              \
-        const int h_ = LAYOUT == LAYOUT_R64 ? ((S) & 1) : 0;                                                       \
-        const int qo_ = LAYOUT == LAYOUT_R64 ? ((S) >> 1) * kQ40ChunkBytes : (S) * r16_quad_bytes(Q8);             \
+        const int h_ = LAYOUT == LAYOUT_R64 ? prompt_r64_half((S), nq) : 0;                                        \
+        const int qo_ = LAYOUT == LAYOUT_R64 ? prompt_r64_chunk((S), nq, kQ40ChunkBytes)                           \
+                                             : prompt_r16_quad((S), nq, r16_quad_bytes(Q8));                       \
         _Pragma("unroll") for (int j = 0; j < 4; j++) _Pragma("unroll") for (int x = 0; x < NW; x++)               \
             wd[SLOT][j][x] = __builtin_amdgcn_raw_buffer_load_b32(                                                 \
                 wres, nvo + (LAYOUT == LAYOUT_R64 ? 1024 : 256) * j + 1024 * x, qo_ + 4096 * h_, 0);               \
         sw[SLOT] = __builtin_amdgcn_raw_buffer_load_b16(wres, svo, qo_ + 512 * h_, 0);                             \
         _Pragma("unroll") for (int k = 0; k < KT; k++) xsr[SLOT][k] = __builtin_bit_cast(                          \
-            float, __builtin_amdgcn_raw_buffer_load_b32(sres, lane * 4, ((tt + k) * nq + (S)) * 256, 0));          \
+            float, __builtin_amdgcn_raw_buffer_load_b32(sres, lane * 4, prompt_unit(tt + k, (S), n16, nq) * 256, 0)); \
     }
     uint32_t one = 0x64006400u;  // two f16 1024
     asm("" : "+v"(one));
@@ -290,24 +294,23 @@ __global__ __launch_bounds__(256, KT == 4 ? 3 : 4) void gemm_k_prompt_kernel(Pro
         (void*)(p.w + (size_t)(LAYOUT == LAYOUT_R16K ? ts : ts >> 2) * tile_bytes), 0, tile_bytes, 0x00020000);
     const int hvo = LAYOUT == LAYOUT_R16K ? r * 16 : (16 * (ts & 3) + r) * 16, nvo = hvo + 4 * g;
     const int uk = wv % KT, uj = wv / KT;  // this wave's share of a stage's units
-    const int ubase = (tt + uk) * nq * 4096 + uj * 1024;
     uint32_t wd[WD][2][2], hdn[6];
     float xar[WD][KT], xst[SD];
     uint4 st[SD][KT];
 #define NC_PK_UNITS(S, SLOT)                                                                                       \
     {                                                                                                              \
+        const int un_ = prompt_unit(tt + uk, (S), n16, nq);                                                        \
         _Pragma("unroll") for (int u = 0; u < KT; u++) st[SLOT][u] = __builtin_bit_cast(                           \
-            uint4, __builtin_amdgcn_raw_buffer_load_b128(xres, lane * 16 + u * (4 / KT) * 1024, ubase + (S) * 4096, 0)); \
+            uint4, __builtin_amdgcn_raw_buffer_load_b128(xres, lane * 16 + u * (4 / KT) * 1024, un_ * 4096 + uj * 1024, 0)); \
         xst[SLOT] = __builtin_bit_cast(                                                                            \
-            float, __builtin_amdgcn_raw_buffer_load_b32(sres, lane * 4, ((tt + uk) * nq + (S)) * 256, 0));         \
+            float, __builtin_amdgcn_raw_buffer_load_b32(sres, lane * 4, un_ * 256, 0));                            \
     }
 #define NC_PK_WEIGHTS(S, SLOT, HEAD)                                                                               \
     {                                                                                                              \
-        const int sb_ = (S) >> 1;                                                                                  \
-        const int co_ = LAYOUT == LAYOUT_R16K ? (sb_ >> 2) * CHUNK + 256 * (sb_ & 3) : sb_ * CHUNK;                \
+        const int co_ = prompt_k_chunk(LAYOUT == LAYOUT_R16K, (S), nq, CHUNK);                                     \
         _Pragma("unroll") for (int pp = 0; pp < 2; pp++) _Pragma("unroll") for (int x = 0; x < 2; x++)             \
             wd[SLOT][pp][x] = __builtin_amdgcn_raw_buffer_load_b32(                                                \
-                wres, nvo + 1024 * (2 * pp + x), co_ + (QS + 4 * ((S) & 1)) * 1024, 0);                            \
+                wres, nvo + 1024 * (2 * pp + x), co_ + (QS + 4 * prompt_k_half((S), nq)) * 1024, 0);                            \
         if (HEAD) {                                                                                                \
             const uint4 h_ = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(wres, hvo, co_, 0));  \
             hdn[0] = h_.x, hdn[1] = h_.y, hdn[2] = h_.z, hdn[3] = h_.w;                                            \
@@ -317,7 +320,7 @@ __global__ __launch_bounds__(256, KT == 4 ? 3 : 4) void gemm_k_prompt_kernel(Pro
             }                                                                                                      \
         }                                                                                                          \
         _Pragma("unroll") for (int k = 0; k < KT; k++) xar[SLOT][k] = __builtin_bit_cast(                          \
-            float, __builtin_amdgcn_raw_buffer_load_b32(ares, lane * 4, ((tt + k) * nq + (S)) * 256, 0));          \
+            float, __builtin_amdgcn_raw_buffer_load_b32(ares, lane * 4, prompt_unit(tt + k, (S), n16, nq) * 256, 0)); \
     }
     uint32_t one = 0x64006400u;  // two f16 1024
     asm("" : "+v"(one));

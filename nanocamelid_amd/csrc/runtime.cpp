@@ -12,6 +12,7 @@
 
 #include "gguf.h"
 #include "nc_internal.h"
+#include "nc_offsets.h"
 
 #include <cerrno>
 #include <fcntl.h>
@@ -58,7 +59,7 @@ struct nc_session {
     nc_ctx* ctx = nullptr;
     hipStream_t stream = nullptr;
     int64_t max_ctx = 0;
-    int64_t ctx_stride = 0;  // max_ctx rounded up to 4: KV rows, V position quads, score rows
+    int64_t ctx_stride = 0;  // kv_positions(max_ctx): KV rows, V position quads, score rows
     int max_batch = 0;
     int64_t maxw = 0;
     float *kcache = nullptr, *vcache = nullptr;  // K [L][Hkv][hd/4][ctx_stride][4], V [L][Hkv][ctx_stride/4][hd][4]
@@ -1827,7 +1828,7 @@ int nc_session_create(nc_model* m, int64_t max_ctx, int32_t max_batch, nc_sessio
     s->m = m;
     s->ctx = m->ctx;
     s->max_ctx = max_ctx;
-    s->ctx_stride = (max_ctx + 3) / 4 * 4;
+    s->ctx_stride = kv_positions(max_ctx);
     s->attn_chunks = (int)((max_ctx + 63) / 64);  // 64-position chunks of the split-order attention
     s->max_batch = max_batch;
     NC_HIP(hipStreamCreate(&s->stream));
