@@ -1,6 +1,6 @@
-// Scalar (wave-uniform) parts of buffer-load offsets that run ahead of what is used, as functions that
-// the kernels and a host check of their ranges share.
+// Offsets and launch limits that the kernels, their launches and a host check of their ranges share.
 //
+// Scalar (wave-uniform) parts of buffer-load offsets that run ahead of what is used.
 // The range check of a raw buffer load is documented for the per-lane offset; the scalar one is not part of
 // it on every reading of the rule, so no load here relies on it: a prefetched stage or step past the last
 // one, or a token tile past the last one, takes the last one's place.  What it brings is never used.
@@ -37,5 +37,14 @@ NC_HD constexpr int prompt_k_half(int stage, int nq) { return clamp_last(stage, 
 NC_HD constexpr long long kv_positions(long long max_ctx) { return (max_ctx + 15) / 16 * 16; }
 // The 16-position step of a value or probability load, of ctx = kv_positions(...) positions.
 NC_HD constexpr int kv_step(int step, int ctx) { return clamp_last(step, ctx / 16); }
+
+// The Q6_K kernel's launches: a workgroup per 16-row tile and group of at most 8 tokens, of at most 512
+// threads, where a grid holds fewer than 2^32 threads along x.  The most tokens of one launch; a batch
+// beyond them (2^29 outputs at least) takes several.
+constexpr int kQ6KTokens = 8, kQ6KThreads = 512;
+NC_HD constexpr long long q6k_launch_tokens(long long tiles) {
+    const long long groups = 0xffffffffLL / (kQ6KThreads * tiles);
+    return kQ6KTokens * (groups < 1 ? 1 : groups);
+}
 
 }  // namespace nc

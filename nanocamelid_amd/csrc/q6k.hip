@@ -25,6 +25,7 @@
 // 13 slots of [64 lanes x 16 B] (ql 8, qh 4, scales 1), then [64 lanes] f16 d.
 #include "nc_internal.h"
 #include "nc_device.h"
+#include "nc_offsets.h"
 
 namespace nc {
 
@@ -183,7 +184,7 @@ int64_t q6k_layout_bytes(int64_t rows, int64_t cols) {
     return (rows + 15) / 16 * ((cols / 256 + 3) / 4) * kQ6KQuadBytes;
 }
 
-// Any number of tokens: groups of at most 8 (the registers of one wave), as even as they come.
+// Up to q6k_launch_tokens tokens: groups of at most 8 (the registers of one wave), as even as they come.
 int launch_gemm_q6k(const QMatDev& w, const GemmParams& p0, hipStream_t st) {
     GemmParams p = p0;
     const int nb = (int)(w.cols / 256), nquads = (nb + 3) / 4;
@@ -194,8 +195,8 @@ int launch_gemm_q6k(const QMatDev& w, const GemmParams& p0, hipStream_t st) {
     p.M = (int)w.rows;
     p.K = (int)w.cols;
     p.ntiles = (int)w.tiles;
-    const int groups = (p.N + 7) / 8, per = (p.N + groups - 1) / groups;
-    if (w.tiles * groups > 0x7fffffff) return fail(NC_ERANGE, "Q6_K matmul: rows x batch too large");
+    const int groups = (p.N + kQ6KTokens - 1) / kQ6KTokens, per = (p.N + groups - 1) / groups;
+    if (p.N > q6k_launch_tokens(w.tiles)) return fail(NC_ERANGE, "Q6_K matmul: rows x batch too large for one launch");
     // waves per workgroup: a power of two up to the quads of a row; four, so that a wave is a small part
     // of a SIMD's work and the last ones end together (128256 x 4096, one wave a group -> four: 119 ->
     // 98 us at 1 token, 32768 x 4096 at 5 tokens 82 -> 79 us), eight where the launch is short of four

@@ -1170,9 +1170,11 @@ static bool prompt_matrix_ok(const QMatDev& q) {
     return false;
 }
 
-// Tokens per launch of a matrix without a prompt kernel: the Q6_K kernel takes any number (its token
-// groups share a launch), the others 16.
-static int slice_tokens(const QMatDev& q, int n) { return q.type == NC_TYPE_Q6_K ? n : 16; }
+// Tokens per launch of a matrix without a prompt kernel: the Q6_K kernel takes as many as one grid holds
+// (its token groups share a launch), the others 16.
+static int slice_tokens(const QMatDev& q, int n) {
+    return q.type == NC_TYPE_Q6_K ? (int)std::min<int64_t>(n, q6k_launch_tokens(q.tiles)) : 16;
+}
 
 // Whether the verify kernels of a matrix read the activations' block sums: for the mins of Q4_K and
 // Q5_K, and for the offset of the unsigned Q4_0 nibbles on the int8 MFMA path.

@@ -1,7 +1,7 @@
 """Every buffer load of the prompt matmuls and the tiled attention lies inside its buffer, whatever the
 range check of a raw buffer load covers: the offsets (nc_offsets.h, the functions the kernels use) are
 walked on the host in the kernels' loop order, prefetched stages and token tiles past the last ones
-included, and compared with the bytes the host allocates.
+included, and compared with the bytes the host allocates.  The slices of a large Q6_K batch fit a grid.
 """
 import os
 import subprocess
@@ -71,7 +71,17 @@ static void attention(int max_ctx, int hd) {
         }
 }
 
+// rows x tokens in launches of q6k_launch_tokens: every grid below 2^32 threads, no more launches than needed
+static void q6k(long long rows, long long tokens) {
+    const long long tiles = (rows + 15) / 16, most = q6k_launch_tokens(tiles);
+    const long long n = tokens < most ? tokens : most;
+    inside("Q6_K grid", 0, tiles * ((n + 7) / 8) * 512, 0xffffffffLL, (int)rows, (int)tokens);
+    inside("outputs of the smallest first launch", 0, 1LL << 29, 16 * tiles * most, (int)rows, (int)tokens);
+}
+
 int main() {
+    for (long long rows : {1, 17, 4096, 32000, 128256, 256000})
+        for (long long tokens : {1, 16, 255, 8368, 16400, 1 << 20, 1 << 28}) q6k(rows, tokens);
     for (int n : {1, 2, 15, 16, 17, 31, 33, 48, 49, 64, 65, 113, 250, 256})
         for (int nb = 1; nb <= 200; nb += nb < 40 ? 1 : 7) {
             for (int KT : {1, 2, 4}) prompt(n, nb, KT, 2, KT == 1 ? 2 : 1, false);

@@ -39,6 +39,25 @@ def test_q6_k_tile_edges(ctx, M, K):
     check(ctx, nc._ffi.NC_TYPE_Q6_K, w, O.matmul_q6_k, M, K, [1, 2, 3, 4, 5, 6, 7, 8, 9, 16, 17, 50], 3)
 
 
+# more workgroups than one grid of 256-thread workgroups holds: the batch takes several launches, and its first
+# and last rows and those around their boundary are what the same rows give in a small batch
+def test_q6_k_batch_past_one_grid(ctx):
+    import torch
+    M, K, N = 131072, 2304, 16400
+    if torch.cuda.mem_get_info()[0] < 24 << 30:
+        pytest.skip("needs 24 GB of free device memory")
+    w = np.tile(GW.q6_k_weights(1024 * K // 256, seed=11).reshape(1024, K // 256, 210), (M // 1024, 1, 1))
+    qm = nc.QMat(ctx, nc._ffi.NC_TYPE_Q6_K, M, K, w)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x = torch.randint(-127, 128, (N, K), dtype=torch.int8, device="cuda", generator=g)
+    s = torch.rand(N, K // 32, device="cuda", generator=g)
+    out = nc.matmul_quantized_batch(ctx, qm, x, s)
+    for lo in (0, 8176, 8184, 8192, N // 2, N - 9):
+        some = nc.matmul_quantized_batch(ctx, qm, x[lo:lo + 9], s[lo:lo + 9])
+        assert torch.equal(out[lo:lo + 9].view(torch.int32), some.view(torch.int32)), lo
+    qm.close()
+
+
 # K: one block, a cut quad, a whole one, a cut chunk of 8 quads, 12 term waves (>= 64 quads); N: every width
 # the kernel is built for, both widths with their chains on term waves (9, 16) and a cut 16-token slice
 @pytest.mark.parametrize("M,K", [(1, 32), (17, 96), (100, 1024), (64, 1120), (33, 8224), (1040, 64)])
