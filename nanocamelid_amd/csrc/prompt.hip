@@ -241,6 +241,11 @@ int launch_gemm_prompt(const QMatDev& w, float* out, int ld_out, int N, hipStrea
 // q8.rs:1551-1594), with W_j = sum q * x (unsigned values) and A_j = sum x of the sub-block; that
 // super-block sum is added to the row's sum.  W_j arrives as an exact f32 from f16 MFMA, mn_j * A_j from a
 // one-term f32 MFMA, as in the kernel above; four VALU operations per output and sub-block remain.
+// The values q are unsigned and below 2^10, so their bits alone are the f16 subnormal q * 2^-24, which the matrix
+// core multiplies exactly: unpacking is a shift and a mask, W_j comes times 2^-24 and sc_j carries the 2^24 (both
+// exact, so the product rounds as before).  With an or and a packed subtraction a pair, as the signed Q4_0 values
+// need, 4096 x 4096 at 96 tokens took 31.4 us against 27.8, 5120 x 3072 at 64 25.5 against 22.5, 8192 x 3072 at 250
+// 51.2 against 47.8 (two calls in turn).
 // Sub-block 2p is the low nibbles of bytes 32p..32p+31, 2p + 1 the high nibbles.  Lane (g, r)
 // decodes its row's scales and mins of sub-blocks 2g and 2g + 1 into a per-wave LDS table.  Same tiles,
 // stages (half a super-block) and activation staging as gemm_b32_prompt_kernel; weights stay in the verify
@@ -248,7 +253,8 @@ int launch_gemm_prompt(const QMatDev& w, float* out, int ld_out, int N, hipStrea
 // chunk), each chunk 9 (Q5_K 11) slots of [64 lanes x 16 B]: header (d, dmin, 12 scale bytes), Q5_K's two
 // slots of high-bit bytes, nibbles.
 // Q4_K, 250 / 256 tokens, against int8 MFMA with conversions and 32 x 32 wave tiles: 8192 x 3072 58 -> 56 us,
-// 3072 x 8192 92 -> 73, 16384 x 3072 108 -> 97.  Q5_K 14336 x 4096 took 16-token slices (16 x 62 us), now 137.
+// 3072 x 8192 92 -> 73, 16384 x 3072 108 -> 97 (before the subnormals).  Q5_K 14336 x 4096 took 16-token slices (16 x 62 us), now 137.
+constexpr float kSubnormal = 16777216.0f;  // 2^24: an f16 subnormal's bits over its value
 struct PromptGemmK {
     const uint8_t* w = nullptr;
     int nsb = 0, groups = 0, tiles16 = 0;  // super-blocks per row; R16K chunks per tile; 16-row tiles stored
@@ -322,8 +328,6 @@ __global__ __launch_bounds__(256, KT == 4 ? 3 : 4) void gemm_k_prompt_kernel(Pro
         _Pragma("unroll") for (int k = 0; k < KT; k++) xar[SLOT][k] = __builtin_bit_cast(                          \
             float, __builtin_amdgcn_raw_buffer_load_b32(ares, lane * 4, prompt_unit(tt + k, (S), n16, nq) * 256, 0)); \
     }
-    uint32_t one = 0x64006400u;  // two f16 1024
-    asm("" : "+v"(one));
     p_v4f acc[KT], part[KT];
 #pragma unroll
     for (int k = 0; k < KT; k++) acc[k] = p_v4f{0.0f, 0.0f, 0.0f, 0.0f};
@@ -348,7 +352,7 @@ __global__ __launch_bounds__(256, KT == 4 ? 3 : 4) void gemm_k_prompt_kernel(Pro
                 for (int e = 0; e < 2; e++) {
                     uint32_t sv, mv;
                     q4k_scale_min_dev(2 * g + e, hdn[1], hdn[2], hdn[3], &sv, &mv);
-                    tab[wv][2 * g + e][0][r] = d * (float)sv;
+                    tab[wv][2 * g + e][0][r] = (d * (float)sv) * kSubnormal;
                     tab[wv][2 * g + e][1][r] = dmin * (float)mv;
                 }
                 if (Q5) h0 = hdn[4], h1 = hdn[5];
@@ -368,14 +372,12 @@ __global__ __launch_bounds__(256, KT == 4 ? 3 : 4) void gemm_k_prompt_kernel(Pro
                 uint32_t u[4] = {w0 >> sh, w1 >> sh, w0 >> (8 + sh), w1 >> (8 + sh)};
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    u[i] = (u[i] & 0x000F000Fu) | one;
+                    u[i] = u[i] & 0x000F000Fu;
                     if constexpr (Q5) {  // bit 4 b + j of a byte of h0 / h1 is the value's bit 4
                         const uint32_t h = (i & 1 ? h1 : h0) >> (8 * (i >> 1));
                         const int bit = 4 * b + j;
                         u[i] |= (bit < 4 ? h << (4 - bit) : h >> (bit - 4)) & 0x00100010u;
                     }
-                    const p_h2 v = __builtin_bit_cast(p_h2, u[i]);
-                    u[i] = __builtin_bit_cast(uint32_t, v - (p_h2){(_Float16)1024.0f, (_Float16)1024.0f});
                 }
                 a[j] = __builtin_bit_cast(p_h8, make_uint4(u[0], u[1], u[2], u[3]));
             }

@@ -99,3 +99,16 @@ def test_k_quant_tile_edges(ctx, qtype, M, K):
         check(ctx, nc.NC_TYPE_Q4_K, random_q4_k(M, K, seed=M + K), O.matmul_q4_k, M, K, batches, 7)
     else:
         check(ctx, nc.NC_TYPE_Q5_K, random_q5_k(M, K, seed=M + K), O.matmul_q5_k, M, K, batches, 8)
+
+
+# the K-quant prompt matmul's values are f16 subnormals and its scales carry the 2^24: super-block scales at the ends
+# of f16's range, subnormal, zero and negative
+@pytest.mark.parametrize("qtype", ["q4_k", "q5_k"])
+def test_prompt_k_quant_extreme_scales(ctx, qtype):
+    M, K = 80, 768
+    w = random_q4_k(M, K, seed=31) if qtype == "q4_k" else random_q5_k(M, K, seed=31)
+    bits = np.array([0x0001, 0x03ff, 0x0400, 0x7bff, 0x8001, 0x83ff, 0xfbff, 0x0000, 0x8000, 0x3c00], np.uint16)
+    pick = np.random.default_rng(32).integers(0, len(bits), (M, K // 256, 2))
+    w[:, :, 0:4] = np.ascontiguousarray(bits[pick]).view(np.uint8).reshape(M, K // 256, 4)
+    t, ref = (nc.NC_TYPE_Q4_K, O.matmul_q4_k) if qtype == "q4_k" else (nc.NC_TYPE_Q5_K, O.matmul_q5_k)
+    check(ctx, t, w, ref, M, K, [18, 40], 33)
