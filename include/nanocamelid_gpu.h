@@ -128,9 +128,10 @@ int64_t nc_qmat_device_bytes(const nc_qmat* w);
  * (token-major, as write_batch_out src/inference.rs:1333-1341).  batch_size >= 1, no upper
  * limit (matmul_quantized_batch takes any batch): up to 16 tokens run on the verify kernels;
  * more run on the f16 MFMA prompt matmul (every type but Q6_K; slices of up to 256 tokens through
- * buffers that nc_ctx_create allocates, 36 MiB; Q5_K and Q8_0 matrices of 2 GiB or more as 16-token
- * slices), or for Q6_K on the verify kernel in groups of up to 8 tokens.  Calls that share a
- * context and overlap on different streams race on those buffers.
+ * buffers that nc_ctx_create allocates, 72 MiB; Q5_K and Q8_0 matrices of 2 GiB or more as 16-token
+ * slices), or for Q6_K on the verify kernel in groups of up to 8 tokens.  Calls that share a context
+ * and overlap on different streams race on those buffers, but for Q8_0: the first stream with such a
+ * Q8_0 call has buffers of its own, on other streams and under capture they run as 16-token slices.
  * stream: a hipStream_t or NULL for the context's default stream. */
 int nc_matmul_quantized_batch(nc_ctx* ctx, const nc_qmat* w, const int8_t* x_i8, const float* x_scales,
                               float* out, int batch_size, int64_t rows, int64_t cols, void* stream);

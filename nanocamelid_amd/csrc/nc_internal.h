@@ -6,6 +6,7 @@
 
 #include <cstdint>
 #include <cstdio>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -273,6 +274,12 @@ struct nc_ctx {
     int8_t* pxm = nullptr;
     float* pxsm = nullptr;
     float* pxam = nullptr;
+    // the same for Q8_0, whose calls need nothing of another call's: only those on the stream that asked
+    // first use them, one launch sequence at a time (q8_mu); other streams take 16-token slices, which use none
+    int8_t* q8_xm = nullptr;
+    float* q8_xsm = nullptr;
+    std::mutex q8_mu;
+    hipStream_t q8_stream = nullptr;
     // device address of the static scratch array on this context's device (never freed)
     int32_t* static_scratch = nullptr;
     int gemm_kernel = NC_GEMM_KERNEL_AUTO;  // dot-product path of the quantized matmuls

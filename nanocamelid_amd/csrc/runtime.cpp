@@ -1447,6 +1447,8 @@ int nc_ctx_create(int device, nc_ctx** out) {
     if (e == hipSuccess) e = hipMalloc((void**)&c->pxm, 2 * kPromptRows * (kCtxScratchCols + 128));
     if (e == hipSuccess) e = hipMalloc((void**)&c->pxsm, kPromptRows * (kCtxScratchCols / 128 + 1) * 4 * sizeof(float));
     if (e == hipSuccess) e = hipMalloc((void**)&c->pxam, kPromptRows * (kCtxScratchCols / 128 + 1) * 4 * sizeof(float));
+    if (e == hipSuccess) e = hipMalloc((void**)&c->q8_xm, 2 * kPromptRows * (kCtxScratchCols + 128));
+    if (e == hipSuccess) e = hipMalloc((void**)&c->q8_xsm, kPromptRows * (kCtxScratchCols / 128 + 1) * 4 * sizeof(float));
     if (e != hipSuccess) {
         nc_ctx_free(c);
         return fail(NC_EHIP, std::string("nc_ctx_create: ") + hipGetErrorString(e));
@@ -1463,6 +1465,8 @@ void nc_ctx_free(nc_ctx* c) {
     if (c->pxm) (void)hipFree(c->pxm);
     if (c->pxsm) (void)hipFree(c->pxsm);
     if (c->pxam) (void)hipFree(c->pxam);
+    if (c->q8_xm) (void)hipFree(c->q8_xm);
+    if (c->q8_xsm) (void)hipFree(c->q8_xsm);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
 }
@@ -1537,19 +1541,31 @@ static int prompt_slice_tokens(int64_t cols) {
     return (int)std::min<int64_t>(kPromptRows, (int64_t)kPromptRows * (int64_t)kCtxScratchCols / cols / 16 * 16);
 }
 
-// The prompt matmul (Q4_0 or Q4_K) of batch_size > 16 tokens through the context's repack
+// The prompt matmul (every type but Q6_K) of batch_size > 16 tokens through the context's repack
 // buffers, in slices of prompt_slice_tokens (every token's outputs are the same bits in any
 // slicing).
 static int ctx_prompt_matmul(nc_ctx* ctx, const QMatDev& w, const int8_t* x, const float* xs, float* out, int n,
                              hipStream_t st) {
     const int cols = (int)w.cols, T = prompt_slice_tokens(cols);
+    const bool q8 = w.type == NC_TYPE_Q8_0;
     for (int i = 0; i < n; i += T) {
         const int len = std::min(T, n - i);
         int rc = prompt_matmul(w, x + (size_t)i * cols, xs + (size_t)i * (cols / 32), out + (size_t)i * w.rows,
-                               (int)w.rows, len, st, ctx->pxm, ctx->pxsm, ctx->pxam);
+                               (int)w.rows, len, st, q8 ? ctx->q8_xm : ctx->pxm, q8 ? ctx->q8_xsm : ctx->pxsm,
+                               ctx->pxam);
         if (rc) return rc;
     }
     return NC_OK;
+}
+
+// Whether a Q8_0 call on st may use the context's Q8_0 repack buffers (under q8_mu): the first stream that
+// asks keeps them, and a call under capture (whose graph runs at any time) never does.  Ordering the streams with
+// an event at the end of each call instead cost 3.5 us a call, of 48.
+static bool q8_buffers_for(nc_ctx* ctx, hipStream_t st) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return false;
+    if (!ctx->q8_stream) ctx->q8_stream = st;
+    return ctx->q8_stream == st;
 }
 
 int nc_matmul_quantized_batch(nc_ctx* ctx, const nc_qmat* w, const int8_t* x_i8, const float* x_scales, float* out,
@@ -1560,8 +1576,11 @@ int nc_matmul_quantized_batch(nc_ctx* ctx, const nc_qmat* w, const int8_t* x_i8,
     NC_HIP(hipSetDevice(ctx->device));
     hipStream_t st = stream ? (hipStream_t)stream : ctx->stream;
     // more than 16 tokens: the MFMA prompt matmul (every type but Q6_K)
-    if (batch_size > 16 && prompt_matrix_ok(w->m) && prompt_slice_tokens(cols) >= 16)
-        return ctx_prompt_matmul(ctx, w->m, x_i8, x_scales, out, batch_size, st);
+    if (batch_size > 16 && prompt_matrix_ok(w->m) && prompt_slice_tokens(cols) >= 16) {
+        if (w->m.type != NC_TYPE_Q8_0) return ctx_prompt_matmul(ctx, w->m, x_i8, x_scales, out, batch_size, st);
+        std::lock_guard<std::mutex> lock(ctx->q8_mu);
+        if (q8_buffers_for(ctx, st)) return ctx_prompt_matmul(ctx, w->m, x_i8, x_scales, out, batch_size, st);
+    }
     const int slice = slice_tokens(w->m, batch_size);
     for (int i = 0; i < batch_size; i += slice) {
         const int nb = std::min(slice, batch_size - i);

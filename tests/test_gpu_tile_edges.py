@@ -112,3 +112,38 @@ def test_prompt_k_quant_extreme_scales(ctx, qtype):
     w[:, :, 0:4] = np.ascontiguousarray(bits[pick]).view(np.uint8).reshape(M, K // 256, 4)
     t, ref = (nc.NC_TYPE_Q4_K, O.matmul_q4_k) if qtype == "q4_k" else (nc.NC_TYPE_Q5_K, O.matmul_q5_k)
     check(ctx, t, w, ref, M, K, [18, 40], 33)
+
+
+# Q8_0 calls of more than 16 tokens share no scratch with any other call: on two streams at once, beside Q4_0 ones
+# on a third, and replayed from a graph, every output is the one that the same call gives alone
+def test_q8_0_prompt_matmul_on_several_streams():
+    import torch
+    M, K, N, reps = 4096, 2048, 100, 12
+    ctx = nc.Context(0)
+    q8 = nc.QMat(ctx, nc.NC_TYPE_Q8_0, M, K, random_q8_0(M, K, seed=12))
+    q4 = nc.QMat(ctx, nc.NC_TYPE_Q4_0, M, K, random_q4_0(M, K, seed=13))
+    calls = [(w, *[torch.from_numpy(a).cuda() for a in q8_activations(N, K, 20 + i)[1:]]) for i, w in enumerate((q8, q8, q4, q8))]
+    streams = [torch.cuda.Stream() for _ in calls]
+    torch.cuda.synchronize()
+    with torch.cuda.stream(streams[0]):  # the first stream: the one with the buffers
+        want = [nc.matmul_quantized_batch(ctx, w, x, s) for w, x, s in calls]
+    got = [[torch.zeros_like(want[0]) for _ in range(reps)] for _ in calls]
+    captured = torch.zeros_like(want[0])
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=streams[3]):
+        nc.matmul_quantized_batch(ctx, *calls[3], out=captured)
+    for j in range(reps):
+        for i in range(3):
+            with torch.cuda.stream(streams[i]):
+                nc.matmul_quantized_batch(ctx, *calls[i], out=got[i][j])
+        with torch.cuda.stream(streams[3]):
+            captured.zero_()
+            graph.replay()
+            got[3][j].copy_(captured)
+    torch.cuda.synchronize()
+    for i in range(4):
+        for j in range(reps):
+            assert torch.equal(got[i][j].view(torch.int32), want[i].view(torch.int32)), (i, j)
+    q8.close()
+    q4.close()
