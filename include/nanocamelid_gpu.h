@@ -140,7 +140,8 @@ int nc_matmul_quantized_batch(nc_ctx* ctx, const nc_qmat* w, const int8_t* x_i8,
  * loops that forbid hipMalloc).  Same arguments, semantics and results; its only scratch is a
  * static per-device array sized for batch_size * cols <= 16 * 65536 (larger: NC_ERANGE;
  * batch_size above 16: NC_EINVAL).  It
- * calls no hipMalloc/hipFree.  Calls that overlap on one device share that array and race. */
+ * calls no hipMalloc/hipFree.  Calls with block sums (K-quants of rows too long for the kernel's own or
+ * of more than 16320 rows, Q4_0 on the MFMA path) that overlap on one device share that array and race. */
 int nc_matmul_quantized_batch_noalloc(nc_ctx* ctx, const nc_qmat* w, const int8_t* x_i8, const float* x_scales,
                                       float* out, int batch_size, int64_t rows, int64_t cols, void* stream);
 /* Debug/parity variant: writes the int32 per-block dot products (Q4_0:

@@ -152,6 +152,7 @@ inline size_t q4k_r16_lds_bytes(const QMatDev& w, int n, bool own_sums) {
     const size_t nmax = n <= 9 ? n : 16, S = w.groups >= 8 ? 8 : 4;
     return 2 * 4 * S * nmax * 16 * sizeof(float) + (own_sums ? (size_t)n * w.units * 8 * sizeof(float) : 0);
 }
+bool needs_block_sums(const nc_ctx* ctx, const QMatDev& q, int n);  // of an operator call of n <= 16 tokens
 int launch_blockdots(const QMatDev& w, const int8_t* x, int32_t* dots, int N, hipStream_t stream);
 // Q6_K matmul of up to q6k_launch_tokens tokens (plain outputs or the head's logits + argmax partials)
 int launch_gemm_q6k(const QMatDev& w, const GemmParams& p, hipStream_t stream);

@@ -1161,7 +1161,7 @@ static int sample_session_rows(nc_session* s, int row0, int rows, float temp, co
 }
 
 // ---------------------------------------------------------------- prompt passes
-// Matrices with an MFMA prompt matmul: Q4_0 (R16 or R64 tiles) and Q4_K (R16K or R64).
+// Matrices with an MFMA prompt matmul: every type but Q6_K.
 static bool prompt_matrix_ok(const QMatDev& q) {
     if (q.type == NC_TYPE_Q4_0) return q.layout == LAYOUT_R16 || q.layout == LAYOUT_R64;
     if (q.type == NC_TYPE_Q4_K) return q.layout == LAYOUT_R16K || q.layout == LAYOUT_R64;
@@ -1180,7 +1180,7 @@ static int slice_tokens(const QMatDev& q, int n) {
 // Q5_K, and for the offset of the unsigned Q4_0 nibbles on the int8 MFMA path.
 // A plain K-quant matmul of n tokens on 16-row tiles sums for itself where the sums fit in 64 KB of LDS
 // beside its terms.
-static bool needs_block_sums(const nc_ctx* ctx, const QMatDev& q, int n) {
+bool needs_block_sums(const nc_ctx* ctx, const QMatDev& q, int n) {
     if (q.layout == LAYOUT_R16K && !getenv("NC_Q4K_PS") && q4k_r16_lds_bytes(q, n, true) <= 65536) return false;
     return q.type == NC_TYPE_Q4_K || q.type == NC_TYPE_Q5_K ||
            (q.type == NC_TYPE_Q4_0 && ctx->gemm_kernel == NC_GEMM_KERNEL_MFMA);
