@@ -87,7 +87,6 @@ struct TpSegInfo {
 };
 struct TpEnt {
     double cstart, cend;  // uncorrected start and end of a sensitive run, relative to its segment
-    double shift;         // true end - uncorrected end (global), after the walk
     int run;              // run index in the row (term run * kSmE is its first term)
     int pad;
 };
@@ -238,7 +237,8 @@ __global__ __launch_bounds__(kSmT) void tp_sum_kernel(const float* probs, int64_
 //   tps_finish  the boundaries between segments; if any check failed, or a segment had more
 //               sensitive runs than it lists, S is evaluated segment after segment as
 //               tp_sum_kernel does.  With NORM, one workgroup per segment also scales its
-//               probabilities by 1 / S (in that rare case every one evaluates S).
+//               probabilities by 1 / S (in that rare case the first one evaluates S and scales
+//               the whole row).
 // 5 rows of 128256 (launches included): 30 us, where walk, verify, finish and norm as four launches and a margin of
 // 256 ulps, which rows of N(0, 2.5) logits overran on some binade edges, took 50 us, or 130 with such a row.
 // As in exact_chain_sum, the result is the sequential chain whenever it is accepted: the
