@@ -88,3 +88,19 @@ def test_prompt_and_oracle_drafter_match_oracle():
     for p in range(32, 400, 7):
         for alpha in (0.5, 0.8):
             assert nc.oracle_draft(9, p, alpha, greedy, 32, 128256) == O.oracle_draft(9, p, alpha, greedy, 32, 128256)
+
+
+def test_stream_handle_without_torchs_private_getter(monkeypatch):
+    """The operator wrappers pass torch's current stream as a raw handle; where torch lacks the function
+    that gives it, they take it from the public Stream object."""
+    import types
+
+    import torch
+
+    import nanocamelid_amd as nc
+    tensor = types.SimpleNamespace(device=torch.device("cuda", 0))
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 100 + index, raising=False)
+    assert nc._stream_of(tensor) == 100
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream")
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device: types.SimpleNamespace(cuda_stream=7))
+    assert nc._stream_of(tensor) == 7
