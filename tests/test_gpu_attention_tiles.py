@@ -9,10 +9,10 @@ from oracle import oracle as O
 pytestmark = pytest.mark.gpu
 
 
-# heads, KV heads, head dim and the chunk lengths of one prompt, each a pass of >= 1024 * 128 / hd units: rows
-# that cut a tile (35, 70, 101), tiles across two heads' rows, eight and one heads per KV head, starts
-# off the 16- and 256-position steps
-@pytest.mark.parametrize("H,Hkv,hd,chunks", [(32, 4, 128, [35, 70, 256, 33]), (32, 32, 128, [101, 48]),
+# heads, KV heads, head dim and the chunk lengths of one prompt, each a pass of at least 1536 (head dim 128) or 2048
+# (64) units, where the tiles begin: rows that cut a tile (49, 51, 101), tiles across two heads' rows, eight and one
+# heads per KV head, starts off the 16- and 256-position steps
+@pytest.mark.parametrize("H,Hkv,hd,chunks", [(32, 4, 128, [49, 70, 256, 51]), (32, 32, 128, [101, 48]),
                                              (32, 8, 64, [70, 190, 67, 256]), (64, 8, 64, [35, 33, 200])])
 def test_tiled_attention_vs_oracle(H, Hkv, hd, chunks):
     ctx = nc.Context(0)
@@ -35,6 +35,49 @@ def test_tiled_attention_vs_oracle(H, Hkv, hd, chunks):
     assert np.array_equal(preds, opreds)
     for i in range(5):
         assert np.array_equal(gs.logits(i).view(np.uint32), ologits[i].view(np.uint32)), i
+
+
+def filled(H, Hkv, hd, start, end):
+    """A two-layer model's session and the oracle's, both with the same keys and values before start."""
+    ctx = nc.Context(0)
+    img = nc.synth_gguf(layers=2, embedding_length=H * hd, head_count=H, head_count_kv=Hkv, feed_forward_length=256,
+                        vocab_size=300, context_length=16384, tied=1, norm_mode=1, seed=H + Hkv + hd + start)
+    gs = nc.Session(nc.Model(ctx, data=img), end, 16)
+    os_ = O.Session(O.Model(data=img.tobytes(), nthreads=8), end, 16)
+    gs.fill_kv(start, 9)
+    os_.fill_kv(start, 9)
+    return gs, os_
+
+
+def verify_both(gs, os_, pos, rows):
+    toks = nc.uniform_prompt(pos + rows, rows, 300)
+    _, _, _, preds = gs.verify_greedy(toks, pos)
+    opreds, _, ologits = os_.verify_greedy(toks, pos, want_logits=True)
+    assert np.array_equal(preds, opreds)
+    for i in range(rows):
+        assert np.array_equal(gs.logits(i).view(np.uint32), ologits[i].view(np.uint32)), (pos, i)
+
+
+# the same at long positions, over a filled cache: a pass of 49 or 67 rows (1568, 2144 units) that ends past 2048, 4096
+# and 8192 positions and at the last position a pass can have before the verify rows (16384 in all)
+@pytest.mark.parametrize("H,Hkv,hd,start,rows", [(32, 4, 128, 2030, 49), (32, 32, 128, 4090, 49), (32, 4, 128, 8190, 49),
+                                                 (32, 4, 128, 16384 - 54, 49), (32, 8, 64, 4090, 67), (32, 4, 64, 8150, 67)])
+def test_tiled_attention_at_long_positions_vs_oracle(H, Hkv, hd, start, rows):
+    gs, os_ = filled(H, Hkv, hd, start, start + rows + 5)
+    toks = nc.uniform_prompt(start, rows, 300)
+    gs.prefill_pass_batch(toks, start, want_logits=False)
+    for i in range(0, rows, 16):
+        os_.prefill_pass_batch(toks[i:i + 16], start + i)
+    verify_both(gs, os_, start + rows, 5)  # reads layer 1's keys and values, made from layer 0's tiles
+
+
+# wide verify passes (more units than CUs, too few for the tiles) on the 256-thread softmax and V kernels, at the last
+# and the first row length of each: up to 2048, 4096 and 8192 positions, and the one extra position a thread past 8192
+@pytest.mark.parametrize("H,Hkv,hd,rows", [(32, 4, 128, 9), (64, 8, 64, 5)])
+@pytest.mark.parametrize("longest", [2048, 2049, 4096, 4097, 8192, 8199])
+def test_wide_verify_at_long_positions_vs_oracle(H, Hkv, hd, rows, longest):
+    gs, os_ = filled(H, Hkv, hd, longest - rows, longest)
+    verify_both(gs, os_, longest - rows, rows)
 
 
 # rows just past the one-kernel attention (512, 1024 or 1536 positions by head dim and units) and the scores'

@@ -303,9 +303,8 @@ def test_long_context_logits(ctx, hd, checks):
 @pytest.mark.parametrize("hd,wt", [(64, 2), (128, 2), (128, 12), (128, 8), (64, 13)],
                          ids=["hd64-q4_0", "hd128-q4_0", "hd128-q4_k", "hd128-q8_0", "hd64-q5_k"])
 def test_prompt_passes_match_oracle(ctx, hd, wt):
-    """Prompts of 32 or more tokens on Q4_0 and Q4_K models run as MFMA prompt passes of up to
-    256 tokens, Q8_0 and Q5_K models as the same passes with their matmuls in 16-token slices of the
-    verify kernel (epilogues as separate kernels, attention in 64-row groups): a 300-token prompt
+    """Prompts of 32 or more tokens run as prompt passes of up to 256 tokens: MFMA prompt matmuls,
+    epilogues as separate kernels, the attention of all rows at once.  A 300-token prompt
     without logits (passes of 256 + 44) and 400 more with logits (passes of 256 + 128, then the
     last 16 rows as a verify-sized pass), then a 9-row verify: every logit bit-identical to the
     oracle's after 16-token chunks, i.e. the same KV cache bits."""
@@ -322,6 +321,27 @@ def test_prompt_passes_match_oracle(ctx, hd, wt):
     batch = nc.uniform_prompt(700, 9, 1000)
     _, _, _, preds = gs.verify_greedy(batch, 700)
     opreds, _, ologits = os_.verify_greedy(batch, 700, want_logits=True)
+    assert np.array_equal(preds, opreds)
+    for i in range(9):
+        assert _same(gs.logits(i), ologits[i]), i
+
+
+def test_prompt_pass_of_a_wide_q4_k_gateup(ctx):
+    """An interleaved Q4_K gate,up of 16384 rows on 16-row tiles: its 256-token prompt pass is the one
+    that takes four token tiles a workgroup on that layout; then 40 tokens on one.  Layer 0's outputs
+    feed layer 1's keys and values, which the verify's logits read."""
+    import nanocamelid_amd as nc
+    spec = dict(TINY, head_count=4, head_count_kv=2, embedding_length=256, feed_forward_length=8192,
+                context_length=512, weight_type=12)
+    _, gm, om = _models(ctx, spec, seed=77)
+    prompt = nc.uniform_prompt(78, 296, 1000)
+    gs, os_ = nc.Session(gm, 512, 16), O.Session(om, 512, 16)
+    gs.prefill_pass_batch(prompt, 0, want_logits=False)
+    for i in range(0, 296, 16):
+        os_.prefill_pass_batch(prompt[i:min(i + 16, 296)], i)
+    batch = nc.uniform_prompt(296, 9, 1000)
+    _, _, _, preds = gs.verify_greedy(batch, 296)
+    opreds, _, ologits = os_.verify_greedy(batch, 296, want_logits=True)
     assert np.array_equal(preds, opreds)
     for i in range(9):
         assert _same(gs.logits(i), ologits[i]), i
@@ -505,12 +525,12 @@ def test_long_context_many_units(ctx):
 
 @pytest.mark.parametrize("hd", [64, 128])
 def test_long_prompt_many_unit_tiers_vs_oracle(ctx, hd):
-    """A 4300-token prompt on a two-layer model with 8 query heads: its prompt passes run the
-    attention of 64-row groups (512 (row, head) units) through the one-kernel tiers, then the
-    256-thread softmax tiers at up to 2048, 4096 and 8192 positions with the software-pipelined
-    weighted-V loop.  Layer 0's attention outputs feed layer 1's keys and values, so a 9-row
+    """A 4300-token prompt on a two-layer model with 8 query heads: its 256-row prompt passes are
+    2048 (row, head) units and run on the 16-query tiles from the first position on, the last one of
+    204 rows (1632 units) at head dim 64 on the tiled scores and the 256-thread softmax and V kernel
+    of up to 8192 positions.  Layer 0's attention outputs feed layer 1's keys and values, so a 9-row
     verify at 4300 whose every logit is bit-identical to the oracle's (16-token chunks) pins
-    those tiers."""
+    them.  The other 256-thread kernels: test_wide_verify_at_long_positions_vs_oracle."""
     import nanocamelid_amd as nc
     spec = dict(layers=2, embedding_length=8 * hd, head_count=8, head_count_kv=2, feed_forward_length=512,
                 vocab_size=1000, context_length=4400, tied=1, norm_mode=1)

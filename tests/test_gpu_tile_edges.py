@@ -66,11 +66,14 @@ def test_q8_0_tile_edges(ctx, M, K):
     check(ctx, nc.NC_TYPE_Q8_0, w, O.matmul_q8_0, M, K, [1, 2, 3, 4, 5, 6, 7, 8, 9, 16, 17, 50], 4)
 
 
-# the prompt matmul's wave tiles: 16 x 32 (few workgroups), 16 x 64 and 32 x 64 (many), on 16-row tiles and, from
-# 65536 rows of Q4_0, on 64-row tiles; K: one block, cut quads, an odd number of quads; ragged rows and tokens
+# the prompt matmuls' workgroups: 64 rows x 16, 32 or 64 tokens (one, two or four token tiles a wave), by how many a
+# launch has.  K: one unit, cut quads, an odd number of quads; ragged rows and tokens.  K-quants: one tile up to 200 rows
+# and at 40 and 4 (of 260) tokens of 16000, two at 66 to 260 tokens of 16000 and more, on 64-row tiles from 16321
+# rows four at 200 and 256 tokens and, for the 257th token alone, one.  (Four on 16-row tiles needs an
+# interleaved gate,up: test_prompt_pass_of_a_wide_q4_k_gateup.)
 @pytest.mark.parametrize("qtype", ["q4_k", "q5_k"])
-@pytest.mark.parametrize("M,K,batches", [(17, 256, [17, 33, 64]), (200, 1280, [40, 130, 300]), (16401, 512, [129, 66]),
-                                         (16000, 256, [260, 40])])
+@pytest.mark.parametrize("M,K,batches", [(17, 256, [17, 33, 64]), (200, 1280, [40, 130, 300]),
+                                         (16401, 512, [129, 66, 200, 257]), (16000, 256, [260, 40])])
 def test_prompt_k_quant_matmul_wave_tiles(ctx, qtype, M, K, batches):
     if qtype == "q4_k":
         check(ctx, nc.NC_TYPE_Q4_K, random_q4_k(M, K, seed=M), O.matmul_q4_k, M, K, batches, 9)
@@ -78,9 +81,11 @@ def test_prompt_k_quant_matmul_wave_tiles(ctx, qtype, M, K, batches):
         check(ctx, nc.NC_TYPE_Q5_K, random_q5_k(M, K, seed=M), O.matmul_q5_k, M, K, batches, 10)
 
 
+# Q4_0 and Q8_0: one token tile up to 200 rows, two at 20 tokens of 32785, four at 66 tokens and more of 16401; Q4_0 on
+# 64-row tiles from 65473 rows: two at 20 tokens, four at 65 and 256, one for the 257th token alone
 @pytest.mark.parametrize("qtype", ["q4_0", "q8_0"])
 @pytest.mark.parametrize("M,K,batches", [(17, 32, [17, 33, 64]), (200, 416, [40, 130, 300]), (16401, 96, [129, 66]),
-                                         (32785, 288, [130]), (65553, 96, [20, 65]), (20, 8224, [31, 49])])
+                                         (32785, 288, [130, 20]), (65553, 96, [20, 65, 257]), (20, 8224, [31, 49])])
 def test_prompt_block_matmul_wave_tiles(ctx, qtype, M, K, batches):
     if qtype == "q4_0":
         check(ctx, nc.NC_TYPE_Q4_0, random_q4_0(M, K, seed=M), O.matmul_q4_0, M, K, batches, 5)
