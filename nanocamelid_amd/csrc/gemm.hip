@@ -115,8 +115,9 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, const float* 
             case EPI_HEAD: {
                 // logits row + first-max argmax partial of this tile (inference.rs:4836-4846).
                 if (row < p.M) p.out[(size_t)n * p.ld_out + row] = v;
-                float bv = row < p.M ? v : -__builtin_inff();
-                int bi = row < p.M ? row : 0x7fffffff;
+                float bv;
+                int bi;
+                head_entry(v, row, p.M, &bv, &bi);
 #pragma unroll
                 for (int off = 32; off >= 1; off >>= 1) {
                     float ov = __shfl_xor(bv, off, 64);
@@ -474,8 +475,9 @@ __device__ __forceinline__ void gemm_epilogue_r16(const GemmParams& p, float v, 
         case EPI_HEAD: {
             // logits row + first-max argmax partial of this 16-row tile (inference.rs:4836-4846)
             if (row < p.M) p.out[(size_t)n * p.ld_out + row] = v;
-            float bv = row < p.M ? v : -__builtin_inff();
-            int bi = row < p.M ? row : 0x7fffffff;
+            float bv;
+            int bi;
+            head_entry(v, row, p.M, &bv, &bi);
 #pragma unroll
             for (int off = 8; off >= 1; off >>= 1) {
                 const float ov = __shfl_xor(bv, off, 64);

@@ -84,6 +84,15 @@ __device__ __forceinline__ int quantize_lane_q8(float v, float amax, float* scal
     return 0;
 }
 
+// A row's entry in the head's search for the first maximum (inference.rs:4836-4846: from logits[0] on, a
+// later logit wins if it is greater), which the tiles run as pairs (value, lower index on ties): a NaN never
+// wins, except as logits[0], which nothing exceeds then.  Rows past the matrix take no part.
+__device__ __forceinline__ void head_entry(float logit, int row, int rows, float* value, int* index) {
+    const bool nan = logit != logit, in = row < rows && (!nan || row == 0);
+    *value = in ? (nan ? __builtin_inff() : logit) : -__builtin_inff();
+    *index = in ? row : 0x7fffffff;
+}
+
 // Max of |v| over each 32-lane half of the wave (exact: max is order independent).
 __device__ __forceinline__ float halfwave_amax(float v) {
     float a = __builtin_fabsf(v);

@@ -161,8 +161,9 @@ __global__ __launch_bounds__(64 * W) void gemm_q6_k_kernel(GemmParams p, int nb,
         if (row < p.M) p.out[(size_t)n * p.ld_out + row] = acc;
         if (p.epi == EPI_HEAD) {
             // the first maximum of the tile's rows (inference.rs:4836-4846): value, lower index on ties
-            float bv = row < p.M ? acc : -__builtin_inff();
-            int bi = row < p.M ? row : 0x7fffffff;
+            float bv;
+            int bi;
+            head_entry(acc, row, p.M, &bv, &bi);
 #pragma unroll
             for (int off = 8; off >= 1; off >>= 1) {
                 const float ov = __shfl_xor(bv, off, 64);

@@ -347,6 +347,41 @@ def test_prompt_pass_of_a_wide_q4_k_gateup(ctx):
         assert _same(gs.logits(i), ologits[i]), i
 
 
+@pytest.mark.parametrize("ty", [2, 8, 12, 14])
+def test_nan_logits_do_not_hide_others(ctx, ty):
+    """NaN logits in a prediction's own 16- and 64-row tile (the head's rows at the tiles' starts have a NaN
+    scale) leave the prediction as the reference's search gives it, from logits[0] on with each greater one;
+    with logits[0] itself a NaN, that search returns 0."""
+    import nanocamelid_amd as nc
+    from tests import gguf_writer as GW
+    from tests.gpu_util import random_q4_0, random_q4_k, random_q8_0
+    bs, size, d_at = {2: (32, 18, 0), 8: (32, 34, 0), 12: (256, 144, 0), 14: (256, 210, 208)}[ty]
+    blocks = {2: lambda: random_q4_0(1000, 256, 50), 8: lambda: random_q8_0(1000, 256, 50),
+              12: lambda: random_q4_k(1000, 256, 50), 14: lambda: GW.q6_k_weights(1000, 50)}[ty]().ravel()
+    img = np.array(np.frombuffer(GW.with_types(nc.synth_gguf(**TINY, seed=50), {"output.weight": ty}), np.uint8))
+    off, head_ty = next((t[3], t[2]) for t in nc.gguf_tensors(img) if t[0] == "output.weight")
+    assert head_ty == ty
+    img[off:off + blocks.size] = blocks
+    nan_rows, batch = set(), nc.uniform_prompt(51, 9, 1000)
+
+    def passes():
+        for r in nan_rows:
+            img[off + r * (256 // bs) * size + d_at:][:2] = (0x00, 0x7e)
+        gs = nc.Session(nc.Model(ctx, data=img), 64, 16)
+        os_ = O.Session(O.Model(data=img.tobytes(), nthreads=16), 64, 16)
+        _, _, _, preds = gs.verify_greedy(batch, 0)
+        opreds, _, ologits = os_.verify_greedy(batch, 0, want_logits=True)
+        assert np.array_equal(np.isnan(ologits[0]).nonzero()[0], sorted(nan_rows))
+        assert np.array_equal(preds, opreds), (sorted(nan_rows), preds, opreds)
+        return [int(p) for p in preds]
+
+    clean = passes()
+    nan_rows = {p // n * n for p in clean for n in (16, 64)} - set(clean) - {0}
+    assert passes() == clean
+    nan_rows.add(0)
+    assert passes() == [0] * 9
+
+
 @pytest.mark.parametrize("ty", [1, 30, 8, 3, 6, 13, 14])
 def test_embedding_types_model_logits(ctx, ty):
     """Token embeddings stored as F16, BF16, Q8_0, Q4_1, Q5_0, Q5_K or Q6_K (load_f32_or_f16,
