@@ -1091,9 +1091,12 @@ __global__ __launch_bounds__(64 * S) void gemm_q4_k_kernel(GemmParams p) {
 // p.xs8 null (operator calls, whose activations come without block sums): the workgroup sums its
 // activations' blocks itself, into LDS beside the terms, while its first weights arrive.  A separate launch for
 // them cost 2 us of device and 3 us of host time before a 9 us matmul.
+//
+// Registers: a SIMD holds three waves of up to 168, so the widths near that are kept below it (Q4_K at 5 tokens
+// takes 169 by itself: 14336 x 4096 17.7 us, 11008 x 4096 14.9, against 16.8 and 13.3).
 template <int NMAX, int S, int D, bool Q5 = false>
-__global__ __launch_bounds__(64 * S) void gemm_q4_k_r16_kernel(GemmParams p) {
-    static_assert(16 * NMAX <= 64 * S, "chain threads must fit the workgroup");
+__global__ __launch_bounds__(64 * S, NMAX <= (Q5 ? 3 : 5) ? 3 : 1) void gemm_q4_k_r16_kernel(GemmParams p) {
+    constexpr int TPC = (16 * NMAX + 64 * S - 1) / (64 * S);  // chains per thread
     constexpr int NSLOT = Q5 ? 11 : 9, QS = Q5 ? 3 : 1, CHUNK = NSLOT * 1024;
     extern __shared__ float lds[];  // [2][4*S][NMAX][16] super-block terms, then [N][nb] block sums
     const int tile = blockIdx.x;
@@ -1135,7 +1138,7 @@ __global__ __launch_bounds__(64 * S) void gemm_q4_k_r16_kernel(GemmParams p) {
     for (int k = 0; k < D - 1; k++) NC_K16_LOAD(k, k);
     if (own_sums) {
         for (int i = threadIdx.x; i < N * nb; i += 64 * S) {
-            const int* x = (const int*)(p.x + (size_t)(i / nb) * p.K) + 8 * (i % nb);
+            const int* x = (const int*)p.x + 8 * i;  // block i of [N][nb]
             int sum = 0;
 #pragma unroll
             for (int e = 0; e < 8; e++) sum = __builtin_amdgcn_sdot4(x[e], 0x01010101, sum, false);
@@ -1143,8 +1146,10 @@ __global__ __launch_bounds__(64 * S) void gemm_q4_k_r16_kernel(GemmParams p) {
         }
         __syncthreads();
     }
-    float acc = 0.0f;
-    const int cn = threadIdx.x >> 4, cr = threadIdx.x & 15;  // chain thread: token, row
+    float acc[TPC];
+#pragma unroll
+    for (int t = 0; t < TPC; t++) acc[t] = 0.0f;
+    const int cn = threadIdx.x >> 4, cr = threadIdx.x & 15;  // chain t: token cn + 4 S t, row cr
     for (int r0 = 0; r0 < nrounds; r0 += D) {
 #pragma unroll
         for (int k = 0; k < D; k++) {
@@ -1222,15 +1227,20 @@ __global__ __launch_bounds__(64 * S) void gemm_q4_k_r16_kernel(GemmParams p) {
 #pragma unroll
                 for (int n = 0; n < NMAX; n++) buf[((wave * 4 + q) * NMAX + n) * 16 + j] = part[n];
                 __syncthreads();
-                if (threadIdx.x < 16 * NMAX && cn < N) {
-                    const int nblk = min(4 * S, nsb - r * 4 * S);
-                    for (int bl = 0; bl < nblk; bl++) acc = acc + buf[(bl * NMAX + cn) * 16 + cr];
+                const int nblk = min(4 * S, nsb - r * 4 * S);
+#pragma unroll
+                for (int t = 0; t < TPC; t++) {
+                    const int n = cn + 4 * S * t;
+                    if (n < N)  // N <= NMAX
+                        for (int bl = 0; bl < nblk; bl++) acc[t] = acc[t] + buf[(bl * NMAX + n) * 16 + cr];
                 }
             }
         }
     }
 #undef NC_K16_LOAD
-    if (threadIdx.x < 16 * NMAX && cn < N) gemm_epilogue_r16<NMAX>(p, acc, cn, tile, cr);
+#pragma unroll
+    for (int t = 0; t < TPC; t++)
+        if (cn + 4 * S * t < N) gemm_epilogue_r16<NMAX>(p, acc[t], cn + 4 * S * t, tile, cr);
 }
 
 // ---------------------------------------------------------------- Q4_K, 16-row tiles, pair-split
@@ -1613,9 +1623,8 @@ int launch_k(int S, const QMatDev& w, const GemmParams& p, hipStream_t st, hipEv
     }
 }
 
-// Q4_K on 16-row tiles: 8 waves (one quad of super-blocks each per round) when K has at least
-// 8 quads, else 4 (enough chain threads for 16 tokens); a ring of 2 rounds, 1 at 16 rows
-// (registers).
+// Q4_K and Q5_K on 16-row tiles: q4k_r16_waves waves (one quad of super-blocks each per round); a ring of 2
+// rounds, 1 at 16 rows (registers).
 template <int NMAX, bool Q5 = false>
 int launch_k16(const QMatDev& w, const GemmParams& p, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
     constexpr int D = NMAX <= 9 ? 2 : 1;
@@ -1627,10 +1636,16 @@ int launch_k16(const QMatDev& w, const GemmParams& p, hipStream_t st, hipEvent_t
         else
             NC_LAUNCH((gemm_q4_k_r16_kernel<NMAX, S, D, Q5>), dim3(p.ntiles), dim3(64 * S), lds, st, p);
     };
+    auto plain = [&] {
+        const int S = q4k_r16_waves(w);
+        if (S == 8) go.template operator()<8>();
+        else if (S == 4) go.template operator()<4>();
+        else if (S == 2) go.template operator()<2>();
+        else go.template operator()<1>();
+    };
     if constexpr (Q5) {
         if (p.epi == EPI_SWIGLU_Q8) return fail(NC_EINVAL, "gemm: 16-row Q5_K tiles have no SwiGLU epilogue");
-        if (w.groups >= 8) go.template operator()<8>();
-        else go.template operator()<4>();
+        plain();
         NC_HIP(hipGetLastError());
         return NC_OK;
     }
@@ -1663,16 +1678,13 @@ int launch_k16(const QMatDev& w, const GemmParams& p, hipStream_t st, hipEvent_t
             ps.template operator()<3, 1>();
         } else if (forced == 4) {
             ps.template operator()<4, 1>();
-        } else if (w.groups >= 8) {
-            go.template operator()<8>();
         } else {
-            go.template operator()<4>();
+            plain();
         }
     } else {
         if (p.epi == EPI_SWIGLU_Q8)
             return fail(NC_EINVAL, "gemm: the 16-row Q4_K SwiGLU epilogue takes at most 9 tokens");
-        if (w.groups >= 8) go.template operator()<8>();
-        else go.template operator()<4>();
+        plain();
     }
     NC_HIP(hipGetLastError());
     return NC_OK;

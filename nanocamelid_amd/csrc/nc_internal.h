@@ -146,10 +146,18 @@ struct GemmParams {
 // ev0/ev1: optional events stamped at the kernel's own start and end (timing).
 int launch_gemm(const QMatDev& w, const GemmParams& p, hipStream_t stream, hipEvent_t ev0 = nullptr,
                 hipEvent_t ev1 = nullptr);
-// LDS of the 16-row K-quant kernel for n tokens (S = 8 waves from 8 quads on, else 4): two rounds of terms,
-// and the activations' block sums when it makes its own.
+// Waves of the 16-row K-quant kernel: 4, or 8 for rows of at least 8 quads of super-blocks in a launch of at most one
+// workgroup a CU (more of them hold 12 waves a CU as four, 8 as eight: 16000 x 8192 at 1 / 5 tokens 20.3 / 34.8 us with
+// eight, 15.5 / 24.5 with four).  Rows of one or two quads take one or two, as the others would only wait, from
+// two workgroups a CU on, whose waves the idle ones keep out (5 tokens, four / these: 14000 x 1024 13.6 / 7.4 us,
+// 16000 x 2048 15.3 / 9.9; with fewer workgroups the shorter chains and sums of four count: 8000 x 2048 at 16 tokens
+// 14.9 / 15.7).
+inline int q4k_r16_waves(const QMatDev& w) {
+    return w.groups >= 8 && w.tiles <= 256 ? 8 : w.groups > 2 || w.tiles <= 512 ? 4 : (int)w.groups;
+}
+// Its LDS: two rounds of terms, and the activations' block sums when it makes its own.
 inline size_t q4k_r16_lds_bytes(const QMatDev& w, int n, bool own_sums) {
-    const size_t nmax = n <= 9 ? n : 16, S = w.groups >= 8 ? 8 : 4;
+    const size_t nmax = n <= 9 ? n : 16, S = q4k_r16_waves(w);
     return 2 * 4 * S * nmax * 16 * sizeof(float) + (own_sums ? (size_t)n * w.units * 8 * sizeof(float) : 0);
 }
 bool needs_block_sums(const nc_ctx* ctx, const QMatDev& q, int n);  // of an operator call of n <= 16 tokens

@@ -93,11 +93,12 @@ def test_prompt_block_matmul_wave_tiles(ctx, qtype, M, K, batches):
         check(ctx, nc.NC_TYPE_Q8_0, random_q8_0(M, K, seed=M), O.matmul_q8_0, M, K, batches, 6)
 
 
-# K-quant matrices on 16-row tiles (and from 16384 rows on 64-row ones): one super-block, cut quads, both wave
-# counts (4, and 8 from 29 super-blocks), operator calls whose kernel sums the activations itself and, at 16 tokens
-# of a long row, ones that take a separate launch
+# K-quant matrices on 16-row tiles (and from 16321 rows on 64-row ones): one super-block, cut quads, every wave count
+# (4; 8 from 29 super-blocks at up to 4096 rows; 1 and 2 for one and two quads at more than 8192), operator calls whose
+# kernel sums the activations itself and, at 16 tokens of a long row, ones that take a separate launch
 @pytest.mark.parametrize("qtype", ["q4_k", "q5_k"])
-@pytest.mark.parametrize("M,K", [(1, 256), (17, 1280), (100, 768), (40, 7680), (33, 8192), (16400, 256)])
+@pytest.mark.parametrize("M,K", [(1, 256), (17, 1280), (100, 768), (40, 7680), (33, 8192), (4113, 7424), (8209, 768),
+                                 (8209, 1280), (16400, 256)])
 def test_k_quant_tile_edges(ctx, qtype, M, K):
     batches = [1, 2, 3, 4, 5, 6, 7, 8, 9, 16, 18]
     if qtype == "q4_k":
