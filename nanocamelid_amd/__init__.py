@@ -38,8 +38,10 @@ def _stream_of(t):
     # the handle itself where torch gives it: building a torch.cuda.Stream object for it costs 1.7 us, a
     # quarter of a small operator call
     import torch
-    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-    return raw(t.device.index) if raw else torch.cuda.current_stream(t.device).cuda_stream
+    try:
+        return torch._C._cuda_getCurrentRawStream(t.device.index)
+    except AttributeError:
+        return torch.cuda.current_stream(t.device).cuda_stream
 
 
 class Context:
