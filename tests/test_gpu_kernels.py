@@ -241,9 +241,8 @@ def test_q4_k_layouts(ctx, shape, N):
                          ids=["partial-tile", "S8", "partial-group", "one-block"])
 @pytest.mark.parametrize("N", [1, 5, 9, 16, 21])
 def test_q8_0_bit_exact(ctx, shape, N):
-    """Q8_0 matrices (matmul_q8_0_batch, inference.rs:1343-1383) on 64-row tiles with 1-8
-    K-split waves, a partial last tile and a partial last group of 4 blocks; 21 tokens run as
-    16-token slices.  Every output bit-identical to the oracle."""
+    """Q8_0 matrices (matmul_q8_0_batch, inference.rs:1343-1383) on 16-row tiles: a partial
+    last tile, a partial last chunk of 32 blocks, one block; 21 tokens run on the prompt matmul.  Every output bit-identical to the oracle."""
     import nanocamelid_amd as nc
     M, K = shape
     w = random_q8_0(M, K, seed=M + K + N)
@@ -259,9 +258,9 @@ def test_q8_0_bit_exact(ctx, shape, N):
                          ids=["partial-tile", "S12", "one-superblock", "S8x4"])
 @pytest.mark.parametrize("N", [1, 5, 9, 16, 21])
 def test_q5_k_bit_exact(ctx, shape, N):
-    """Q5_K matrices (matmul_q5_k_batch's x86 path, inference.rs:2513-2640) on the 64-row
-    K-quant kernel: one to many super-blocks per row, a partial last tile, 21 tokens as
-    16-token slices.  Every output bit-identical to the oracle."""
+    """Q5_K matrices (matmul_q5_k_batch's x86 path, inference.rs:2513-2640) on the 16-row
+    K-quant kernel: one to many super-blocks per row, a partial last tile, 21 tokens on the prompt
+    matmul.  Every output bit-identical to the oracle."""
     import nanocamelid_amd as nc
     M, K = shape
     w = random_q5_k(M, K, seed=M + K + N)
